@@ -106,7 +106,7 @@ class Engine:
         self.penalty_pc = True
         self.vals_pc = None
         # node Jacobian and residual of the 3D u-p form: 'bins' (per-bin sums -- the Jacobian's
-        # as products on the matrix cores -- into a workspace of up to n_nodes x 11664 values,
+        # as products on the matrix cores -- into a workspace of up to n_nodes x 6480 values,
         # then a fixed-order gather) or 'rows' (one workgroup or thread per node row, no
         # workspace)
         self.jacobian_kernel = os.environ.get('GM_JACOBIAN_KERNEL', 'bins')

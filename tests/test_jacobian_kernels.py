@@ -201,3 +201,51 @@ def test_pattern_from_support_sets_equals_particle_pattern(dim):
     assert int((ext != 0).sum()) > 0
     for a, b in zip(out[0], out[1]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('cells', [(3, 4, 5), (6, 5, 3), (61, 4, 3), (130, 3, 3)])
+def test_line_sums_over_segments_of_any_length(precision, cells):
+    """The line sums cut a bin line into segments (at most 61 bins) that repeat the two bins
+    before them: on grids of one segment and of several the binned matrix equals the node-row
+    one to the round-off of a differently ordered sum (FP64: a few hundred terms of 1e-16;
+    FP32: the products and one rounding a bin, 2**-24 each), every variant writes the same
+    bits, and nothing but the particles' own pairs is read (workspace and matrix full of NaN)."""
+    import torch
+    from geowarp_amd import _lib as L
+    from geowarp_amd.solvers._engine import _stream
+    import geowarp_amd.solvers as gs
+    cfg = P.indent3d(n_cells=cells, dx=0.125, total_steps=10, depth=0.02, footing=0.3, material='Neo-Hookean',
+                     precision=precision, footing_start='surface', penalty_form='physical')
+    s = H.make(gs, cfg)
+    gen = torch.Generator(device=s.device).manual_seed(1)
+    noise = lambda t: torch.rand(t.shape, generator=gen, dtype=torch.float64, device=s.device) - 0.5  # noqa: E731
+    # positions moved by up to 0.2 cells inside the block (the bins hold from none to many particles)
+    lo = torch.tensor([s.start_x, s.start_y, s.start_z], device=s.device) + 0.15 * s.dx
+    hi = torch.tensor([s.end_x, s.end_y, s.end_z], device=s.device) - 0.15 * s.dx
+    s.x_particles.copy_(torch.minimum(torch.maximum(s.x_particles + 0.4 * s.dx * noise(s.x_particles), lo), hi))
+    s.GIMP_lp.mul_(1.0 + 0.2 * noise(s.GIMP_lp))
+    s.deformation_gradient_total_old.add_(0.01 * noise(s.deformation_gradient_total_old))
+    s.particle_pressure_array.copy_(noise(s.particle_pressure_array))
+    s.prepare_step(1, 10)
+    s._new.add_(1e-3 * s.dx * noise(s._new) * s.engine.freem)
+    eng = s.engine
+    eng.stage(s._args(1, 10), want_tangent=True)
+    a = _assemble(s, 'rows').double()
+    b = _assemble(s, 'bins')
+    rel = float((b.double() - a).norm() / a.norm())
+    print(precision, cells, 'nnzb', eng.nnzb, 'bins vs rows', rel)
+    assert rel < (1e-13 if precision == 'fp64' else 1e-6)
+    lib, fp32 = L.lib(), precision == 'mixed'
+    g, bn, pat = L.ctypes.byref(eng.grid), L.ctypes.byref(eng.bins), L.ctypes.byref(eng.pattern)
+    need = int(lib.gm_node_jacobian_work_bytes(g, int(fp32)))
+    w = torch.empty(need, dtype=torch.uint8, device=s.device)
+    vals = torch.empty_like(b)
+    for v in range(4):
+        w.fill_(255)
+        vals.fill_(float('nan'))
+        L.check(lib.gm_jacobian_bins_variant(g, bn, L.ptr(eng.D), int(fp32), v, L.ptr(w), need, _stream()), 'bins')
+        L.check(lib.gm_jacobian_gather_variant(g, bn, pat, int(fp32), v % 3, L.ptr(w), L.ptr(eng.freem), L.ptr(vals),
+                                               int(fp32), _stream()), 'gather')
+        assert torch.equal(vals, b), v
