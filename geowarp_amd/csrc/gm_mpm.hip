@@ -808,6 +808,240 @@ extern "C" int gm_particle_stage(const gm_grid* g, const gm_stage_args* a, hipSt
   return 0;
 }
 
+// ================================================================== 2D strips
+// Residual and Jacobian of the 2D forms, gathered by strips of consecutive node rows.  A
+// workgroup has a wave per stencil line oy: the bins that hold the strip's candidates in line
+// y - oy are consecutive, and so are their particles in bin order.  The wave stages that range
+// a piece of C particles at a time in LDS (per-axis tables and particle rows, loaded once for
+// the strip; odd strides, so that particles a few apart lie on different banks), every lane
+// walks the particles of its row's three bins, and the lines' sums are added in the order
+// oy = 0, 1, 2.  Workgroups of one XCD take consecutive strips: the three lines that read a
+// particle find it in that XCD's L2.
+template <bool COUPLED, typename TY, int ROWS, int NR, int C>
+struct Strip2d {
+  typedef Lay<2, COUPLED> L;
+  static constexpr int NT = COUPLED ? 9 : 6;  // per axis: w, g (, wa)
+  static constexpr int TS = 2 * NT | 1, RS = NR | 1;
+  struct Piece {
+    double t[C * TS];
+    TY r[C * RS];
+    uint8_t ext[C];
+  };
+
+  static __device__ __forceinline__ int first_row() {
+    const int n = gridDim.x, b = blockIdx.x, q = n / 8, r = n % 8, x = b % 8;
+    return (x * q + min(x, r) + b / 8) * ROWS;
+  }
+  // particles of the bins of line oy that strip rows [I0, I0 + ROWS) reach
+  static __device__ __forceinline__ void range(const gm_grid& g, int I0, int oy, const int* cell_start, int* lo,
+                                               int* hi) {
+    const int o = oy * (g.nx + 1);
+    const int b0 = max(I0 - 2 - o, 0), b1 = min(I0 + ROWS, g.n_nodes) - 1 - o;
+    *lo = b1 >= b0 ? cell_start[b0] : 0;
+    *hi = b1 >= b0 ? cell_start[b1 + 1] : 0;
+  }
+  // a row's candidates in line oy: the particles of bins (x - ox, y - oy), none where the row
+  // or the bin is off the grid
+  static __device__ __forceinline__ void bins(const gm_grid& g, int I, bool on, int oy, const int* cell_start, int* ks,
+                                              int* ke) {
+    const int nx1 = g.nx + 1, cx = I % nx1, cy = I / nx1;
+#pragma unroll
+    for (int ox = 0; ox < 3; ++ox) {
+      const bool ok = on && cx >= ox && cy >= oy;
+      const int b = I - ox - oy * nx1;
+      ks[ox] = ok ? cell_start[b] : 0;
+      ke[ox] = ok ? cell_start[b + 1] : 0;
+    }
+  }
+  // particles [k0, k0 + n) into the wave's piece
+  static __device__ __forceinline__ void stage(const gm_grid& g, const double* x_s, const double* lp_s,
+                                               const uint8_t* ext_s, const TY* rows, int k0, int n, Piece& p) {
+    const int lane = threadIdx.x & 63, last = n * NR - 1;
+    const TY* src = rows + (long)k0 * NR;
+    for (int q0 = 0; q0 <= last; q0 += 64 * 6) {
+      TY v[6];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) v[j] = src[min(q0 + j * 64 + lane, last)];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        const int q = q0 + j * 64 + lane;
+        if (q <= last) p.r[q / NR * RS + q % NR] = v[j];
+      }
+    }
+    for (int q = lane; q < 2 * n; q += 64) {
+      const int a = q & 1;
+      const long i = 2 * (long)k0 + q;
+      const Axis ax = gimp_axis(x_s[i], lp_s[i], a ? g.h[1] : g.h[0], a ? g.inv_h[1] : g.inv_h[0]);
+      double* t = p.t + (q >> 1) * TS + a * NT;
+#pragma unroll
+      for (int i3 = 0; i3 < 3; ++i3) {
+        t[i3] = ax.w[i3];
+        t[3 + i3] = ax.g[i3];
+        if (COUPLED) t[6 + i3] = ax.wa[i3];
+      }
+    }
+    if (lane < n) p.ext[lane] = ext_s[k0 + lane];
+  }
+  // orders the wave's LDS traffic between the stages (the piece belongs to one wave)
+  static __device__ __forceinline__ void sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+
+// A lane per (row, dof).  Bound by the LDS reads of each row's 36 candidates.  A thread per row
+// walked the nine bins in global memory and evaluated every particle's axis data nine times.
+// 1,048,576 particles, 264,000 rows, single phase: 281 -> 98 us; 45,000 particles u-p: 32 -> 20 us.
+template <bool COUPLED>
+__global__ void __launch_bounds__(192) k_strip_residual(gm_grid g, const double* x_s, const double* lp_s,
+                                                        const int* cell_start, const uint8_t* ext_s, const double* Y,
+                                                        const uint8_t* freem, double* rhs) {
+  typedef Lay<2, COUPLED> L;
+  constexpr int NB = L::NB, NY = L::NY, ROWS = 64 / NB, C = COUPLED ? 40 : 56;
+  typedef Strip2d<COUPLED, double, ROWS, NY, C> S;
+  constexpr int NT = S::NT;
+  __shared__ typename S::Piece piece[3];
+  __shared__ double OUT[3][ROWS * NB];
+  const int lane = threadIdx.x & 63, row = lane / NB, c = lane % NB;
+  const int I0 = S::first_row(), I = I0 + row;
+  const int oy = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  typename S::Piece& p = piece[oy];
+  int lo, hi, ks[3], ke[3];
+  S::range(g, I0, oy, cell_start, &lo, &hi);
+  S::bins(g, I, row < ROWS && I < g.n_nodes, oy, cell_start, ks, ke);
+  // the dof's rows of Y
+  const int y0 = c < 2 ? c : L::Y_M, y1 = c < 2 ? 2 + c : L::Y_M + 1, y2 = c < 2 ? L::Y_T + c : L::Y_Q;
+  double acc = 0.0;
+  for (int k0 = lo; k0 < hi; k0 += C) {
+    S::sync();
+    S::stage(g, x_s, lp_s, ext_s, Y, k0, min(C, hi - k0), p);
+    S::sync();
+#pragma unroll
+    for (int ox = 0; ox < 3; ++ox)
+      for (int k = max(ks[ox], k0) - k0; k < min(ke[ox] - k0, C); ++k) {
+        const uint8_t ex = p.ext[k];
+        if ((ox == 2 && !(ex & 1)) || (oy == 2 && !(ex & 2))) continue;  // outside the particle's support
+        const double *tx = p.t + k * S::TS, *ty = tx + NT, *yp = p.r + k * S::RS;
+        const double wx = tx[ox], wy = ty[oy], w = wx * wy;
+        acc += tx[3 + ox] * wy * yp[y0] + wx * ty[3 + oy] * yp[y1] + w * yp[y2];
+        if constexpr (COUPLED)
+          if (c == 2) acc += (w - tx[6 + ox] * ty[6 + oy]) * yp[L::Y_S];
+      }
+  }
+  if (row < ROWS) OUT[oy][lane] = acc;
+  __syncthreads();
+  if (oy == 0 && row < ROWS && I < g.n_nodes) {
+    const long d = (long)I * NB + c;
+    rhs[d] = freem[d] ? OUT[0][lane] + OUT[1][lane] + OUT[2][lane] : 0.0;
+  }
+}
+
+// A lane per (row, row dof, column dof): its two E entries come from the lane's own two columns
+// of D, and the 15 sums a line fit in registers.  Bound by the LDS reads of the 36 candidates
+// (18 values a candidate and lane) and by the 15 wavefronts a CU that the pieces' LDS leaves:
+// pieces of 24, 40 and 56 FP64 rows took 407, 407 and 497 us against 378 with 32; 40 FP32 rows
+// 298 us.  One wavefront per row, lanes over its 25 blocks and one particle after the other,
+// took 2750 us FP64 and 2709 us FP32 (1,048,576 particles, 264,000 rows; 210 MB of matrix and
+// 201 MB of D); u-p with 11,628 rows 135 -> 69 us.
+template <bool COUPLED, typename TD, typename TV>
+__global__ void __launch_bounds__(192) k_strip_jacobian(gm_grid g, const double* x_s, const double* lp_s,
+                                                        const int* cell_start, const uint8_t* ext_s, const TD* D,
+                                                        const uint8_t* freem, const int* row_ptr,
+                                                        const uint64_t* row_mask, TV* vals) {
+  typedef Lay<2, COUPLED> L;
+  constexpr int NB = L::NB, NB2 = NB * NB, NY = L::NY, NZ = L::NZ, ROWS = 64 / NB2, C = COUPLED ? 16 : sizeof(TD) == 4 ? 40 : 32;
+  typedef Strip2d<COUPLED, TD, ROWS, NY * NZ, C> S;
+  constexpr int NT = S::NT, RV = 25 * NB2, OS = RV | 1;
+  union Shared {
+    typename S::Piece piece[3];
+    double out[ROWS * OS];
+  };
+  __shared__ Shared sh;
+  const int lane = threadIdx.x & 63, row = lane / NB2, r = lane % NB2 / NB, c = lane % NB;
+  const int I0 = S::first_row(), I = I0 + row;
+  const int oy = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  typename S::Piece& p = sh.piece[oy];
+  int lo, hi, ks[3], ke[3];
+  S::range(g, I0, oy, cell_start, &lo, &hi);
+  S::bins(g, I, row < ROWS && I < g.n_nodes, oy, cell_start, ks, ke);
+  // the dof's rows of L_I and columns of D
+  const int y0 = (r < 2 ? r : L::Y_M) * NZ, y1 = (r < 2 ? 2 + r : L::Y_M + 1) * NZ,
+            y2 = (r < 2 ? L::Y_T + r : L::Y_Q) * NZ;
+  const int z0 = c < 2 ? c : L::Z_G, z1 = c < 2 ? 2 + c : L::Z_G + 1;
+  double acc[3][5];  // [jy][dx + 2]
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int d = 0; d < 5; ++d) acc[j][d] = 0.0;
+  for (int k0 = lo; k0 < hi; k0 += C) {
+    S::sync();
+    S::stage(g, x_s, lp_s, ext_s, D, k0, min(C, hi - k0), p);
+    S::sync();
+#pragma unroll
+    for (int ox = 0; ox < 3; ++ox)
+      for (int k = max(ks[ox], k0) - k0; k < min(ke[ox] - k0, C); ++k) {
+        const uint8_t ex = p.ext[k];
+        if ((ox == 2 && !(ex & 1)) || (oy == 2 && !(ex & 2))) continue;  // outside the particle's support
+        const double *tx = p.t + k * S::TS, *ty = tx + NT;
+        const TD* Dp = p.r + k * S::RS;
+        const double wx = tx[ox], wy = ty[oy], w = wx * wy, g0 = tx[3 + ox] * wy, g1 = wx * ty[3 + oy];
+        double wd = 0.0;
+        if constexpr (COUPLED) wd = w - tx[6 + ox] * ty[6 + oy];
+        // entries (r, z) of E = L_I D_p, then times M_J of the nine columns, one axis after the other
+        auto E = [&](int z) {
+          double e = g0 * (double)Dp[y0 + z] + g1 * (double)Dp[y1 + z] + w * (double)Dp[y2 + z];
+          if constexpr (COUPLED)
+            if (r == 2) e += wd * (double)Dp[L::Y_S * NZ + z];
+          return e;
+        };
+        const double e0 = E(z0), e1 = E(z1);
+#pragma unroll
+        for (int jx = 0; jx < 3; ++jx) {
+          const double u = e0 * tx[3 + jx], v = e1 * tx[jx];
+#pragma unroll
+          for (int jy = 0; jy < 3; ++jy) acc[jy][jx - ox + 2] += u * ty[jy] + v * ty[3 + jy];
+        }
+        if constexpr (COUPLED)
+          if (c == 2) {
+            const double ep = E(L::Z_P), eb = E(L::Z_PB);
+#pragma unroll
+            for (int jx = 0; jx < 3; ++jx) {
+              const double u = ep * tx[jx], v = eb * tx[6 + jx];
+#pragma unroll
+              for (int jy = 0; jy < 3; ++jy) acc[jy][jx - ox + 2] += u * ty[jy] + v * ty[6 + jy];
+            }
+          }
+      }
+  }
+  // the lines' sums, then masks, sign (the system matrix is -dR/du) and identity on fixed or
+  // inactive dofs; consecutive threads write consecutive values of a row
+  __syncthreads();
+  for (int q = threadIdx.x; q < ROWS * OS; q += 192) sh.out[q] = 0.0;
+  for (int o = 0; o < 3; ++o) {
+    __syncthreads();
+    if (oy == o && row < ROWS) {
+      double* out = sh.out + row * OS + r * NB + c;
+#pragma unroll
+      for (int jy = 0; jy < 3; ++jy)
+#pragma unroll
+        for (int d = 0; d < 5; ++d) out[((jy - o + 2) * 5 + d) * NB2] += acc[jy][d];
+    }
+  }
+  __syncthreads();
+  const int nx1 = g.nx + 1;
+  for (int q = threadIdx.x; q < ROWS * RV; q += 192) {
+    const int rw = q / RV, e = q % RV, bit = e / NB2, rr = e % NB2 / NB, cc = e % NB, Ir = I0 + rw;
+    if (Ir >= g.n_nodes) break;
+    const uint64_t m = row_mask[2 * Ir];
+    if (!((m >> bit) & 1ull)) continue;
+    const int Jn = Ir + bit % 5 - 2 + (bit / 5 - 2) * nx1;
+    const bool fr = freem[Ir * NB + rr], fc = freem[Jn * NB + cc];
+    double v = (fr && fc) ? -sh.out[rw * OS + e] : 0.0;
+    if (Jn == Ir && rr == cc && !fr) v = 1.0;
+    vals[((long)row_ptr[Ir] + __popcll(m & ((1ull << bit) - 1ull))) * NB2 + rr * NB + cc] = (TV)v;
+  }
+}
+
 // ================================================================== node residual
 template <int DIM, bool COUPLED>
 __global__ void __launch_bounds__(128) k_node_residual(gm_grid g, const double* x_s, const double* lp_s,
@@ -853,9 +1087,9 @@ extern "C" int gm_node_residual(const gm_grid* g, const gm_bins* b, const double
   int n = g->n_nodes;
   int blk = gm_blocks(n, 128);
   if (g->dim == 2 && !coupled)
-    k_node_residual<2, false><<<blk, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
+    k_strip_residual<false><<<gm_blocks(n, 32), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else if (g->dim == 2)
-    k_node_residual<2, true><<<blk, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
+    k_strip_residual<true><<<gm_blocks(n, 21), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else if (coupled)
     k_node_residual<3, true><<<blk, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else {
@@ -1198,8 +1432,19 @@ extern "C" int gm_node_jacobian(const gm_grid* g, const gm_bins* b, const gm_pat
     else if (vals_fp32) GM_JAC(DIM, CP, double, float);             \
     else GM_JAC(DIM, CP, double, double);                           \
   } while (0)
-  if (g->dim == 2 && !coupled) GM_JAC_T(2, false);
-  else if (g->dim == 2) GM_JAC_T(2, true);
+#define GM_STRIP(CP, TD, TV)                                                                                  \
+  k_strip_jacobian<CP, TD, TV><<<gm_blocks(n, (CP) ? 7 : 16), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, \
+                                                                           b->ext_s, (const TD*)D, freem,     \
+                                                                           pat->row_ptr, pat->row_mask, (TV*)vals)
+#define GM_STRIP_T(CP)                                      \
+  do {                                                     \
+    if (tangent_fp32 && vals_fp32) GM_STRIP(CP, float, float);   \
+    else if (tangent_fp32) GM_STRIP(CP, float, double);          \
+    else if (vals_fp32) GM_STRIP(CP, double, float);             \
+    else GM_STRIP(CP, double, double);                           \
+  } while (0)
+  if (g->dim == 2 && !coupled) GM_STRIP_T(false);
+  else if (g->dim == 2) GM_STRIP_T(true);
   else if (coupled && !getenv("GM_JACOBIAN_ROW_WAVE")) {
     // lanes per (column, column dof) of a bin (k_node_jacobian_up3); GM_JACOBIAN_ROW_WAVE=1
     // selects the one-wavefront-per-row form, which assembles the same matrix
@@ -1216,6 +1461,8 @@ extern "C" int gm_node_jacobian(const gm_grid* g, const gm_bins* b, const gm_pat
     gm::set_error("gm_node_jacobian: 3D single-phase is not a supported form");
     return -1;
   }
+#undef GM_STRIP_T
+#undef GM_STRIP
 #undef GM_JAC_T
 #undef GM_JAC
   GM_LAUNCH_CHECK();

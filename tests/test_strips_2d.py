@@ -1,0 +1,100 @@
+"""GPU: residual and Jacobian of the 2D forms, gathered by strips of node rows, against the dense
+sum over the particles with the oracle's weights: r_I = sum_p L_I Y_p, K_IJ = -sum_p L_I D_p M_J
+between free dofs, identity on the others."""
+import numpy as np
+import pytest
+
+import oracle.gimp as og
+
+
+def _tables(x, lp, h):
+    """Node numbers per axis, and w, g_x, g_y, w_avg of the 9 support nodes of every particle."""
+    lo, w, g, wa, ext = zip(*[og.axis_weights(x[:, a], lp[:, a], h[a], 1.0 / h[a]) for a in range(2)])
+    out = lambda p, q: np.einsum('ni,nj->nij', p, q).reshape(len(x), 9)  # noqa: E731
+    on = out(np.arange(3) < ext[0][:, None], np.arange(3) < ext[1][:, None])
+    cx = np.repeat(np.arange(3), 3)
+    cy = np.tile(np.arange(3), 3)
+    return lo[0][:, None] + cx, lo[1][:, None] + cy, out(w[0], w[1]), out(g[0], w[1]), out(w[0], g[1]), \
+        out(wa[0], wa[1]), on
+
+
+# grids and particle counts: fewer node rows than one strip, a strip's last row, remainders of
+# 7, 16, 21 and 32 rows, grid lines shorter and longer than a strip, no particles in most bins,
+# and ranges of one and of several staged pieces (up to 60 particles in one bin)
+@pytest.mark.gpu
+@pytest.mark.parametrize('coupled', [False, True])
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('cells,n,crowd', [((2, 2), 1, 0), ((3, 3), 5, 0), ((6, 5), 90, 60), ((15, 2), 200, 0),
+                                           ((30, 4), 700, 50), ((70, 3), 40, 0), ((5, 40), 900, 30)])
+def test_strip_residual_and_jacobian_equal_the_dense_sum(coupled, precision, cells, n, crowd):
+    import torch
+    from geowarp_amd.solvers._engine import Engine
+    h = (0.5, 0.5)
+    rng = np.random.default_rng(7 * n + cells[0])
+    lp = np.stack([rng.uniform(0.1, 0.6, n) * h[a] * 0.5 for a in range(2)], 1)
+    x = np.stack([rng.uniform(0.35, cells[a] - 0.35, n) * h[a] for a in range(2)], 1)
+    x[:crowd] = (np.array([1.2, 1.3]) + 0.05 * rng.standard_normal((crowd, 2))) * h
+    x = np.clip(x, lp + 1e-3, np.array(cells) * h - lp - 1e-3)
+    eng = Engine(2, coupled, cells, h, precision=precision)
+    dev = eng.dev
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device=dev)  # noqa: E731
+    X, LP = t(x), t(lp)
+    eng.begin_step(X, LP)
+    nb, NY, NZ = eng.nb, eng.NY, eng.NZ
+    Y = rng.standard_normal((n, NY))
+    D = rng.standard_normal((n, NY, NZ))
+    if precision == 'mixed':
+        D = D.astype(np.float32).astype(np.float64)
+    free = rng.random(eng.n_nodes * nb) < 0.85
+    order = eng.sorted[:n].long().cpu().numpy()
+    eng.Y.copy_(t(Y[order]).reshape(-1))
+    eng.D.copy_(t(D[order]).reshape(-1))
+    eng.freem.copy_(torch.as_tensor(free.astype(np.uint8), device=dev))
+    eng.rhs.fill_(float('nan'))
+    eng.vals.fill_(float('nan'))
+    eng.residual(X, LP)
+    eng.jacobian(X, LP)
+    torch.cuda.synchronize()
+
+    nx, ny, w, gx, gy, wa, on = _tables(x, lp, h)
+    node = nx + ny * (cells[0] + 1)
+    # L (9 x nb x NY) and M (9 x NZ x nb) of every particle; Y = P_xx P_xy P_yx P_yy t_x t_y (q m_x m_y s),
+    # z = H_xx H_xy H_yx H_yy (p pbar g_x g_y)
+    Lm = np.zeros((n, 9, nb, NY))
+    Mm = np.zeros((n, 9, NZ, nb))
+    for c in range(2):
+        Lm[:, :, c, c], Lm[:, :, c, 2 + c], Lm[:, :, c, 4 + c] = gx, gy, w
+        Mm[:, :, c, c], Mm[:, :, 2 + c, c] = gx, gy
+    if coupled:
+        Lm[:, :, 2, 6], Lm[:, :, 2, 7], Lm[:, :, 2, 8], Lm[:, :, 2, 9] = w, gx, gy, w - wa
+        Mm[:, :, 4, 2], Mm[:, :, 5, 2], Mm[:, :, 6, 2], Mm[:, :, 7, 2] = w, wa, gx, gy
+    Lm *= on[:, :, None, None]
+    Mm *= on[:, :, None, None]
+    N = eng.n_nodes
+    r = np.zeros((N, nb))
+    K = np.zeros((N, N, nb, nb))
+    for p in range(n):
+        i = node[p][on[p]]
+        r[i] += Lm[p][on[p]] @ Y[p]
+        K[np.ix_(i, i)] -= np.einsum('iay,yz,jzb->ijab', Lm[p][on[p]], D[p], Mm[p][on[p]])
+    r = np.where(free, r.reshape(-1), 0.0)
+    K = K.transpose(0, 2, 1, 3).reshape(N * nb, N * nb)
+    K[~free] = 0.0
+    K[:, ~free] = 0.0
+    K[~free, ~free] = 1.0
+    row_ptr, col = eng.row_ptr[:N + 1].cpu().numpy(), eng.col_idx[:eng.nnzb].cpu().numpy()
+    got = np.zeros((N, nb, N, nb))
+    v = eng.vals[:eng.nnzb * nb * nb].double().cpu().numpy().reshape(-1, nb, nb)
+    for i in range(N):
+        for s in range(row_ptr[i], row_ptr[i + 1]):
+            got[i, :, col[s], :] = v[s]
+    empty = np.repeat(np.diff(row_ptr) == 0, nb)  # rows outside every support have no blocks
+    got = got.reshape(N * nb, N * nb)
+    got[empty, empty] = K[empty, empty]
+    assert not np.isnan(got).any()
+    er = np.abs(eng.rhs.cpu().numpy() - r).max() / np.abs(r).max()
+    ek = np.abs(got - K).max() / np.abs(K).max()
+    print(coupled, precision, cells, n, 'residual', er, 'Jacobian', ek)
+    # a few hundred terms of 1e-16 of the largest; one FP32 rounding of the entries in the mixed form
+    assert er < 1e-13
+    assert ek < (1e-13 if precision == 'fp64' else 2.0 ** -23)
