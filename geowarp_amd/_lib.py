@@ -141,6 +141,8 @@ _SIGS = {
     'gm_local_eval_2d': (c_int, [_P, _P, _P, _P]),
     'gm_local_vjp_2d': (c_int, [_P, _P, _P]),
     'gm_bsr_transpose': (c_int, [c_int, c_int, c_int, _P, _P, _P, _P, _P]),
+    'gm_dense_inverse_work_bytes': (ctypes.c_size_t, [c_int]),
+    'gm_dense_inverse': (c_int, [c_int, c_int, _P, _P, _P, _P, _P, ctypes.c_size_t, _P, _P]),
     'gm_mg_setup': (c_int, [c_int, c_int, c_int, c_int, _P, _P, _P]),
     'gm_mg_vcycle': (c_int, [c_int, c_int, c_int, c_int, _P, c_int, c_int, c_int, c_double, _P, _P, _P]),
     'gm_mg_level_op': (c_int, [c_int, c_int, _P, c_int, c_int, _P, _P, c_double, _P, _P]),

@@ -1,0 +1,78 @@
+"""GPU: the coarsest operator's dense inverse (gm_dense_inverse) against its definition."""
+import numpy as np
+import pytest
+
+from geowarp_amd import _lib as L
+
+
+def _inverse(nb, blocks, row_ptr, col_idx):
+    import torch
+    lib = L.lib()
+    n = nb * (len(row_ptr) - 1)
+    dev = lambda a, dt: torch.as_tensor(np.ascontiguousarray(a), device='cuda').to(dt)  # noqa: E731
+    rp, ci, v = dev(row_ptr, torch.int32), dev(col_idx, torch.int32), dev(blocks, torch.float64)
+    inv = torch.full((n, n), float('nan'), dtype=torch.float64, device='cuda')
+    need = int(lib.gm_dense_inverse_work_bytes(n))
+    w = torch.full((need,), 255, dtype=torch.uint8, device='cuda')
+    err = torch.full((1,), float('nan'), dtype=torch.float64, device='cuda')
+    s = L.c_void_p(torch.cuda.current_stream().cuda_stream)
+    args = (nb, n // nb, L.ptr(rp), L.ptr(ci), L.ptr(v), L.ptr(inv), L.ptr(w))
+    assert lib.gm_dense_inverse(*args, need - 1, L.ptr(err), s) == -1  # a workspace one byte short is refused
+    L.check(lib.gm_dense_inverse(*args, need, L.ptr(err), s), 'gm_dense_inverse')
+    return inv.cpu().numpy(), float(err.item())
+
+
+def _banded(nb, n_nodes, band, rng, indefinite):
+    """Block-banded operator, |off-diagonal| row sums below half the diagonal, rows and columns scaled
+    over twelve decades; indefinite: the last dof of every node has a negative diagonal (a u-p form)."""
+    n = nb * n_nodes
+    A = rng.uniform(-1, 1, (n, n))
+    I = np.arange(n) // nb
+    A[np.abs(I[:, None] - I[None, :]) > band] = 0.0
+    A *= 0.5 / np.abs(A).sum(1, keepdims=True)
+    A[np.arange(n), np.arange(n)] = np.where((np.arange(n) % nb == nb - 1) & indefinite, -1.0, 1.0)
+    s = 10.0 ** rng.uniform(-6, 6, n)
+    rp, ci, v = [0], [], []
+    for i in range(n_nodes):
+        c = np.arange(max(i - band, 0), min(i + band + 1, n_nodes))
+        ci += list(c)
+        rp.append(len(ci))
+        v += [(A * s[:, None] * s[None, :])[i * nb:(i + 1) * nb, j * nb:(j + 1) * nb] for j in c]
+    return A * s[:, None] * s[None, :], s, np.array(v), np.array(rp), np.array(ci)
+
+
+# one entry, one block of 32, its edges, odd and even numbers of blocks with remainders
+@pytest.mark.gpu
+@pytest.mark.parametrize('nb,n_nodes', [(1, 1), (2, 15), (2, 16), (3, 11), (4, 8), (1, 33), (2, 32), (3, 43), (4, 40)])
+@pytest.mark.parametrize('indefinite', [False, True])
+def test_dense_inverse(nb, n_nodes, indefinite):
+    rng = np.random.default_rng(nb * n_nodes)
+    A, s, v, rp, ci = _banded(nb, n_nodes, 3, rng, indefinite and nb > 1)
+    X, err = _inverse(nb, v, rp, ci)
+    # scaled operator: |entries| <= 1, |inverse| <= 2 in the row-sum norm, so |A X - I| stays below
+    # n growth-free roundings of a few 1e-16
+    e = np.abs((A / s[:, None] / s[None, :]) @ (X * s[:, None] * s[None, :]) - np.eye(len(s))).max()
+    print(nb, n_nodes, indefinite, 'max |A X - I| scaled', e, 'probe', err)
+    assert e < 1e-13 and err < 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind', ['zero row', 'rank', 'nan'])
+def test_dense_inverse_reports_an_operator_it_cannot_invert(kind):
+    """The probe's error is not a small number for a singular operator and for NaN entries; the
+    hierarchy then takes the host's inverse."""
+    from geowarp_amd.solvers._multigrid import DENSE_TOL
+    rng = np.random.default_rng(3)
+    A, s, v, rp, ci = _banded(2, 40, 3, rng, False)
+    at = int(rp[20]) + int(np.flatnonzero(ci[rp[20]:rp[21]] == 20)[0])
+    if kind == 'zero row':
+        v[rp[20]:rp[21], 1, :] = 0.0
+    elif kind == 'rank':  # node 20 decoupled, its diagonal block of rank one
+        v[rp[20]:rp[21]] = 0.0
+        v[np.flatnonzero(ci == 20)] = 0.0
+        v[at] = 1.0
+    else:
+        v[at, 0, 1] = np.nan
+    err = _inverse(2, v, rp, ci)[1]
+    print(kind, err)
+    assert not err <= DENSE_TOL
