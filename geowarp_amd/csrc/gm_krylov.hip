@@ -23,6 +23,8 @@
 
 #define SPMV_T 256
 #define RED_T 256
+#define GS_MAX 257    // Gram-Schmidt coefficients a block holds: restart length + 1
+#define GS_BLOCKS 1024  // workgroups (and partial norms) of the Gram-Schmidt update
 
 // ------------------------------------------------------------------ SpMV
 template <int NB, int G, typename TM, typename TX, typename TY, int T = SPMV_T>
@@ -1187,62 +1189,133 @@ extern "C" int gm_fix_empty_diag(int n_rows, const int* row_ptr, const int* col_
 // is solved on the host, which reads one column of H per iteration.
 // x <- x + M^{-1} V y at the end of every cycle; restart from r = b - A x.
 
-// partial dots of w with basis vectors V[0..k): part[i*nchunk + c]
-// gate: when given, the launch does nothing unless *gate != 0 (a decision taken on the
-// device inside an enqueued Arnoldi step)
-template <typename TV>
-__global__ void k_multidot(const double* gate, long n, int k, const TV* V, long ldv, const TV* w, int nchunk,
-                           double* part) {
-  if (gate && *gate == 0.0) return;
-  __shared__ double sh[RED_T];
-  int i = blockIdx.y;
+// Gram-Schmidt of one Arnoldi step in five to seven launches (k_gs_dots, [k_gs_fin,] k_gs_axpy,
+// the same again for the second pass, k_gs_scale).  Launches of small systems take 2.5 us each
+// whatever they do, so what follows a pass rides on it: w.w on the first pass's products, the new
+// norm on the update, the second-pass decision and the final norm on the kernels that need them,
+// the column of H on the scaling.  One launch a quantity took 14 and a copy: 41 us a step on
+// 5,600 dofs (29 steps) against 17 us, 90 against 40 us on 557,700 dofs in FP32.
+
+// sum over the workgroup (RED_T threads) in a fixed order; every thread gets it
+__device__ __forceinline__ double block_sum(double s, double* sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = sh[0];
+#pragma unroll
+  for (int i = 1; i < RED_T / 64; ++i) s += sh[i];
+  return s;
+}
+
+// the partial sums of ||w||^2 that k_gs_axpy left, added in a fixed order
+__device__ __forceinline__ double norm_of_parts(const double* npart, int np, double* sh) {
   double s = 0.0;
-  const TV* vi = V + (long)i * ldv;
+  for (int c = threadIdx.x; c < np; c += RED_T) s += npart[c];
+  return block_sum(s, sh);
+}
+
+// part[i * nchunk + c]: partial dots of w with basis vectors V[0..k) and, in the first pass
+// (npart null), with itself (i = k).  The second pass first takes the selective
+// reorthogonalisation test (Daniel, Gragg, Kaufman & Stewart 1976) on the norm after the first
+// pass, sc[0], and before it, sc[1]: sc[2] = 1 when the pass removed more than half of ||w||^2 or
+// a norm is NaN; else the pass is left out.
+template <typename TV>
+__global__ void __launch_bounds__(RED_T) k_gs_dots(long n, int k, const TV* V, long ldv, const TV* w, int nchunk,
+                                                   double* part, const double* npart, int np, double* sc) {
+  __shared__ double sh[RED_T / 64];
+  if (npart) {
+    const double after = norm_of_parts(npart, np, sh);
+    const bool second = !(after >= 0.5 * sc[1]);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+      sc[0] = after;
+      sc[2] = second ? 1.0 : 0.0;
+    }
+    if (!second) return;
+  }
+  const int i = blockIdx.y;
+  const TV* vi = i < k ? V + (long)i * ldv : w;
+  double s = 0.0;
   for (long r = blockIdx.x * (long)RED_T + threadIdx.x; r < n; r += (long)nchunk * RED_T)
     s += (double)vi[r] * (double)w[r];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = RED_T / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[(long)i * nchunk + blockIdx.x] = sh[0];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) part[(long)i * nchunk + blockIdx.x] = s;
 }
 
-// h[i] = sum_c part[i*nchunk + c]  (one block per basis vector, fixed order)
-__global__ void k_multidot_fin(const double* gate, int nchunk, const double* part, double* h) {
+// h[i] = sum_c part[i * nchunk + c] for i < k, *ww that of i = k (one block each, fixed order)
+__global__ void __launch_bounds__(RED_T) k_gs_fin(const double* gate, int k, int nchunk, const double* part, double* h,
+                                                  double* ww) {
   if (gate && *gate == 0.0) return;
-  __shared__ double sh[RED_T];
-  int i = blockIdx.x;
+  __shared__ double sh[RED_T / 64];
+  const int i = blockIdx.x;
   double s = 0.0;
   for (int c = threadIdx.x; c < nchunk; c += RED_T) s += part[(long)i * nchunk + c];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = RED_T / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) h[i] = sh[0];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) (i < k ? h[i] : *ww) = s;
 }
 
-// w -= sum_i V_i h_i   (h on the device); one row per thread, four independent partial
-// sums over the basis vectors so that four loads are in flight per thread
+// w -= sum_i V_i h_i, and the partial sums of the new ||w||^2 (npart, one a block).  A row a
+// thread, four independent partial sums over the basis vectors so that four loads are in flight.
+// nchunk > 0: h (and ww, when given) are summed here from part, in every block; block 0 stores them.
 template <typename TV>
-__global__ void __launch_bounds__(256) k_multiaxpy(const double* gate, long n, int k, const TV* V, long ldv,
-                                                   const double* h, TV* w) {
+__global__ void __launch_bounds__(RED_T) k_gs_axpy(const double* gate, long n, int k, const TV* V, long ldv,
+                                                   const double* part, int nchunk, double* h, double* ww, TV* w,
+                                                   double* npart) {
+  __shared__ double hs[GS_MAX], sh[RED_T / 64];
   if (gate && *gate == 0.0) return;
-  long r = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  int i = 0;
-  for (; i + 3 < k; i += 4) {
-    a0 += h[i] * (double)V[(long)i * ldv + r];
-    a1 += h[i + 1] * (double)V[(long)(i + 1) * ldv + r];
-    a2 += h[i + 2] * (double)V[(long)(i + 2) * ldv + r];
-    a3 += h[i + 3] * (double)V[(long)(i + 3) * ldv + r];
+  for (int i = threadIdx.x; i < k + (nchunk && ww ? 1 : 0); i += RED_T) {
+    double s = 0.0;
+    if (nchunk)
+      for (int c = 0; c < nchunk; ++c) s += part[(long)i * nchunk + c];
+    else
+      s = h[i];
+    if (i < k) hs[i] = s;
+    if (nchunk && blockIdx.x == 0) (i < k ? h[i] : *ww) = s;
   }
-  for (; i < k; ++i) a0 += h[i] * (double)V[(long)i * ldv + r];
-  w[r] = (TV)((double)w[r] - ((a0 + a1) + (a2 + a3)));
+  __syncthreads();
+  double q = 0.0;
+  for (long r = blockIdx.x * (long)RED_T + threadIdx.x; r < n; r += (long)gridDim.x * RED_T) {
+    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+    int i = 0;
+    for (; i + 3 < k; i += 4) {
+      a0 += hs[i] * (double)V[(long)i * ldv + r];
+      a1 += hs[i + 1] * (double)V[(long)(i + 1) * ldv + r];
+      a2 += hs[i + 2] * (double)V[(long)(i + 2) * ldv + r];
+      a3 += hs[i + 3] * (double)V[(long)(i + 3) * ldv + r];
+    }
+    for (; i < k; ++i) a0 += hs[i] * (double)V[(long)i * ldv + r];
+    const TV v = (TV)((double)w[r] - ((a0 + a1) + (a2 + a3)));
+    w[r] = v;
+    q += (double)v * (double)v;
+  }
+  q = block_sum(q, sh);
+  if (threadIdx.x == 0) npart[blockIdx.x] = q;
+}
+
+// v = w / ||w|| (zero when the norm is not positive: a breakdown the host sees), and the step's
+// column of H, norms and flag to pinned host memory.  The norm is that of the second pass's
+// partial sums when there was one, else sc[0].
+template <typename TV>
+__global__ void __launch_bounds__(RED_T) k_gs_scale(long n, int k, const TV* w, const double* npart, int np,
+                                                    const double* h, const double* h2, const double* sc, TV* v,
+                                                    double* host, int stride) {
+  __shared__ double sh[RED_T / 64];
+  const bool second = sc[2] != 0.0;
+  const double q = second ? norm_of_parts(npart, np, sh) : sc[0];
+  const double s = (q > 0.0) ? 1.0 / sqrt(q) : 0.0;
+  for (long r = blockIdx.x * (long)RED_T + threadIdx.x; r < n; r += (long)gridDim.x * RED_T)
+    v[r] = (TV)((double)w[r] * s);
+  if (blockIdx.x) return;
+  for (int i = threadIdx.x; i < k; i += RED_T) {
+    host[i] = h[i];
+    if (second) host[stride + i] = h2[i];
+  }
+  if (threadIdx.x == 0) {
+    host[2 * stride] = q;
+    host[2 * stride + 1] = sc[1];
+    host[2 * stride + 2] = sc[2];
+  }
 }
 
 // out = sum_i V_i y_i   (y on the device); one row per thread, four partial sums
@@ -1260,21 +1333,6 @@ __global__ void __launch_bounds__(256) k_combine(long n, int k, const TV* V, lon
   }
   for (; i < k; ++i) a0 += y[i] * (double)V[(long)i * ldv + r];
   out[r] = (TV)((a0 + a1) + (a2 + a3));
-}
-
-// selective reorthogonalisation test (Daniel, Gragg, Kaufman & Stewart 1976) on the
-// device: gate = 1 when the first pass removed more than half of ||w||^2 (or a norm is NaN)
-__global__ void k_reorth_gate(const double* nrm_after, const double* nrm_before, double* gate) {
-  *gate = (*nrm_after >= 0.5 * *nrm_before) ? 0.0 : 1.0;
-}
-
-// b = a / sqrt(*nrm2) (zero when the norm is not positive: a breakdown the host sees)
-template <typename TV>
-__global__ void k_scale_norm(long n, const TV* a, const double* nrm2, TV* b) {
-  const double q = *nrm2;
-  const double s = (q > 0.0) ? 1.0 / sqrt(q) : 0.0;
-  for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < n; r += (long)gridDim.x * blockDim.x)
-    b[r] = (TV)((double)a[r] * s);
 }
 
 template <typename TV>
@@ -1476,9 +1534,17 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
   long n = (long)n_rows * NB;
   long ldv = n;
   int vb = dot_blocks(n);
-  // multidot chunks per basis vector: up to 256 while few vectors exist (fills the chip), within
-  // the 64 (m + 1) partial sums of the workspace
-  auto chunks = [m](int cols) { return std::min(256, 64 * (m + 1) / cols); };
+  // partial norms of the update: the last GS_BLOCKS of the workspace's partial sums
+  const int cap = std::max(64 * (m + 1), 2048);
+  double* npart = part + (cap - GS_BLOCKS);
+  const int ab = (int)std::min<long>(GS_BLOCKS, gm_blocks(n, RED_T));
+  // chunks of a product with one basis vector: 256 fill the chip.  Up to 64 k entries at most 16,
+  // of at least 1024 entries each: few enough for every block of the update to add them up itself
+  // (fold), which saves the launch of k_gs_fin; above, the blocks are many and it costs more
+  const bool fold = n <= 65536;
+  auto chunks = [&](int cols) {
+    return std::max(1, std::min(fold ? (int)std::min<long>(16, n / 1024) : 256, (cap - GS_BLOCKS) / cols));
+  };
   GM_HIP(hipMemsetAsync(x, 0, sizeof(TV) * n, st));
   // ||b||
   k_dot2<TV><<<vb, RED_T, 0, st>>>(n, b, b, nullptr, nullptr, part);
@@ -1558,7 +1624,7 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
       // one Arnoldi step on the device: z_j = M^-1 v_j, w = A z_j, classical Gram-Schmidt
       // with selective reorthogonalisation (Daniel, Gragg, Kaufman & Stewart 1976: a second
       // pass only when the first removed more than half of ||w||^2, decided on the device),
-      // v_{j+1} = w / ||w||, and the column of H copied to pinned host memory.  dh: [0, m+2)
+      // v_{j+1} = w / ||w||, and the column of H stored to pinned host memory.  dh: [0, m+2)
       // pass-1 coefficients, [m+2, 2m+4) pass-2 coefficients, [2m+4] ||w||^2 after the
       // passes, [2m+5] before them, [2m+6] the second-pass flag.
       auto enqueue = [&, j](hipStream_t q) -> int {
@@ -1568,24 +1634,16 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
         int prc = prec.apply(vj, zj, q);
         if (prc) return prc;
         launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, zj, w, nullptr, nullptr, nullptr, q);
-        k_dot2<TV><<<vb, RED_T, 0, q>>>(n, w, w, nullptr, nullptr, part);
-        k_sum_parts<<<1, RED_T, 0, q>>>(part, vb, dh + nsl + 1, nullptr);
-        const int nchunk = chunks(j + 1);
-        k_multidot<TV><<<dim3(nchunk, j + 1), RED_T, 0, q>>>(nullptr, n, j + 1, V, ldv, w, nchunk, part);
-        k_multidot_fin<<<j + 1, RED_T, 0, q>>>(nullptr, nchunk, part, dh);
-        k_multiaxpy<TV><<<gm_blocks(n, 256), 256, 0, q>>>(nullptr, n, j + 1, V, ldv, dh, w);
-        k_dot2<TV><<<vb, RED_T, 0, q>>>(n, w, w, nullptr, nullptr, part);
-        k_sum_parts<<<1, RED_T, 0, q>>>(part, vb, dh + nsl, nullptr);
-        k_reorth_gate<<<1, 1, 0, q>>>(dh + nsl, dh + nsl + 1, dh + gate);
-        k_multidot<TV><<<dim3(nchunk, j + 1), RED_T, 0, q>>>(dh + gate, n, j + 1, V, ldv, w, nchunk, part);
-        k_multidot_fin<<<j + 1, RED_T, 0, q>>>(dh + gate, nchunk, part, dh + (m + 2));
-        k_multiaxpy<TV><<<gm_blocks(n, 256), 256, 0, q>>>(dh + gate, n, j + 1, V, ldv, dh + (m + 2), w);
-        const int nc1 = chunks(1);
-        k_multidot<TV><<<dim3(nc1, 1), RED_T, 0, q>>>(dh + gate, n, 1, w, ldv, w, nc1, part);
-        k_multidot_fin<<<1, RED_T, 0, q>>>(dh + gate, nc1, part, dh + nsl);
-        k_scale_norm<TV><<<vb, RED_T, 0, q>>>(n, w, dh + nsl, vj1);
+        const int nchunk = chunks(j + 2), fc = fold ? nchunk : 0;
+        double *h2 = dh + (m + 2), *sc = dh + nsl;
+        k_gs_dots<TV><<<dim3(nchunk, j + 2), RED_T, 0, q>>>(n, j + 1, V, ldv, w, nchunk, part, nullptr, 0, sc);
+        if (!fold) k_gs_fin<<<j + 2, RED_T, 0, q>>>(nullptr, j + 1, nchunk, part, dh, sc + 1);
+        k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(nullptr, n, j + 1, V, ldv, part, fc, dh, sc + 1, w, npart);
+        k_gs_dots<TV><<<dim3(nchunk, j + 1), RED_T, 0, q>>>(n, j + 1, V, ldv, w, nchunk, part, npart, ab, sc);
+        if (!fold) k_gs_fin<<<j + 1, RED_T, 0, q>>>(sc + 2, j + 1, nchunk, part, h2, nullptr);
+        k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(sc + 2, n, j + 1, V, ldv, part, fc, h2, nullptr, w, npart);
+        k_gs_scale<TV><<<vb, RED_T, 0, q>>>(n, j + 1, w, npart, ab, dh, h2, sc, vj1, host, m + 2);
         GM_LAUNCH_CHECK();
-        GM_HIP(hipMemcpyAsync(host, dh, sizeof(double) * 3 * (m + 2), hipMemcpyDeviceToHost, q));
         return 0;
       };
       int prc = run_step(sg, j, st, enqueue);
@@ -1857,58 +1915,88 @@ __global__ void k_rap(Dims f, Dims c, int n_coarse, const int* rp_c, const uint6
   for (int k = 0; k < NB * NB; ++k) out[k] = acc[k];
 }
 
-// b_c = P^T r_f (free fine dofs only)
+// b_c = P^T r_f (free fine dofs only) and, with dinv, the coarse level's first sweep
+// x_c = omega Dinv b_c.  A thread a coarse dof, the dofs of a node next to each other (NPB nodes a
+// block, so that a node's b_c are in one block).  Bound by latency: all 3^DIM values are loaded
+// before any is looked at, where a branch on each flag made the loads wait for one another:
+// 4.8 -> 3.0 us for 11,628 u-p nodes, 11 -> 5.2 us on average over the levels of 139,425 in 3D,
+// and the coarse level's first sweep no longer needs a launch of its own.
 template <int DIM, int NB, typename T>
-// one thread per coarse dof (consecutive threads: the dofs of a node, then the next node)
-__global__ void k_restrict(Dims f, Dims c, int n_coarse, const uint8_t* freem_f, const T* r_f, T* b_c) {
-  long gid = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (gid >= (long)n_coarse * NB) return;
-  int I = (int)(gid / NB), k = (int)(gid % NB);
+__global__ void __launch_bounds__(256) k_restrict(Dims f, Dims c, int n_coarse, const uint8_t* freem_f, const T* r_f,
+                                                  T* b_c, const T* dinv, double omega, T* x_c) {
+  constexpr int NPB = 256 / NB, M = DIM == 3 ? 27 : 9;
+  __shared__ double bs[NPB * NB];
+  const int t = threadIdx.x, I = min((int)blockIdx.x * NPB + t / NB, n_coarse - 1), k = t % NB;
+  const bool on = t < NPB * NB && (int)blockIdx.x * NPB + t / NB < n_coarse;
   int A[3];
   coords<DIM>(I, c.n[0], c.n[1], A);
+  T v[M];
+  uint8_t fr[M];
+  double wt[M];
+#pragma unroll
+  for (int q = 0; q < M; ++q) {
+    const int d[3] = {q % 3 - 1, q / 3 % 3 - 1, DIM == 3 ? q / 9 - 1 : 0};
+    int a[3] = {0, 0, 0};
+    double w = 1.0;
+#pragma unroll
+    for (int ax = 0; ax < DIM; ++ax) {
+      const int at = 2 * A[ax] + d[ax];
+      a[ax] = min(max(at, 0), f.n[ax]);
+      w *= at != a[ax] ? 0.0 : (d[ax] ? 0.5 : 1.0);
+    }
+    const long i = (long)node_of<DIM>(a, f.n[0], f.n[1]) * NB + k;
+    v[q] = r_f[i];
+    fr[q] = freem_f[i];
+    wt[q] = w;
+  }
   double acc = 0.0;
-  const int oz = (DIM == 3) ? 1 : 0;
-  for (int dz = -oz; dz <= oz; ++dz)
-    for (int dy = -1; dy <= 1; ++dy)
-      for (int dx = -1; dx <= 1; ++dx) {
-        int a[3] = {2 * A[0] + dx, 2 * A[1] + dy, 2 * A[2] + dz};
-        if (a[0] < 0 || a[0] > f.n[0] || a[1] < 0 || a[1] > f.n[1]) continue;
-        if (DIM == 3 && (a[2] < 0 || a[2] > f.n[2])) continue;
-        double w = (dx == 0 ? 1.0 : 0.5) * (dy == 0 ? 1.0 : 0.5) * ((DIM == 3 && dz != 0) ? 0.5 : 1.0);
-        int i = node_of<DIM>(a, f.n[0], f.n[1]);
-        if (freem_f[(long)i * NB + k]) acc += w * (double)r_f[(long)i * NB + k];
-      }
-  b_c[gid] = (T)acc;
+#pragma unroll
+  for (int q = 0; q < M; ++q) acc += (fr[q] && wt[q] != 0.0) ? wt[q] * (double)v[q] : 0.0;
+  const T bc = (T)acc;
+  const long gid = (long)I * NB + k;
+  if (on) b_c[gid] = bc;
+  if (!dinv) return;
+  if (on) bs[t] = (double)bc;
+  __syncthreads();
+  if (!on) return;
+  double s = 0.0;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) s += (double)dinv[gid * NB + j] * bs[t - k + j];
+  x_c[gid] = (T)(omega * s);
 }
 
-// x_f += P x_c (free fine dofs only); one thread per fine dof
+// x_f += P x_c (free fine dofs only); one thread per fine dof, its parents' values loaded together
 template <int DIM, int NB, typename T>
 __global__ void k_prolong_add(Dims f, Dims c, int n_fine, const uint8_t* freem_f, const T* x_c, T* x_f) {
+  constexpr int M = DIM == 3 ? 8 : 4;
   long gid = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (gid >= (long)n_fine * NB) return;
   int i = (int)(gid / NB), k = (int)(gid % NB);
-  if (!freem_f[gid]) return;
   int a[3];
   coords<DIM>(i, f.n[0], f.n[1], a);
-  int lo[3], hi[3];
+  const uint8_t fr = freem_f[gid];
+  const T x = x_f[gid];
+  T v[M];
 #pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    lo[ax] = a[ax] >> 1;
-    hi[ax] = (a[ax] + 1) >> 1;  // == lo for even a
+  for (int q = 0; q < M; ++q) {
+    // parents along an axis: both neighbours of an odd coordinate, the node itself of an even one
+    int A[3] = {0, 0, 0};
+#pragma unroll
+    for (int ax = 0; ax < DIM; ++ax) A[ax] = (a[ax] + ((q >> ax) & 1)) >> 1;
+    v[q] = x_c[(long)node_of<DIM>(A, c.n[0], c.n[1]) * NB + k];
   }
-  double acc = 0.0;
-  const int zc = (DIM == 3) ? 2 : 1;
-  for (int pz = 0; pz < zc; ++pz)
-    for (int py = 0; py < 2; ++py)
-      for (int px = 0; px < 2; ++px) {
-        int A[3] = {px ? hi[0] : lo[0], py ? hi[1] : lo[1], pz ? hi[2] : lo[2]};
-        // even coordinate: one parent (skip the duplicate), odd: two parents of weight 0.5
-        if ((px && hi[0] == lo[0]) || (py && hi[1] == lo[1]) || (DIM == 3 && pz && hi[2] == lo[2])) continue;
-        double w = ((a[0] & 1) ? 0.5 : 1.0) * ((a[1] & 1) ? 0.5 : 1.0) * ((DIM == 3 && (a[2] & 1)) ? 0.5 : 1.0);
-        int J = node_of<DIM>(A, c.n[0], c.n[1]);
-        acc += w * (double)x_c[(long)J * NB + k];
-      }
-  x_f[gid] = (T)((double)x_f[gid] + acc);
+  if (!fr) return;
+  double w = 1.0, acc = 0.0;
+#pragma unroll
+  for (int ax = 0; ax < DIM; ++ax) w *= (a[ax] & 1) ? 0.5 : 1.0;
+#pragma unroll
+  for (int q = 0; q < M; ++q) {
+    bool twice = false;  // the even coordinate's node again
+#pragma unroll
+    for (int ax = 0; ax < DIM; ++ax) twice = twice || (((q >> ax) & 1) && !(a[ax] & 1));
+    if (!twice) acc += w * (double)v[q];
+  }
+  x_f[gid] = (T)((double)x + acc);
 }
 
 // x = omega Dinv b; one thread per dof
@@ -2032,8 +2120,9 @@ static int smooth(const gm_mg_level& lv, int l, const T* b, T* x, int count, dou
   return 0;
 }
 
+// started: x already holds the first sweep (the restriction to this level made it)
 template <int DIM, int NB, typename T>
-static int vcycle(const Cycle& cy, int l, const T* b, T* x, hipStream_t st) {
+static int vcycle(const Cycle& cy, int l, const T* b, T* x, hipStream_t st, bool started = false) {
   const gm_mg_level& lv = cy.L[l];
   int n = lv.n_nodes;
   const T* dinv = (const T*)lv.dinv;
@@ -2046,7 +2135,7 @@ static int vcycle(const Cycle& cy, int l, const T* b, T* x, hipStream_t st) {
     return 0;
   }
   int sweeps = coarsest ? cy.coarse_sweeps : cy.nu_pre;
-  k_jac_first<NB, T><<<gm_blocks((long)n * NB, 256), 256, 0, st>>>(n, dinv, b, cy.omega, x);
+  if (!started) k_jac_first<NB, T><<<gm_blocks((long)n * NB, 256), 256, 0, st>>>(n, dinv, b, cy.omega, x);
   GM_LAUNCH_CHECK();
   int rc = smooth<NB, T>(lv, l, b, x, sweeps - 1, cy.omega, st);
   if (rc) return rc;
@@ -2055,10 +2144,12 @@ static int vcycle(const Cycle& cy, int l, const T* b, T* x, hipStream_t st) {
   const int gamma = lv.gamma > 1 ? lv.gamma : 1;  // 1: V-cycle, 2: W-cycle at this level
   for (int g = 0; g < gamma; ++g) {
     level_op<NB, 1, T>(lv, l, x, b, nullptr, 0.0, r, st);  // r = b - A x
-    k_restrict<DIM, NB, T><<<gm_blocks((long)cv.n_nodes * NB, 256), 256, 0, st>>>(
-        dims_of(lv), dims_of(cv), cv.n_nodes, lv.freem, r, (T*)cv.b);
+    const bool dense = l + 1 == cy.n_levels - 1 && cv.dense_inv;
+    k_restrict<DIM, NB, T><<<gm_blocks(cv.n_nodes, 256 / NB), 256, 0, st>>>(
+        dims_of(lv), dims_of(cv), cv.n_nodes, lv.freem, r, (T*)cv.b, dense ? nullptr : (const T*)cv.dinv, cy.omega,
+        (T*)cv.x);
     GM_LAUNCH_CHECK();
-    rc = vcycle<DIM, NB, T>(cy, l + 1, (const T*)cv.b, (T*)cv.x, st);
+    rc = vcycle<DIM, NB, T>(cy, l + 1, (const T*)cv.b, (T*)cv.x, st, !dense);
     if (rc) return rc;
     k_prolong_add<DIM, NB, T><<<gm_blocks((long)n * NB, 256), 256, 0, st>>>(dims_of(lv), dims_of(cv), n, lv.freem,
                                                                              (const T*)cv.x, x);
