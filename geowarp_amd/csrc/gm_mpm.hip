@@ -431,16 +431,96 @@ extern "C" int gm_bsr_pattern(const gm_grid* g, const gm_bins* b, gm_pattern* pa
 }
 
 // ================================================================== particle stage
-// NHONLY: an instance for the Neo-Hookean skeleton alone, compiled without the
-// Hencky-family return maps (eigen-decomposition, local Newton solves) and so with
-// a fraction of the general instance's registers.
-template <int DIM, bool COUPLED, typename TD, bool NHONLY = false>
+// Rows of W values, one a lane, to and from memory through the wave's LDS tile, so that
+// consecutive lanes touch consecutive values (a lane writing its own row of 9 to 17 doubles
+// touches a cache line a lane and store).  Every lane of the wave takes part; the first `n` lanes
+// have a row.
+template <typename T>
+struct WaveRows {
+  T* tile;
+  int lane, n;
+  static __device__ __forceinline__ void sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  template <int W>
+  __device__ __forceinline__ void put(const double* v) {
+    sync();
+#pragma unroll
+    for (int i = 0; i < W; ++i) tile[lane * (W | 1) + i] = (T)v[i];
+    sync();
+  }
+  // lane l's row to row index(l) of an array of W values a row
+  template <int W>
+  __device__ __forceinline__ void store(T* base, int row, const double* v) {
+    put<W>(v);
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const int q = i * 64 + lane, l = q / W, e = q % W;
+      const long r = __shfl(row, l, 64);
+      if (l < n) base[r * W + e] = tile[l * (W | 1) + e];
+    }
+  }
+  // the first w of the tile's W values a lane (at stride W | 1) to base + lane * stride
+  template <int W>
+  __device__ __forceinline__ void flush(T* base, int stride, int w) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const int q = i * 64 + lane, l = q / W, e = q % W;
+      if (l < n && e < w) base[l * stride + e] = tile[l * (W | 1) + e];
+    }
+  }
+  // rows by index: the loads, then the exchange
+  template <int W>
+  __device__ __forceinline__ void load(const T* base, int row, T* t) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const int q = i * 64 + lane, l = min(q / W, n - 1), e = q % W;
+      t[i] = base[(long)__shfl(row, l, 64) * W + e];
+    }
+  }
+  template <int W>
+  __device__ __forceinline__ void take(const T* t, double* v) {
+    sync();
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const int q = i * 64 + lane;
+      tile[q / W * (W | 1) + q % W] = t[i];
+    }
+    sync();
+#pragma unroll
+    for (int i = 0; i < W; ++i) v[i] = (double)tile[lane * (W | 1) + i];
+  }
+};
+
+// One particle a lane, an instance a material (MAT): the return maps of the others would cost it
+// registers.  The per-particle arrays and the rows of Y and D pass through LDS (WaveRows); D is
+// formed row by row, R rows a pass of the tile (1 and 4 FP32 rows a pass: 658 and 763 us where 2
+// take 672).  Bound by the memory traffic of those rows.  1,048,576 particles, a lane writing its
+// own rows and D by columns before: 3D u-p Neo-Hookean 334 -> 265 us without the tangent, 1282 ->
+// 672 with FP32 and 2404 -> 1024 with FP64 rows of D; 2D J2 220 -> 149 and 340 -> 229 us; 37,128
+// particles of 3D Drucker-Prager 151 -> 73 us.  A few thousand particles take the latency of one
+// wavefront either way (25 and 29 us).
+template <int DIM, bool COUPLED, typename TD, int MAT>
 __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args a) {
   typedef Lay<DIM, COUPLED> L;
-  const bool neo_hookean = NHONLY || a.mat_kind == MAT_NEOHOOKEAN;
-  int kq = blockIdx.x * blockDim.x + threadIdx.x;  // bin-sorted position: Y/D row
-  if (kq >= a.n_particles) return;
-  int p = a.sorted ? a.sorted[kq] : kq;               // particle id: state arrays
+  constexpr bool neo_hookean = MAT == MAT_NEOHOOKEAN;
+  constexpr int NY = L::NY, NZ = L::NZ;
+  constexpr int R = sizeof(TD) == 4 ? 2 : 1;  // rows of D a pass
+  constexpr int CMAX = NY > 9 ? NY : 9;
+  constexpr int TILE = 64 * (CMAX | 1) * 8 > 64 * (R * NZ | 1) * (int)sizeof(TD) ? 64 * (CMAX | 1) * 8
+                                                                                 : 64 * (R * NZ | 1) * (int)sizeof(TD);
+  __shared__ double tiles[2][TILE / 8];
+  const int lane = threadIdx.x & 63, k0 = blockIdx.x * 128 + (threadIdx.x & 64);
+  const int n = min(64, a.n_particles - k0);
+  if (n <= 0) return;  // the whole wave
+  const bool on = lane < n;
+  const int kq = k0 + min(lane, n - 1);  // bin-sorted position: Y/D row
+  const int p = a.sorted ? a.sorted[kq] : kq;  // particle id: state arrays
+  WaveRows<double> rows{tiles[threadIdx.x >> 6], lane, n};
+  double Ft[9], bt[9];
+  rows.template load<9>(a.F_old, p, Ft);
+  rows.template load<9>(a.b_old, p, bt);
   Axis ax[DIM];
   load_axes<DIM>(g, a.x, a.lp, p, ax);
   double H[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -448,39 +528,54 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
   double pp = 0, ppo = 0, ppa = 0, ppoa = 0;
   double graw[3] = {0, 0, 0};
   const int NB = L::NB;
-  // gather over the support, reference loop order (i outer ... k inner)
-  const int ez = (DIM == 3) ? ax[2].ext : 1;
+  // gather over the support, reference loop order (i outer ... k inner); the first two nodes of
+  // the last axis, which every particle has, are loaded together
+  auto load = [&](int i, int j, int k, double* un, double* uo) {
+    const int c[3] = {ax[0].lo + i, ax[1].lo + j, DIM == 3 ? ax[2].lo + k : 0};
+    const int node = node_index<DIM>(g, c);
+#pragma unroll
+    for (int cc = 0; cc < NB; ++cc) {
+      un[cc] = a.u_new[node * NB + cc];
+      uo[cc] = COUPLED ? a.u_old[node * NB + cc] : 0.0;
+    }
+  };
+  auto add = [&](int i, int j, int k, const double* un, const double* uo) {
+    const int o[3] = {i, j, k};
+    double w, G[3], wa, du[3];
+    node_geom<DIM>(ax, o, w, G, wa);
+#pragma unroll
+    for (int cc = 0; cc < DIM; ++cc) du[cc] = COUPLED ? un[cc] - uo[cc] : un[cc];
+#pragma unroll
+    for (int aa = 0; aa < DIM; ++aa)
+#pragma unroll
+      for (int cc = 0; cc < DIM; ++cc) H[aa][cc] += G[aa] * du[cc];
+    if (COUPLED) {
+#pragma unroll
+      for (int cc = 0; cc < DIM; ++cc) dup[cc] += w * du[cc];
+      const double pn = un[NB - 1], po = uo[NB - 1];
+      pp += w * pn;
+      ppo += w * po;
+      ppa += wa * pn;
+      ppoa += wa * po;
+#pragma unroll
+      for (int aa = 0; aa < DIM; ++aa) graw[aa] += G[aa] * pn;
+    }
+  };
+  const int el = ax[DIM - 1].ext;
   for (int i = 0; i < ax[0].ext; ++i)
-    for (int j = 0; j < ax[1].ext; ++j)
-      for (int k = 0; k < ez; ++k) {
-        int o[3] = {i, j, k};
-        int c[3] = {ax[0].lo + i, ax[1].lo + j, (DIM == 3) ? ax[2].lo + k : 0};
-        int node = node_index<DIM>(g, c);
-        double w, G[3], wa;
-        node_geom<DIM>(ax, o, w, G, wa);
-        double du[3];
-#pragma unroll
-        for (int cc = 0; cc < DIM; ++cc) {
-          du[cc] = a.u_new[node * NB + cc];
-          if (COUPLED) du[cc] -= a.u_old[node * NB + cc];
-        }
-#pragma unroll
-        for (int aa = 0; aa < DIM; ++aa)
-#pragma unroll
-          for (int cc = 0; cc < DIM; ++cc) H[aa][cc] += G[aa] * du[cc];
-        if (COUPLED) {
-#pragma unroll
-          for (int cc = 0; cc < DIM; ++cc) dup[cc] += w * du[cc];
-          double pn = a.u_new[node * NB + DIM];
-          double po = a.u_old[node * NB + DIM];
-          pp += w * pn;
-          ppo += w * po;
-          ppa += wa * pn;
-          ppoa += wa * po;
-#pragma unroll
-          for (int aa = 0; aa < DIM; ++aa) graw[aa] += G[aa] * pn;
-        }
+    for (int j = 0; j < (DIM == 3 ? ax[1].ext : 1); ++j) {
+      auto at = [&](int k) { return DIM == 3 ? k : 0; };
+      auto jt = [&](int k) { return DIM == 3 ? j : k; };
+      double n0[NB], o0[NB], n1[NB], o1[NB];
+      load(i, jt(0), at(0), n0, o0);
+      load(i, jt(1), at(1), n1, o1);
+      add(i, jt(0), at(0), n0, o0);
+      add(i, jt(1), at(1), n1, o1);
+      if (el == 3) {
+        load(i, jt(2), at(2), n0, o0);
+        add(i, jt(2), at(2), n0, o0);
       }
+    }
   // kinematics: incr_F = I + delta_u_GRAD (mpm_utils.py:510-517, 1199-1206)
   M3 f = m3_eye();
 #pragma unroll
@@ -498,14 +593,15 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
   } else {
     A = m3_inv(f);
   }
-  M3 Fo = m3_load(a.F_old + 9 * p);
+  M3 Fo, bo;
+  rows.template take<9>(Ft, &Fo.a[0][0]);
+  rows.template take<9>(bt, &bo.a[0][0]);
   M3 Fn = m3_mul(f, Fo);
   double J = m3_det(Fn);
   double Jo = m3_det(Fo);
-  M3 bo = m3_load(a.b_old + 9 * p);
   M3 btr = m3_mul(f, m3_mul(bo, m3_T(f)));
   MatParams mp;
-  mp.kind = a.mat_kind;
+  mp.kind = MAT;
   mp.dp_apex = a.dp_apex;
   mp.lam = a.lam;
   mp.mu = a.mu;
@@ -523,7 +619,7 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
   double alpha_o = a.alpha_old ? a.alpha_old[p] : 0.0;
   double alpha_n = alpha_o;
   M3 sig;
-  if (neo_hookean) {
+  if constexpr (neo_hookean) {
     // sigma = mu/J (F F^T - I) + lambda/J ln J I (mpm_utils.py:915)
     M3 FFt = m3_mul(Fn, m3_T(Fn));
     double lnJ = log(J);
@@ -536,17 +632,17 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
         tau.a[i][j] = sig.a[i][j] * J;
       }
     bn = btr;
-  } else if constexpr (!NHONLY) {
+  } else {
     hencky_family(btr, mp, alpha_o, ss, tau, bn, alpha_n);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j) sig.a[i][j] = tau.a[i][j] / J;
   }
-  m3_store(a.F_new + 9 * p, Fn);
-  m3_store(a.b_new + 9 * p, bn);
-  m3_store(a.sigma + 9 * p, sig);
-  if (a.alpha_new) a.alpha_new[p] = alpha_n;
+  rows.template store<9>(a.F_new, p, &Fn.a[0][0]);
+  rows.template store<9>(a.b_new, p, &bn.a[0][0]);
+  rows.template store<9>(a.sigma, p, &sig.a[0][0]);
+  if (a.alpha_new && on) a.alpha_new[p] = alpha_n;
 
   // ---- particle stress vector Y
   double V = a.p_vol * J;
@@ -591,7 +687,7 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
         Y[L::Y_T + 2] += pen_z;
       }
     }
-    if (a.pen_force) a.pen_force[p] = pen_in ? -pen_z : 0.0;
+    if (a.pen_force && on) a.pen_force[p] = pen_in ? -pen_z : 0.0;
     // mass balance and PPP (mpm_utils.py:1006-1015, 1284-1294)
     double lnJ = log(J), lnJo = log(Jo);
     Y[L::Y_Q] = (lnJ - lnJo) * V;
@@ -618,13 +714,12 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
     double cpp = (pp - ppa) - (ppo - ppoa);
     Y[L::Y_S] = tau_s * cpp * V;
   }
-#pragma unroll
-  for (int y = 0; y < L::NY; ++y) a.Y[(long)kq * L::NY + y] = Y[y];
+  rows.template put<NY>(Y);
+  rows.template flush<NY>(a.Y + (long)k0 * NY, NY, NY);
   if (!a.want_tangent) return;
 
-  // ---- tangent D = dY/dz, written column by column (every entry exactly once)
-  TD* D = (TD*)a.D + (long)kq * L::NY * L::NZ;
-  auto put = [&](int y, int z, double v) { D[y * L::NZ + z] = (TD)v; };
+  // ---- tangent D = dY/dz, row by row (every entry exactly once)
+  WaveRows<TD> drows{(TD*)tiles[threadIdx.x >> 6], lane, n};
   // M = tau - p J I; P = -V0 A^T M
   M3 Mm = tau;
   if (COUPLED)
@@ -640,9 +735,31 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
       for (int k = 0; k < DIM; ++k) s += A.a[k][i] * Mm.a[k][j];
       AtM.a[i][j] = s;
     }
-  M3 Bnh;  // F_old F^T for Neo-Hookean, b_old f^T for the Hencky family
-  if (neo_hookean) Bnh = m3_mul(Fo, m3_T(Fn));
-  else Bnh = m3_mul(bo, m3_T(f));
+  // d b = dH B + B^T dH^T: B = F_old F^T for Neo-Hookean (b = F F^T), b_old f^T for the Hencky family
+  const M3 B = neo_hookean ? m3_mul(Fo, m3_T(Fn)) : m3_mul(bo, m3_T(f));
+  // Hencky family: d tau of the symmetric unit tensors E_aj + E_ja (E_aa), pairs (0,0) (0,1) (0,2)
+  // (1,1) (1,2) (2,2); S = d tau / d ln J (NorSand's return depends on the specific volume)
+  constexpr int NP = DIM == 3 ? 6 : 5;
+  M3 K[NP], S;
+  if constexpr (!neo_hookean) {
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      const int pa = q < 3 ? 0 : (q < 5 ? 1 : 2), pj = q < 3 ? q : (q < 5 ? q - 2 : 2);
+      M3 db = m3_zero();
+      db.a[pa][pj] = db.a[pj][pa] = 1.0;
+      K[q] = spectral_dtau(ss, db);
+    }
+    if constexpr (MAT == MAT_NORSAND)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          double s = 0.0;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) s += ss.V.a[i][k] * ss.TJ[k] * ss.V.a[j][k];
+          S.a[i][j] = s;
+        }
+  }
   double lnJ = log(J), lnJo = log(Jo);
   // A^T A, A g, A^T g, A^T A g (mass-balance terms)
   double AtA[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -665,114 +782,104 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
 #pragma unroll
       for (int k = 0; k < DIM; ++k) AtAg[i] += A.a[k][i] * Ag[k];
   }
-  const double kdt = a.mobility * a.dt * a.p_vol;
-  for (int aa = 0; aa < DIM; ++aa)
-    for (int bb = 0; bb < DIM; ++bb) {
-      int z = aa * DIM + bb;  // column of dH_ab
-      double dJ = J * A.a[bb][aa];
-      M3 dtau;
-      if (neo_hookean) {
-        // d tau = mu (dH B + B^T dH^T) + lambda tr(A dH) I, B = F_old F^T
+  const double kdt = a.mobility * a.dt * a.p_vol, kdtJ = kdt * J, ts = 0.5 / a.mu * a.p_vol * J;
+  TD* D = (TD*)a.D + (long)k0 * NY * NZ;
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+  for (int y = 0; y < NY; ++y) {
+    double row[NZ];
 #pragma unroll
-          for (int j = 0; j < 3; ++j)
-            dtau.a[i][j] = a.mu * ((i == aa ? Bnh.a[bb][j] : 0.0) + (j == aa ? Bnh.a[bb][i] : 0.0)) +
-                           ((i == j) ? a.lam * A.a[bb][aa] : 0.0);
-      } else {
-        // d b_tr = dH C + C^T dH^T, C = b_old f^T; spectral tangent
-        M3 db;
+    for (int z = 0; z < NZ; ++z) row[z] = 0.0;
+    if (y < L::NH) {
+      // dP = -V0 [ dA^T M + A^T (dtau - p dJ I) ],  (dA^T X)[i][c] = -A[b][i] (A^T X)[a][c]
+      const int i = y / DIM, c = y % DIM;
+      double T[DIM][3], ab = 0.0;  // Hencky family: A^T d tau by (a, j); Neo-Hookean: (A^T B^T)_ib below
+      if constexpr (!neo_hookean) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+        for (int aa = 0; aa < DIM; ++aa)
 #pragma unroll
-          for (int j = 0; j < 3; ++j) db.a[i][j] = (i == aa ? Bnh.a[bb][j] : 0.0) + (j == aa ? Bnh.a[bb][i] : 0.0);
-        dtau = spectral_dtau(ss, db);
-        if (a.mat_kind == MAT_NORSAND) {
-          // the return also depends on ln J (specific volume): d ln J / d H_ab = A_ba
-          const double dlnJ = A.a[bb][aa];
+          for (int j = 0; j < 3; ++j) {
+            const int lo = aa < j ? aa : j, hi = aa < j ? j : aa, q = lo == 0 ? hi : (lo == 1 ? hi + 2 : 5);
+            double s = 0.0;
 #pragma unroll
-          for (int i = 0; i < 3; ++i)
+            for (int k = 0; k < DIM; ++k) s += A.a[k][i] * K[q].a[k][c];
+            T[aa][j] = aa == j ? 2.0 * s : s;
+          }
+        if constexpr (MAT == MAT_NORSAND)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
+          for (int k = 0; k < DIM; ++k) ab += A.a[k][i] * S.a[k][c];
+      }
+#pragma unroll
+      for (int aa = 0; aa < DIM; ++aa)
+#pragma unroll
+        for (int bb = 0; bb < DIM; ++bb) {  // column dH_ab
+          const double dJ = J * A.a[bb][aa];
+          double t2;
+          if constexpr (neo_hookean) {
+            // d tau = mu (dH B + B^T dH^T) + lambda tr(A dH) I
+            t2 = a.mu * A.a[aa][i] * B.a[bb][c] + A.a[c][i] * a.lam * A.a[bb][aa];
+            if (aa == c) {
               double s = 0.0;
 #pragma unroll
-              for (int k = 0; k < 3; ++k) s += ss.V.a[i][k] * ss.TJ[k] * ss.V.a[j][k];
-              dtau.a[i][j] += dlnJ * s;
+              for (int k = 0; k < DIM; ++k) s += A.a[k][i] * B.a[bb][k];
+              t2 += a.mu * s;
             }
-        }
-      }
-      // dP = -V0 [ dA^T M + A^T (dtau - p dJ I) ],  (dA^T X)[i][c] = -A[b][i] (A^T X)[a][c]
-#pragma unroll
-      for (int i = 0; i < DIM; ++i)
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) {
-          double t1 = -A.a[bb][i] * AtM.a[aa][c];
-          double t2 = 0.0;
-#pragma unroll
-          for (int k = 0; k < DIM; ++k) t2 += A.a[k][i] * (dtau.a[k][c] - ((COUPLED && k == c) ? pp * dJ : 0.0));
-          put(i * DIM + c, z, -a.p_vol * (t1 + t2));
-        }
-      if (!COUPLED) {
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) put(L::Y_T + c, z, 0.0);
-      } else {
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) put(L::Y_T + c, z, a.gravity[c] * a.p_vol * dJ);
-        put(L::Y_Q, z, a.p_vol * (1.0 + lnJ - lnJo) * dJ);
-#pragma unroll
-        for (int i = 0; i < DIM; ++i) {
-          double v;
-          if (DIM == 3) {
-            // m = kdt J A^T g
-            v = kdt * (J * (-A.a[bb][i] * Atg[aa]) + dJ * Atg[i]);
           } else {
-            // m = kdt J A^T A g ; d(A^T A g) = dA^T (A g) + A^T (dA g), (dA g)[k] = -A[k][a] (A g)[b]
-            double dAtAg = -A.a[bb][i] * AtAg[aa];
-            double AtdAg = 0.0;
+            t2 = ab * A.a[bb][aa];
 #pragma unroll
-            for (int k = 0; k < DIM; ++k) AtdAg += A.a[k][i] * (-A.a[k][aa] * Ag[bb]);
-            v = kdt * (dJ * AtAg[i] + J * (dAtAg + AtdAg));
+            for (int j = 0; j < 3; ++j) t2 += T[aa][j] * B.a[bb][j];
           }
-          put(L::Y_M + i, z, v);
+          if (COUPLED) t2 -= A.a[c][i] * pp * dJ;
+          row[aa * DIM + bb] = -a.p_vol * (t2 - A.a[bb][i] * AtM.a[aa][c]);
         }
-        put(L::Y_S, z, Y[L::Y_S] * A.a[bb][aa]);
-      }
-    }
-  if (COUPLED) {
-    double ts = 0.5 / a.mu * a.p_vol * J;
-    double kdtJ = kdt * J;
-    // column du_z (3D indenter penalty)
-    if (DIM == 3) {
+      if constexpr (COUPLED) row[L::Z_P] = a.p_vol * J * A.a[c][i];  // dP/dp = V0 J A^T
+    } else if constexpr (COUPLED) {
 #pragma unroll
-      for (int y = 0; y < L::NY; ++y) put(y, L::Z_DU, (y == L::Y_T + 2 && pen_in) ? a.pen_par : 0.0);
-    }
-    // column p: dP/dp = V0 J A^T, ds/dp = ts
+      for (int aa = 0; aa < DIM; ++aa)
 #pragma unroll
-    for (int y = 0; y < L::NY; ++y) {
-      double v = 0.0;
-      if (y < L::NH) {
-        int i = y / DIM, c = y % DIM;
-        v = a.p_vol * J * A.a[c][i];
-      } else if (y == L::Y_S) {
-        v = ts;
-      }
-      put(y, L::Z_P, v);
-    }
-    // column pbar: ds/dpbar = -ts
+        for (int bb = 0; bb < DIM; ++bb) {
+          const double dJ = J * A.a[bb][aa];
+          double v = 0.0;
+          if (y < L::Y_Q) {
+            v = a.gravity[y - L::Y_T] * a.p_vol * dJ;
+          } else if (y == L::Y_Q) {
+            v = a.p_vol * (1.0 + lnJ - lnJo) * dJ;
+          } else if (y < L::Y_S) {
+            const int i = y - L::Y_M;
+            if (DIM == 3) {
+              // m = kdt J A^T g
+              v = kdt * (J * (-A.a[bb][i] * Atg[aa]) + dJ * Atg[i]);
+            } else {
+              // m = kdt J A^T A g ; d(A^T A g) = dA^T (A g) + A^T (dA g), (dA g)[k] = -A[k][a] (A g)[b]
+              double dAtAg = -A.a[bb][i] * AtAg[aa];
+              double AtdAg = 0.0;
 #pragma unroll
-    for (int y = 0; y < L::NY; ++y) put(y, L::Z_PB, (y == L::Y_S) ? -ts : 0.0);
-    // columns grad p: dm/dg = kdt J A^T (3D) or kdt J A^T A (2D)
-#pragma unroll
-    for (int k = 0; k < DIM; ++k)
-#pragma unroll
-      for (int y = 0; y < L::NY; ++y) {
-        double v = 0.0;
-        if (y >= L::Y_M && y < L::Y_M + DIM) {
-          int i = y - L::Y_M;
-          v = kdtJ * (DIM == 3 ? A.a[k][i] : AtA[i][k]);
+              for (int k = 0; k < DIM; ++k) AtdAg += A.a[k][i] * (-A.a[k][aa] * Ag[bb]);
+              v = kdt * (dJ * AtAg[i] + J * (dAtAg + AtdAg));
+            }
+          } else {
+            v = Y[L::Y_S] * A.a[bb][aa];
+          }
+          row[aa * DIM + bb] = v;
         }
-        put(y, L::Z_G + k, v);
+      if (DIM == 3 && y == L::Y_T + 2 && pen_in) row[L::Z_DU] = a.pen_par;  // 3D indenter penalty
+      if (y == L::Y_S) {
+        row[L::Z_P] = ts;
+        row[L::Z_PB] = -ts;
       }
+      // dm/dg = kdt J A^T (3D) or kdt J A^T A (2D)
+      if (y >= L::Y_M && y < L::Y_S)
+#pragma unroll
+        for (int k = 0; k < DIM; ++k) row[L::Z_G + k] = kdtJ * (DIM == 3 ? A.a[k][y - L::Y_M] : AtA[y - L::Y_M][k]);
+    }
+    constexpr int TS = R * NZ | 1;
+    const int slot = y % R;
+    if (slot == 0) drows.sync();
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) drows.tile[lane * TS + slot * NZ + z] = (TD)row[z];
+    if (slot == R - 1 || y == NY - 1) {
+      drows.sync();
+      drows.template flush<R * NZ>(D + (y - slot) * NZ, NY * NZ, (slot + 1) * NZ);
+    }
   }
 }
 
@@ -782,16 +889,20 @@ extern "C" int gm_particle_stage(const gm_grid* g, const gm_stage_args* a, hipSt
   if (n == 0) return 0;
   GM_REQUIRE(!a->want_tangent || a->D, "gm_particle_stage: tangent requested without D");
   int blk = gm_blocks(n, 128);
-  const bool nh = a->mat_kind == MAT_NEOHOOKEAN;
-#define GM_STAGE(D, C)                                                                               \
-  do {                                                                                              \
-    if (nh) {                                                                                       \
-      if (a->tangent_fp32) k_particle_stage<D, C, float, true><<<blk, 128, 0, s>>>(*g, *a);         \
-      else k_particle_stage<D, C, double, true><<<blk, 128, 0, s>>>(*g, *a);                        \
-    } else {                                                                                        \
-      if (a->tangent_fp32) k_particle_stage<D, C, float, false><<<blk, 128, 0, s>>>(*g, *a);        \
-      else k_particle_stage<D, C, double, false><<<blk, 128, 0, s>>>(*g, *a);                       \
-    }                                                                                               \
+#define GM_STAGE_M(D, C, M)                                                                       \
+  do {                                                                                           \
+    if (a->tangent_fp32) k_particle_stage<D, C, float, M><<<blk, 128, 0, s>>>(*g, *a);            \
+    else k_particle_stage<D, C, double, M><<<blk, 128, 0, s>>>(*g, *a);                           \
+  } while (0)
+#define GM_STAGE(D, C)                                                  \
+  do {                                                                 \
+    switch (a->mat_kind) {                                             \
+      case MAT_NEOHOOKEAN: GM_STAGE_M(D, C, MAT_NEOHOOKEAN); break;    \
+      case MAT_J2: GM_STAGE_M(D, C, MAT_J2); break;                    \
+      case MAT_DP: GM_STAGE_M(D, C, MAT_DP); break;                    \
+      case MAT_NORSAND: GM_STAGE_M(D, C, MAT_NORSAND); break;          \
+      default: GM_STAGE_M(D, C, MAT_HENCKY);                           \
+    }                                                                  \
   } while (0)
   if (g->dim == 2 && !a->coupled) {
     GM_STAGE(2, false);
@@ -804,6 +915,7 @@ extern "C" int gm_particle_stage(const gm_grid* g, const gm_stage_args* a, hipSt
     return -1;
   }
 #undef GM_STAGE
+#undef GM_STAGE_M
   GM_LAUNCH_CHECK();
   return 0;
 }
