@@ -60,3 +60,35 @@ def test_stage_rows_do_not_depend_on_the_launch(name):
     for q, v in plain.items():
         assert bool(torch.isnan(v).all()) if q == 'D' else same(v, full[q]), q
     print(name, 'particles', n, 'max |D|', float(full['D'].abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('name', ['bar_hencky', 'terzaghi', 'indent_nh'])
+def test_g2p_of_any_particle_count(name):
+    """G2P of the first n particles (one, a block's edges): the states are copied, the positions are those
+    of the launch of all, and nothing behind the n rows is touched."""
+    import torch
+    s, _ = _state(name)
+    eng = s.engine
+    N, dim = s.x_particles.shape
+    gen = torch.Generator(device=s.device).manual_seed(5)
+    rnd = lambda *sh: torch.rand(sh, generator=gen, dtype=torch.float64, device=s.device)  # noqa: E731
+    new, old = 1e-3 * rnd(eng.n_nodes * eng.nb), 1e-3 * rnd(eng.n_nodes * eng.nb)
+    F, b, al = rnd(N, 9), rnd(N, 9), rnd(N)
+
+    def run(n):
+        x, lp = s.x_particles.clone(), s.GIMP_lp.clone()
+        Fo, bo, ao, pp = (torch.full(sh, -7.0, dtype=torch.float64, device=s.device) for sh in ((N, 9), (N, 9), N, N))
+        eng.g2p(x[:n], lp, new, old, Fo, F, bo, b, ao, al, pp)
+        torch.cuda.synchronize()
+        return x, Fo, bo, ao, pp
+
+    full = run(N)
+    assert torch.equal(full[1], F) and torch.equal(full[2], b) and torch.equal(full[3], al)
+    assert not torch.equal(full[0], s.x_particles)
+    start = (s.x_particles,) + tuple(torch.full_like(a, -7.0) for a in full[1:])
+    for n in (1, 127, 128, 129):
+        if n >= N:
+            continue
+        for got, want, before in zip(run(n), full, start):
+            assert torch.equal(got[:n], want[:n]) and torch.equal(got[n:], before[n:]), n
