@@ -122,6 +122,9 @@ _SIGS = {
                              ctypes.POINTER(c_double), _P]),
     'gm_bicgstab': (c_int, [c_int, c_int, c_int, _P, _P, _P, _P, _P, ctypes.POINTER(gm_krylov_ws), c_double, c_int,
                             c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_double), _P]),
+    'gm_pcg_window': (c_int, [ctypes.POINTER(gm_grid), ctypes.POINTER(gm_pattern), _P, _P, _P,
+                              ctypes.POINTER(gm_krylov_ws), c_double, c_int, c_int, c_int,
+                              ctypes.POINTER(c_int), ctypes.POINTER(c_double), _P]),
     'gm_pcg': (c_int, [c_int, c_int, c_int, _P, _P, _P, _P, _P, ctypes.POINTER(gm_krylov_ws), c_double, c_int,
                        c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_double), _P]),
     'gm_gmres': (c_int, [c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_double, c_int,

@@ -382,6 +382,19 @@ static void launch_lo_convert(int n_rows, const int* rp, const TM* vals, gm_half
 static int spmv_blocks(int n_rows, int nb) { return gm_blocks(n_rows, SPMV_T / spmv_lanes(nb)); }
 
 // ------------------------------------------------------------------ reductions
+// sum over the workgroup (RED_T threads) in a fixed order; every thread gets it
+__device__ __forceinline__ double block_sum(double s, double* sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = sh[0];
+#pragma unroll
+  for (int i = 1; i < RED_T / 64; ++i) s += sh[i];
+  return s;
+}
+
 // Sum `n` partial pairs (stride 2) deterministically into out[0], out[1].
 __global__ void k_sum_parts(const double* part, int n, double* out0, double* out1) {
   __shared__ double a[RED_T], b[RED_T];
@@ -880,13 +893,35 @@ __global__ void __launch_bounds__(PCG_WIDE) k_pcg_alpha(const double* part, int 
   }
 }
 
-// x += alpha p, r -= alpha q, z = Dinv r; per-workgroup partials of r.z and r.r
+// x += alpha p, r -= alpha q, z = Dinv r; per-workgroup partials of r.z and r.r.
+// pq_parts > 0: alpha is formed here, by every workgroup, from that many partial sums of p.q
+// (pq), with the rules of k_pcg_alpha; workgroup 0 stores it.
 template <int NB, typename TM, typename TV>
-__global__ void k_pcg_xr(int n_rows, const double* sc, TV* x, TV* r, const TV* p, const TV* q, const TM* dinv,
-                         TV* z, double* part) {
-  if (sc[C_DONE] != 0.0) return;
+__global__ void __launch_bounds__(RED_T) k_pcg_xr(int n_rows, const double* pq, int pq_parts, double* sc, TV* x, TV* r,
+                                                  const TV* p, const TV* q, const TM* dinv, TV* z, double* part) {
   __shared__ double a[RED_T], c[RED_T];
-  const double alpha = sc[C_ALPHA];
+  if (sc[C_DONE] != 0.0) {
+    if (pq_parts && blockIdx.x == 0 && threadIdx.x == 0) sc[C_GATE] = 1.0;
+    return;
+  }
+  double alpha;
+  if (pq_parts) {
+    double u = 0.0;
+    for (int i = threadIdx.x; i < pq_parts; i += RED_T) u += pq[i];
+    u = block_sum(u, a);
+    const double rz = sc[C_RZN];
+    const bool ok = u > 0.0 && u < 1e308 && sc[C_FLAG] == 0.0;
+    alpha = ok ? rz / u : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      sc[C_PQ] = u;
+      sc[C_RZ] = rz;
+      sc[C_ALPHA] = alpha;
+      if (!ok) sc[C_FLAG] = 1.0;
+    }
+    __syncthreads();  // a is used again
+  } else {
+    alpha = sc[C_ALPHA];
+  }
   double s0 = 0.0, s1 = 0.0;
   for (int row = blockIdx.x * RED_T + threadIdx.x; row < n_rows; row += gridDim.x * RED_T) {
 #pragma unroll
@@ -941,6 +976,65 @@ __global__ void __launch_bounds__(RED_T) k_pcg_p(long n, const double* part, int
     p[i] = (TV)((double)z[i] + beta * (double)p[i]);
 }
 
+// y = A x of a scalar matrix in a grid's window pattern (at most 5^DIM entries a row, in window
+// order), and the workgroups' partial sums of x.y.  The columns of a full row follow from its
+// number, so col_idx is read only for the rows the boundary cuts and no load of x waits for one.
+// G lanes a row, its entries and x loaded together.  Bound by HBM: 139,425 rows of 125 take 33 us
+// for 139 MB, 36 us with the columns read.  A workgroup takes several steps of rows so that p.q
+// comes as 1024 partial sums, few enough for every workgroup of the update to add up: a launch
+// (k_pcg_alpha, 4.6 us) less an iteration.  One step a workgroup: 31 us, but 16 for the update
+// (16 -> 6.5).  The next rows' entries loaded a step ahead: 49 us, for the registers they take.
+constexpr int WIN_T = 512, WIN_BLOCKS = 1024;
+template <int DIM>
+__global__ void __launch_bounds__(WIN_T) k_window_mv(int n_rows, int nx1, int nxy, const int* rp, const int* ci,
+                                                     const double* vals, const double* x, double* y, double* part,
+                                                     const double* gate) {
+  constexpr int W = DIM == 3 ? 125 : 25, G = DIM == 3 ? 16 : 8, U = (W + G - 1) / G;
+  __shared__ double sh[WIN_T / 64];
+  if (gate && *gate != 0.0) return;  // a gated launch after its solve has converged
+  const int lane = threadIdx.x % G;
+  int off[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int k = min(lane + G * u, W - 1);
+    off[u] = k % 5 - 2 + (k / 5 % 5 - 2) * nx1 + (DIM == 3 ? (k / 25 - 2) * nxy : 0);
+  }
+  double d = 0.0;
+  for (int row = blockIdx.x * (WIN_T / G) + threadIdx.x / G; row < n_rows; row += gridDim.x * (WIN_T / G)) {
+    const int s = rp[row], e = rp[row + 1];
+    double acc = 0.0;
+    if (e - s == W) {
+      double v[U], xv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        v[u] = vals[s + min(lane + G * u, W - 1)];
+        xv[u] = x[row + off[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc += lane + G * u < W ? v[u] * xv[u] : 0.0;
+    } else {
+      for (int k = s + lane; k < e; k += G) acc += vals[k] * x[ci[k]];
+    }
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, G);
+    if (lane == 0) {
+      y[row] = acc;
+      d += acc * x[row];
+    }
+  }
+  if (!part) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = d;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < WIN_T / 64; ++i) s += sh[i];
+    part[blockIdx.x] = s;
+  }
+}
+
 // lumped (row-sum) diagonal preconditioner of a scalar matrix: dinv = 1 / sum_k A_ik
 // (a consistent-mass matrix has non-negative entries and row sums equal to the lumped
 // nodal masses)
@@ -956,7 +1050,7 @@ __global__ void k_rowsum_inv(int n_rows, const int* rp, const TM* vals, TM* dinv
 template <int NB, typename TM, typename TV>
 static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, const TV* b, TV* x, gm_krylov_ws* ws,
                     double tol, int maxiter, int check_every, int options, int* iters_out, double* relres_out,
-                    hipStream_t st) {
+                    hipStream_t st, const gm_grid* window = nullptr) {
   const bool lumped = options & 1, warm = options & 2;
   long n = (long)n_rows * NB;
   TV *r = (TV*)ws->r, *p = (TV*)ws->p, *q = (TV*)ws->v, *z = (TV*)ws->z;
@@ -964,8 +1058,25 @@ static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, co
   double* sc = ws->sc;
   double* part = ws->part;
   const int rb = gm_blocks(n_rows, 256);
-  const int db = std::min(1024, gm_blocks(n_rows, RED_T));
+  // window: the pattern is the grid's; p.q comes as WIN_BLOCKS partial sums at most and the
+  // update forms alpha itself, its own partial pairs behind them (workspace: 2048 values)
+  const int db = std::min(window ? 512 : 1024, gm_blocks(n_rows, RED_T));
   const int sb = spmv_blocks(n_rows, NB);
+  const int wb = std::min(WIN_BLOCKS, gm_blocks(n_rows, WIN_T / (window && window->dim == 3 ? 16 : 8)));
+  double* xpart = window ? part + WIN_BLOCKS : part;
+  auto mv = [&](const TV* in, TV* out, double* pq, const double* gate) {
+    if constexpr (NB == 1 && sizeof(TM) == 8 && sizeof(TV) == 8) {
+      if (window) {
+        const int nx1 = window->nx + 1, nxy = nx1 * (window->ny + 1);
+        if (window->dim == 3)
+          k_window_mv<3><<<wb, WIN_T, 0, st>>>(n_rows, nx1, nxy, rp, ci, vals, in, out, pq, gate);
+        else
+          k_window_mv<2><<<wb, WIN_T, 0, st>>>(n_rows, nx1, nxy, rp, ci, vals, in, out, pq, gate);
+        return;
+      }
+    }
+    launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, in, out, pq ? in : nullptr, nullptr, pq, st, 0, gate);
+  };
   if (NB == 1 && lumped)
     k_rowsum_inv<TM><<<rb, 256, 0, st>>>(n_rows, rp, vals, dinv);
   else
@@ -973,7 +1084,7 @@ static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, co
   k_pcg_init_sc<<<1, 1, 0, st>>>(sc);
   k_dot2<TV><<<dot_blocks(n), RED_T, 0, st>>>(n, b, b, nullptr, nullptr, part);
   k_sum_parts<<<1, RED_T, 0, st>>>(part, dot_blocks(n), sc + C_BB, nullptr);
-  if (warm) launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, x, q, nullptr, nullptr, nullptr, st);
+  if (warm) mv(x, q, nullptr, nullptr);
   k_pcg_start<NB, TM, TV><<<db, RED_T, 0, st>>>(n_rows, b, warm ? q : nullptr, dinv, x, r, z, p, part);
   k_sum_parts<<<1, RED_T, 0, st>>>(part, db, sc + C_RZN, sc + C_RR);
   GM_LAUNCH_CHECK();
@@ -998,10 +1109,10 @@ static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, co
   while (it < maxiter && rel > tol) {
     const int nrun = std::min(check_every, maxiter - it);
     for (int k = 0; k < nrun; ++k) {
-      launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, p, q, p, nullptr, part, st, 0, sc + C_DONE);
-      k_pcg_alpha<<<1, PCG_WIDE, 0, st>>>(part, sb, sc);
-      k_pcg_xr<NB, TM, TV><<<db, RED_T, 0, st>>>(n_rows, sc, x, r, p, q, dinv, z, part);
-      k_pcg_p<TV><<<gm_blocks(n, RED_T), RED_T, 0, st>>>(n, part, db, sc, z, p, thr2);
+      mv(p, q, part, sc + C_DONE);
+      if (!window) k_pcg_alpha<<<1, PCG_WIDE, 0, st>>>(part, sb, sc);
+      k_pcg_xr<NB, TM, TV><<<db, RED_T, 0, st>>>(n_rows, part, window ? wb : 0, sc, x, r, p, q, dinv, z, xpart);
+      k_pcg_p<TV><<<gm_blocks(n, RED_T), RED_T, 0, st>>>(n, xpart, db, sc, z, p, thr2);
     }
     GM_LAUNCH_CHECK();
     GM_HIP(hipMemcpyAsync(hs, sc, sizeof(double) * C_NSC, hipMemcpyDeviceToHost, st));
@@ -1042,6 +1153,18 @@ extern "C" int gm_pcg(int nb, int fp32, int n_rows, const int* row_ptr, const in
 #undef GM_PCG
   gm::set_error("gm_pcg: unsupported block size %d", nb);
   return -1;
+}
+
+// gm_pcg for an FP64 scalar matrix in the grid's own pattern (the consistent mass)
+extern "C" int gm_pcg_window(const gm_grid* g, const gm_pattern* pat, const double* vals, const double* b, double* x,
+                             gm_krylov_ws* ws, double tol, int maxiter, int check_every, int options, int* iters,
+                             double* relres, hipStream_t s) {
+  GM_REQUIRE(g && pat && ws && iters && relres, "gm_pcg_window: null argument");
+  GM_REQUIRE(g->dim == 2 || g->dim == 3, "gm_pcg_window: dim must be 2 or 3");
+  GM_REQUIRE((long)(g->nx + 1) * (g->ny + 1) * (g->dim == 3 ? g->nz + 1 : 1) == g->n_nodes,
+             "gm_pcg_window: n_nodes does not match the grid");
+  return pcg_impl<1, double, double>(g->n_nodes, pat->row_ptr, pat->col_idx, vals, b, x, ws, tol, maxiter,
+                                     check_every < 1 ? 1 : check_every, options, iters, relres, s, g);
 }
 
 // y = A x  (A in FP64 or FP32, x and y in FP64 or FP32; FP64 accumulation)
@@ -1195,19 +1318,6 @@ extern "C" int gm_fix_empty_diag(int n_rows, const int* row_ptr, const int* col_
 // norm on the update, the second-pass decision and the final norm on the kernels that need them,
 // the column of H on the scaling.  One launch a quantity took 14 and a copy: 41 us a step on
 // 5,600 dofs (29 steps) against 17 us, 90 against 40 us on 557,700 dofs in FP32.
-
-// sum over the workgroup (RED_T threads) in a fixed order; every thread gets it
-__device__ __forceinline__ double block_sum(double s, double* sh) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  s = sh[0];
-#pragma unroll
-  for (int i = 1; i < RED_T / 64; ++i) s += sh[i];
-  return s;
-}
 
 // the partial sums of ||w||^2 that k_gs_axpy left, added in a fixed order
 __device__ __forceinline__ double norm_of_parts(const double* npart, int np, double* sh) {

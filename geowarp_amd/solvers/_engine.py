@@ -275,8 +275,10 @@ class Engine:
                 L.ptr(xp), L.ctypes.byref(ws), tol, maxiter)
         tail = (L.ctypes.byref(it), L.ctypes.byref(rr), _stream())
         # CG stops on the device; the host reads its state every 16 iterations
-        L.check(lib.gm_pcg(*head, 16, int(self.mass_lumped_pc) | (2 if x0 is not None else 0), *tail),
-                'gm_pcg(mass)')
+        L.check(lib.gm_pcg_window(L.ctypes.byref(self.grid), L.ctypes.byref(self.pattern), L.ptr(self.mvals),
+                                  L.ptr(mrhs), L.ptr(xp), L.ctypes.byref(ws), tol, maxiter, 16,
+                                  int(self.mass_lumped_pc) | (2 if x0 is not None else 0), *tail),
+                'gm_pcg_window(mass)')
         self.mass_solver = 'pcg'
         if not (rr.value <= tol):
             its = it.value
