@@ -78,7 +78,7 @@ def test_g2p_of_any_particle_count(name):
 
     def run(n):
         x, lp = s.x_particles.clone(), s.GIMP_lp.clone()
-        Fo, bo, ao, pp = (torch.full(sh, -7.0, dtype=torch.float64, device=s.device) for sh in ((N, 9), (N, 9), N, N))
+        Fo, bo, ao, pp = (torch.full(sh, -7.0, dtype=torch.float64, device=s.device) for sh in ((N, 9), (N, 9), (N,), (N,)))
         eng.g2p(x[:n], lp, new, old, Fo, F, bo, b, ao, al, pp)
         torch.cuda.synchronize()
         return x, Fo, bo, ao, pp
