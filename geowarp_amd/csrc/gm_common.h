@@ -4,8 +4,12 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include "gm_types.h"
+
 namespace gm {
 void set_error(const char* fmt, ...);
+void launch_mass(const gm_grid& g, const gm_bins& b, const gm_pattern& pat, double p_mass, double* mvals,
+                 hipStream_t s);
 }
 
 #define GM_HIP(call)                                                                  \

@@ -1666,21 +1666,18 @@ extern "C" int gm_penalty_pc(const gm_grid* g, const gm_bins* b, const gm_patter
 // Node-gather form of P2G_2d / P2G_coupled_2d / P2G_coupled_3d (mpm_utils.py:83-383).
 //  act:     activation (threshold < 0: every support node, as P2G_2d; else w > threshold)
 //  bflag:   pressure-Dirichlet flags are OR-ed into the p dof (coupled)
-//  mvals:   consistent mass in the node pattern (b = 1), may be null
 //  mrhs:    consistent-mass rhs, may be null
 template <int DIM>
 __global__ void k_p2g(gm_grid g, int nb, const double* x_s, const double* lp_s, const int* cell_start,
                       const int* sorted, const uint8_t* ext_s, double threshold, const uint8_t* pbc_flag,
-                      double node_h_last, double p_mass, const double* p_part, const int* row_ptr,
-                      const uint64_t* row_mask, uint8_t* act, uint8_t* bflag, double* mvals, double* mrhs) {
+                      double node_h_last, double p_mass, const double* p_part, uint8_t* act, uint8_t* bflag,
+                      double* mrhs) {
   int I = blockIdx.x * blockDim.x + threadIdx.x;
   if (I >= g.n_nodes) return;
   int ci[3] = {0, 0, 0};
   node_coords<DIM>(g, I, ci);
   bool a_on = false, pb = false;
   double rhs = 0.0;
-  int rp = row_ptr ? row_ptr[I] : 0;
-  uint64_t m0 = row_mask ? row_mask[2 * I] : 0, m1 = row_mask ? row_mask[2 * I + 1] : 0;
   for_candidates<DIM>(g, ci, cell_start, ext_s, [&](int k, const int* o, const int* b, bool in) {
     int p = sorted[k];
     // pressure boundary: 2D loops over the support, 3D over all 27 nodes (mpm_utils.py:225-235, 349-352)
@@ -1694,36 +1691,12 @@ __global__ void k_p2g(gm_grid g, int nb, const double* x_s, const double* lp_s, 
     double w, G[3], wa;
     node_geom<DIM>(ax, o, w, G, wa);
     if (threshold < 0.0 || w > threshold) a_on = true;
-    if (DIM == 3 && !mvals && mrhs) {
-      // sum of the particle's weights over its support, one axis at a time (the
-      // 3D mass matrix comes from gm_mass_binned)
+    if (mrhs) {
+      // sum of the particle's weights over its support, one axis at a time
       double wsum = 1.0;
 #pragma unroll
-      for (int aa = 0; aa < 3; ++aa) wsum *= ax[aa].w[0] + ax[aa].w[1] + ax[aa].w[2];
+      for (int aa = 0; aa < DIM; ++aa) wsum *= ax[aa].w[0] + ax[aa].w[1] + ax[aa].w[2];
       rhs += w * wsum * p_mass * p_part[p];
-    } else if (mvals || mrhs) {
-      double wsum = 0.0;
-      uint8_t ex = ext_s[k];
-      int e[3];
-#pragma unroll
-      for (int aa = 0; aa < DIM; ++aa) e[aa] = ((ex >> aa) & 1) ? 3 : 2;
-      const int kz_n = (DIM == 3) ? e[2] : 1;
-      for (int kx = 0; kx < e[0]; ++kx)
-        for (int ky = 0; ky < e[1]; ++ky)
-          for (int kz = 0; kz < kz_n; ++kz) {
-            int oJ[3] = {kx, ky, kz};
-            double wJ, GJ[3], waJ;
-            node_geom<DIM>(ax, oJ, wJ, GJ, waJ);
-            wsum += wJ;
-            if (mvals) {
-              int rx = kx - o[0] + 2, ry = ky - o[1] + 2, rz = (DIM == 3) ? kz - o[2] + 2 : 0;
-              int bit = rx + 5 * ry + 25 * rz;
-              int before = (bit < 64) ? __popcll(m0 & ((1ull << bit) - 1ull))
-                                      : __popcll(m0) + __popcll(m1 & ((1ull << (bit - 64)) - 1ull));
-              mvals[rp + before] += w * wJ * p_mass;
-            }
-          }
-      if (mrhs) rhs += w * wsum * p_mass * p_part[p];
     }
   });
   if (a_on)
@@ -1739,18 +1712,15 @@ extern "C" int gm_p2g(const gm_grid* g, const gm_bins* b, const gm_pattern* pat,
   int n = g->n_nodes;
   if (mvals) {
     GM_REQUIRE(pat, "gm_p2g: mass matrix needs the pattern");
-    GM_HIP(hipMemsetAsync(mvals, 0, sizeof(double) * pat->nnzb, s));
+    gm::launch_mass(*g, *b, *pat, p_mass, mvals, s);
+    GM_LAUNCH_CHECK();
   }
-  const int* rp = pat ? pat->row_ptr : nullptr;
-  const uint64_t* rm = pat ? pat->row_mask : nullptr;
   if (g->dim == 2)
     k_p2g<2><<<gm_blocks(n, 128), 128, 0, s>>>(*g, g->nb, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold,
-                                               pbc_flag, node_h_last, p_mass, p_part, rp, rm, act, bflag, mvals,
-                                               mrhs);
+                                               pbc_flag, node_h_last, p_mass, p_part, act, bflag, mrhs);
   else
     k_p2g<3><<<gm_blocks(n, 128), 128, 0, s>>>(*g, g->nb, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold,
-                                               pbc_flag, node_h_last, p_mass, p_part, rp, rm, act, bflag, mvals,
-                                               mrhs);
+                                               pbc_flag, node_h_last, p_mass, p_part, act, bflag, mrhs);
   GM_LAUNCH_CHECK();
   return 0;
 }

@@ -89,3 +89,42 @@ def test_window_cg_reports_what_the_general_cg_reports():
     assert rc == 0 and its == 0 and float(x.abs().max()) == 0.0
     rc, its, rel, x = solve(b, -eng.mvals)
     assert rc == 0 and its <= 200 and rel > 1e-12
+
+
+# fewer rows than a strip of 21, remainders, grid lines shorter and longer than a strip, and (crowd) bins
+# whose ranges take several pieces of 96 particles
+@pytest.mark.gpu
+@pytest.mark.parametrize('cells', [(2, 2), (3, 6), (20, 3), (41, 7), (2, 2, 2), (6, 4, 3), (21, 3, 4), (3, 5, 9)])
+@pytest.mark.parametrize('crowd', [False, True])
+def test_mass_matrix_equals_the_dense_sum(cells, crowd):
+    """M_IJ = m sum_p w_I w_J with the oracle's weights, every entry of the pattern written; the
+    right-hand side is m sum_p w_I p_p sum_J w_J."""
+    import torch
+    import oracle.gimp as og
+    eng, b, x, lp = _mass_system(cells, 8 if crowd else 2, seed=1)
+    dim, N = len(cells), eng.n_nodes
+    lo, w, _, _, _ = zip(*[og.axis_weights(x[:, a], lp[:, a], 0.5, 2.0) for a in range(dim)])
+    # dense products one axis at a time: W_a (particles x nodes of the axis)
+    W = []
+    for a in range(dim):
+        Wa = np.zeros((len(x), cells[a] + 3))
+        for i in range(3):
+            np.add.at(Wa, (np.arange(len(x)), lo[a] + i), w[a][:, i])
+        W.append(Wa[:, :cells[a] + 1])
+    P = W[0]
+    for a in range(1, dim):
+        P = np.einsum('pi,pj->pij', W[a], P.reshape(len(x), -1)).reshape(len(x), -1)  # x fastest
+    M = 0.7 * P.T @ P
+    rp, ci = eng.row_ptr[:N + 1].cpu().numpy(), eng.col_idx[:eng.nnzb].cpu().numpy()
+    got = np.zeros((N, N))
+    got[np.repeat(np.arange(N), np.diff(rp)), ci] = eng.mvals[:eng.nnzb].cpu().numpy()
+    err = np.abs(got - M).max() / np.abs(M).max()
+    print(cells, crowd, 'particles', len(x), 'entries', eng.nnzb, 'max error', err)
+    assert err < 1e-13  # sums of up to a few thousand positive terms of 1e-16 each
+    eng.mvals.fill_(float('nan'))
+    X, LP = (torch.as_tensor(np.ascontiguousarray(q), device=eng.dev) for q in (x, lp))
+    pp = torch.as_tensor(np.random.default_rng(2).standard_normal(len(x)), device=eng.dev)
+    b = eng.p2g(X, LP, 1e-9, torch.zeros(len(x), dtype=torch.uint8, device=eng.dev), 0.0, 0.7, pp, mass=True)
+    assert not bool(torch.isnan(eng.mvals[:eng.nnzb]).any())
+    r = 0.7 * P.T @ (pp.cpu().numpy() * P.sum(1))
+    assert np.abs(b.cpu().numpy() - r).max() < 1e-12 * np.abs(r).max()
