@@ -19,11 +19,13 @@
 //                 sign and identity rows as in the node-row kernels.
 // Both steps are deterministic (fixed accumulation order).  The workspace holds n_nodes x
 // 6480 values, written once and read once per assembly.
-//   64 x 64 x 32 cells, 1,048,576 particles (MI355X), per assembly: FP32 2.60 + 1.06 ms
+//   64 x 64 x 32 cells, 1,048,576 particles (MI355X), per assembly: FP32 2.23 + 1.05 ms
 //   (one workgroup per bin, 11664 values per node in the workspace: 2.84 + 1.56 ms), FP64
-//   4.1 + 1.95 ms (5.6 + 2.9).  k_jac_line issues its products at 40 % (FP32) and 50 %
-//   (FP64) of the matrix rate; the rest is the operand waves' FP64 arithmetic, which shares
-//   the SIMDs with the products.  k_jac_gather moves 4.7 GB (FP32) at 4.4 TB/s.
+//   4.0 + 1.83 ms (5.6 + 2.9).  k_jac_line: the products take 0.95 (FP32) and 1.3 ms (FP64),
+//   the stores of the line sums 0.7 and 1.95 (3.6 and 7.2 GB), and one follows the other in the
+//   product waves; the operand waves' FP64 arithmetic adds 0.4 and 0.2.  With the shape-function
+//   tables made by an operand wave rather than the last product wave FP32 took 2.60.
+//   k_jac_gather moves 4.7 GB (FP32) at 4.5 TB/s.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -99,6 +101,11 @@ __device__ __forceinline__ int zsel(int c, int beta) {
   if (beta == 4) return Z_PB;
   return Z_G + beta - 1;
 }
+
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
 
 constexpr int MAX_SEG = 61;  // bins of a line segment (with two before it and the end, one a lane)
 
@@ -189,6 +196,35 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
   };
   Group cur{x0, 0, 0};
   seek(cur);
+  // shape-function tables of particles [tabs, tabs + BATCH) of the sweep: 48 lanes of the last
+  // product wave, which has a row tile less than the first ones, from positions loaded one batch
+  // ahead (one wave's FP64 chain a batch rather than a group)
+  const int ps = cs(x0), n_sweep = cs(xe) - ps;
+  const int tl = wave == CW - 1 ? lane : -1;
+  const int tp = tl >= 0 && tl < 3 * BATCH ? tl / 3 : 0, ta = tl >= 0 ? tl % 3 : 0;
+  int tabs = 0;
+  double xa, la;
+  auto load_tables = [&](int e) {
+    const long at = (long)(ps + min(e + tp, n_sweep - 1)) * 3 + ta;
+    xa = x_s[at];
+    la = lp_s[at];
+  };
+  // q: the last group of a round (none: the sweep ends in that round)
+  auto tables_for = [&](const Group& q) {
+    if ((q.x < xe ? min(q.p0 + PG, q.ke) - ps : n_sweep) <= tabs) return;  // uniform
+    if (tl >= 0 && tl < 3 * BATCH) {
+      const Axis ax = gimp_axis(xa, la, g.h[ta], g.inv_h[ta]);
+      double* T = AXT_[(tabs + tp) % RING][ta];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        T[i] = ax.w[i];
+        T[3 + i] = ax.g[i];
+        T[6 + i] = ax.wa[i];
+      }
+    }
+    tabs += BATCH;
+    load_tables(tabs);
+  };
   if (wave < CW) {
     // ---------------------------------------------------------------- products
     typedef typename Mfma<TC>::acc ACC;
@@ -235,26 +271,49 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
         }
       }
     };
+    Group gt = cur;  // the last group of the round whose tables come next
+    if (wave == CW - 1) {
+#pragma unroll
+      for (int k = 1; k < TEAMS; ++k) gt = next(gt);
+      load_tables(0);
+      tables_for(gt);
+      gt = next_round(gt);
+      tables_for(gt);
+    }
     __syncthreads();
     __syncthreads();
     for (int buf = 0; cur.x < xe; buf ^= 1) {
+      if (wave == CW - 1) {
+        gt = next_round(gt);
+        tables_for(gt);
+      }
 #pragma unroll 1
       for (int k = 0; k < TEAMS && cur.x < xe; ++k) {
+        // particles past the bin's last have zero B; a tile's operands are read before its products
         const TC *E = E_[k][buf], *BT = BT_[k][buf];
-        // particles past the bin's last have zero B
+        TC b[5];
 #pragma unroll
-        for (int beta = 0; beta < 5; ++beta) {
-          const TC bk = BT[bbase + beta * BB];
+        for (int beta = 0; beta < 5; ++beta) b[beta] = BT[bbase + beta * BB];
+        auto products = [&](auto tile) {
+          constexpr int s = decltype(tile)::value;
+          TC a[4][5];
 #pragma unroll
-          for (int s = 0; s < TILES; ++s) {
-            if (s == TILES - 1 && !last) break;  // wave-uniform
+          for (int beta = 0; beta < 5; ++beta)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const int z = zsel(c, beta);  // resolved at compile time
-              if (z != ZERO) acc[s][c] = Mfma<TC>::step(E[abase[s] + z * 4], bk, acc[s][c]);
-            }
-          }
+            for (int c = 0; c < 4; ++c)
+              if (zsel(c, beta) != ZERO) a[c][beta] = E[abase[s] + zsel(c, beta) * 4];
+#pragma unroll
+          for (int beta = 0; beta < 5; ++beta)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)  // (c, beta) resolved at compile time
+              if (zsel(c, beta) != ZERO) acc[s][c] = Mfma<TC>::step(a[c][beta], b[beta], acc[s][c]);
+        };
+        if constexpr (TILES == 4) {
+          products(Int<0>{});
+          products(Int<1>{});
         }
+        products(Int<TILES - 2>{});
+        if (last) products(Int<TILES - 1>{});  // wave-uniform
         const Group nxt = next(cur);
         if (nxt.x != cur.x) {  // the bin's last group
           if (BIN_SUMS) {
@@ -304,35 +363,6 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
       }
     }
   };
-  // shape-function tables of particles [tabs, tabs + BATCH) of the sweep: 48 lanes of the
-  // last wave, from positions loaded one batch ahead (one wave's FP64 chain a batch rather
-  // than a group)
-  const int ps = cs(x0), n_sweep = cs(xe) - ps;
-  const int tl = team == TEAMS - 1 ? t - 192 : -1;
-  const int tp = tl >= 0 && tl < 3 * BATCH ? tl / 3 : 0, ta = tl >= 0 ? tl % 3 : 0;
-  int tabs = 0;
-  double xa, la;
-  auto load_tables = [&](int e) {
-    const long at = (long)(ps + min(e + tp, n_sweep - 1)) * 3 + ta;
-    xa = x_s[at];
-    la = lp_s[at];
-  };
-  // q: the last group of a round (none: the sweep ends in that round)
-  auto tables_for = [&](const Group& q) {
-    if ((q.x < xe ? min(q.p0 + PG, q.ke) - ps : n_sweep) <= tabs) return;  // uniform
-    if (tl >= 0 && tl < 3 * BATCH) {
-      const Axis ax = gimp_axis(xa, la, g.h[ta], g.inv_h[ta]);
-      double* T = AXT_[(tabs + tp) % RING][ta];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        T[i] = ax.w[i];
-        T[3 + i] = ax.g[i];
-        T[6 + i] = ax.wa[i];
-      }
-    }
-    tabs += BATCH;
-    load_tables(tabs);
-  };
   auto operands = [&](const Group& q, int buf) {
     const int np = min(PG, q.ke - q.p0), rot = q.x % 3;  // node ox of the bin lies in slot (ox + rot) % 3
     // B operand: threads (J, particle)
@@ -375,7 +405,7 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
         gz[i] = AX[2][3 + i];
         az[i] = AX[2][6 + i];
       }
-#pragma unroll 1
+#pragma unroll
       for (int ix = 0; ix < 3; ++ix) {
         TC* Eo = E_[team][buf] + p * EP + zr + 9 * EI * (ix + rot >= 3 ? ix + rot - 3 : ix + rot);
         const double wx = AX[0][ix], u = AX[0][3 + ix] * d0 + wx * dw, v = wx * d1, qx = wx * d2, a = AX[0][6 + ix] * dwa;
@@ -392,13 +422,10 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
   Group g0 = cur;
   for (int k = 0; k < team; ++k) g0 = next(g0);
   Group g1 = next_round(g0), g2 = next_round(g1), g3 = next_round(g2);
-  load_tables(0);
   load_group(g0, even);
   load_group(g1, odd);
   stage_group(g0, 0, even);
   load_group(g2, even);
-  tables_for(g0);
-  tables_for(g1);
   __syncthreads();
   if (g0.x < xe) operands(g0, 0);
   stage_group(g1, 1, odd);
@@ -409,7 +436,6 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
   while (cur.x < xe) {
     if (g1.x < xe) operands(g1, 1);
     stage_group(g2, 0, even);
-    tables_for(g2);
     const Group g4 = next_round(g3);
     load_group(g4, even);
     __syncthreads();
@@ -417,7 +443,6 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
     if (cur.x >= xe) break;
     if (g2.x < xe) operands(g2, 0);
     stage_group(g3, 1, odd);
-    tables_for(g3);
     g1 = g3;
     g2 = g4;
     g3 = next_round(g4);
@@ -465,8 +490,11 @@ __global__ void __launch_bounds__(T) k_jac_gather(gm_grid g, const int* cell_sta
   const int slot = bit < 64 ? __popcll(m0 & ((1ull << (bit & 63)) - 1ull))
                             : __popcll(m0) + __popcll(m1 & ((1ull << (bit & 63)) - 1ull));
   __syncthreads();
-#pragma unroll 1
-  for (int c = t >> 7; c < 4; c += T / 128) {
+  // column dofs a thread has in flight: all of them in FP64 (1.95 -> 1.83 ms), one in FP32 (1.06; all 1.09)
+  constexpr int UC = sizeof(TC) == 8 ? 4 * 128 / T : 1;
+#pragma unroll UC
+  for (int c0 = 0; c0 < 4 * 128 / T; ++c0) {
+    const int c = (t >> 7) + c0 * (T / 128);
     V4 v[9];
     bool on[9];
 #pragma unroll
@@ -861,18 +889,21 @@ int cu_count() {
   return n;
 }
 
-// Segments of a bin line: every segment after the first repeats the products of two bins,
-// and the last round of workgroups may leave slots idle.  The number of segments with the
-// least rounds x (bins of a segment + 2); lines without particles end at once and are
-// left out of the count (some six particles a bin are taken for granted).
+// Segments of a bin line: every segment after the first repeats the products of two bins, and
+// the workgroups do not come out even over the CUs: the number of segments with the least
+// (rounds + 1/2) x (bins of a segment + 2), at least one round.  The half round is what the
+// lines without particles (which end at once) and the XCDs' shares make of the last one: whole
+// rounds instead pick 1, 3 and 3 segments for 21 x 17 x 13, 48 x 9 x 7 and 64 x 64 x 32 cells,
+// 249, 149 and 2268 us in FP32 where 2, 6 and 2 take 212, 117 and 2233.  (Some six particles a
+// bin are taken for granted.)
 int best_segments(int nbx, int lines, int n_p, int slots) {
-  const long busy = std::max(1L, std::min<long>(lines, (long)n_p / (6L * nbx)));
+  const double busy = std::max(1.0, std::min<double>(lines, n_p / (6.0 * nbx)));
   int best = 1;
-  long cost = 0;
+  double cost = 0.0;
   for (int k = (nbx + MAX_SEG - 1) / MAX_SEG; k <= (nbx + 1) / 2; ++k) {
     const int len = (nbx + k - 1) / k;
-    const long c = ((busy * k + slots - 1) / slots) * (len + (k > 1 ? 2 : 0));
-    if (cost == 0 || c < cost) {
+    const double c = std::max(1.0, busy * k / slots + 0.5) * (len + (k > 1 ? 2 : 0));
+    if (cost == 0.0 || c < cost) {
       cost = c;
       best = k;
     }
