@@ -1673,11 +1673,29 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
   if (bnorm == 0.0) return 0;
   std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m), hcol(m + 2);
   const int nsl = 2 * (m + 2), gate = 2 * m + 6;
+  // a step's column of H comes back in one of two halves of the pinned buffer, its arrival marked
+  // by an event of the same parity: the next step is queued before this one's column is looked at
+  // when two more steps at the last one's rate would not reach the tolerance, so that the stream
+  // does not wait for the host: load steps of small grids 3 % faster (3.26 -> 3.17 and 7.51 -> 7.26
+  // ms), the gradient of a load path 11 %.  A step queued in vain writes nothing that is read.
+  const int half = 3 * (m + 2);
   double* host = nullptr;
   {
-    int prc = pinned_buffer(3 * (m + 2), &host);
+    int prc = pinned_buffer(2 * half, &host);
     if (prc) return prc;
   }
+  struct Events {
+    hipStream_t st;
+    bool busy = false;  // a step may be on its way: no return before it has written its column
+    hipEvent_t e[2] = {nullptr, nullptr};
+    explicit Events(hipStream_t s) : st(s) {}
+    ~Events() {
+      if (busy) (void)hipStreamSynchronize(st);
+      for (auto q : e)
+        if (q) (void)hipEventDestroy(q);
+    }
+  } events(st);
+  for (auto& e : events.e) GM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   StepGraphs* sg = nullptr;
   if (graphs_on()) {
     std::vector<char> key;
@@ -1729,7 +1747,8 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
     k_scale_copy<TV><<<vb, RED_T, 0, st>>>(n, V, 1.0 / beta, V);
     std::fill(g.begin(), g.end(), 0.0);
     g[0] = beta;
-    int j = 0;
+    int j = 0, queued = 0;
+    double rate = 0.1;  // residual reduction of the last step
     for (; j < m && total < maxiter; ++j, ++total) {
       // one Arnoldi step on the device: z_j = M^-1 v_j, w = A z_j, classical Gram-Schmidt
       // with selective reorthogonalisation (Daniel, Gragg, Kaufman & Stewart 1976: a second
@@ -1737,7 +1756,7 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
       // v_{j+1} = w / ||w||, and the column of H stored to pinned host memory.  dh: [0, m+2)
       // pass-1 coefficients, [m+2, 2m+4) pass-2 coefficients, [2m+4] ||w||^2 after the
       // passes, [2m+5] before them, [2m+6] the second-pass flag.
-      auto enqueue = [&, j](hipStream_t q) -> int {
+      auto enqueue = [&](int j, hipStream_t q) -> int {
         TV* vj = V + (long)j * ldv;
         TV* vj1 = V + (long)(j + 1) * ldv;
         TV* zj = Zs ? Zs + (long)j * ldv : z;
@@ -1752,14 +1771,19 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
         k_gs_dots<TV><<<dim3(nchunk, j + 1), RED_T, 0, q>>>(n, j + 1, V, ldv, w, nchunk, part, npart, ab, sc);
         if (!fold) k_gs_fin<<<j + 1, RED_T, 0, q>>>(sc + 2, j + 1, nchunk, part, h2, nullptr);
         k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(sc + 2, n, j + 1, V, ldv, part, fc, h2, nullptr, w, npart);
-        k_gs_scale<TV><<<vb, RED_T, 0, q>>>(n, j + 1, w, npart, ab, dh, h2, sc, vj1, host, m + 2);
+        k_gs_scale<TV><<<vb, RED_T, 0, q>>>(n, j + 1, w, npart, ab, dh, h2, sc, vj1,
+                                               host + (j & 1) * half, m + 2);
         GM_LAUNCH_CHECK();
         return 0;
       };
-      int prc = run_step(sg, j, st, enqueue);
-      if (prc) return prc;
-      GM_HIP(hipStreamSynchronize(st));
-      const double* hh = host;
+      for (; queued <= j || (queued == j + 1 && queued < m && total + 1 < maxiter && rel * rate * rate > tol); ++queued) {
+        events.busy = true;
+        int prc = run_step(sg, queued, st, [&](hipStream_t q) { return enqueue(queued, q); });
+        if (prc) return prc;
+        GM_HIP(hipEventRecord(events.e[queued & 1], st));
+      }
+      GM_HIP(hipEventSynchronize(events.e[j & 1]));
+      const double* hh = host + (j & 1) * half;
       const bool second = hh[gate] != 0.0;
       for (int i = 0; i <= j; ++i) hcol[i] = second ? hh[i] + hh[(m + 2) + i] : hh[i];
       double hn = sqrt(fmax(hh[nsl], 0.0));
@@ -1785,7 +1809,9 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
       g[j + 1] = -sn[j] * g[j];
       g[j] = cs[j] * g[j];
       for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = hcol[i];
+      const double was = rel;
       rel = fabs(g[j + 1]) / bnorm;
+      rate = std::min(1.0, rel / was);
       if (rel <= tol || hn == 0.0) {
         ++j;
         ++total;
@@ -1810,6 +1836,7 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
       if (prc) return prc;
     }
     GM_HIP(hipStreamSynchronize(st));
+    events.busy = false;
     if (rel <= tol) break;
   }
   *iters_out = total;
