@@ -960,6 +960,11 @@ struct Strip2d {
       ke[ox] = ok ? cell_start[b + 1] : 0;
     }
   }
+  // a split's first particle of a bin that starts at ks, in the piece that starts at k0
+  static __device__ __forceinline__ int first(int ks, int k0, int split, int n) {
+    const int k = ks + split;  // then every n-th
+    return k >= k0 ? k - k0 : (n - (k0 - k) % n) % n;
+  }
   // particles [k0, k0 + n) into the wave's piece
   static __device__ __forceinline__ void stage(const gm_grid& g, const double* x_s, const double* lp_s,
                                                const uint8_t* ext_s, const TY* rows, int k0, int n, Piece& p) {
@@ -996,26 +1001,33 @@ struct Strip2d {
   }
 };
 
-// A lane per (row, dof).  Bound by the LDS reads of each row's 36 candidates.  A thread per row
-// walked the nine bins in global memory and evaluated every particle's axis data nine times.
-// 1,048,576 particles, 264,000 rows, single phase: 281 -> 98 us; 45,000 particles u-p: 32 -> 20 us.
+// A lane per (row, dof, every fourth particle).  Bound by the staging of the particles' rows: a
+// thread per row walked the nine bins in global memory and evaluated every particle's axis data
+// nine times.  Strips of 8 rows (5 u-p), so that a piece of 40 particles holds a line's range and
+// no lane waits for its bins: 32 (21) rows with pieces of 56 (40) and a lane for all of a bin's
+// particles take 98 and 20 us where this takes 94 and 10, 16 rows with two lanes 109 and 12, 4
+// with seven 130 and 12.  1,048,576 particles, 264,000 rows, single phase: 281 -> 94 us; 45,000
+// particles u-p: 32 -> 10 us.  (The Jacobian gains nothing from it: see below.)
+constexpr int RES_ROWS = 8, RES_ROWS_UP = 5, RES_SPLIT = 4, RES_C = 40;
+
 template <bool COUPLED>
 __global__ void __launch_bounds__(192) k_strip_residual(gm_grid g, const double* x_s, const double* lp_s,
                                                         const int* cell_start, const uint8_t* ext_s, const double* Y,
                                                         const uint8_t* freem, double* rhs) {
   typedef Lay<2, COUPLED> L;
-  constexpr int NB = L::NB, NY = L::NY, ROWS = 64 / NB, C = COUPLED ? 40 : 56;
+  constexpr int NB = L::NB, NY = L::NY, ROWS = COUPLED ? RES_ROWS_UP : RES_ROWS, SPLIT = RES_SPLIT, C = RES_C;
   typedef Strip2d<COUPLED, double, ROWS, NY, C> S;
   constexpr int NT = S::NT;
   __shared__ typename S::Piece piece[3];
   __shared__ double OUT[3][ROWS * NB];
-  const int lane = threadIdx.x & 63, row = lane / NB, c = lane % NB;
+  constexpr int PART = ROWS * NB;  // lanes of a split
+  const int lane = threadIdx.x & 63, split = lane / PART, row = lane % PART / NB, c = lane % PART % NB;
   const int I0 = S::first_row(), I = I0 + row;
   const int oy = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   typename S::Piece& p = piece[oy];
   int lo, hi, ks[3], ke[3];
   S::range(g, I0, oy, cell_start, &lo, &hi);
-  S::bins(g, I, row < ROWS && I < g.n_nodes, oy, cell_start, ks, ke);
+  S::bins(g, I, split < SPLIT && I < g.n_nodes, oy, cell_start, ks, ke);
   // the dof's rows of Y
   const int y0 = c < 2 ? c : L::Y_M, y1 = c < 2 ? 2 + c : L::Y_M + 1, y2 = c < 2 ? L::Y_T + c : L::Y_Q;
   double acc = 0.0;
@@ -1025,7 +1037,7 @@ __global__ void __launch_bounds__(192) k_strip_residual(gm_grid g, const double*
     S::sync();
 #pragma unroll
     for (int ox = 0; ox < 3; ++ox)
-      for (int k = max(ks[ox], k0) - k0; k < min(ke[ox] - k0, C); ++k) {
+      for (int k = S::first(ks[ox], k0, split, SPLIT); k < min(ke[ox] - k0, C); k += SPLIT) {
         const uint8_t ex = p.ext[k];
         if ((ox == 2 && !(ex & 1)) || (oy == 2 && !(ex & 2))) continue;  // outside the particle's support
         const double *tx = p.t + k * S::TS, *ty = tx + NT, *yp = p.r + k * S::RS;
@@ -1035,9 +1047,12 @@ __global__ void __launch_bounds__(192) k_strip_residual(gm_grid g, const double*
           if (c == 2) acc += (w - tx[6 + ox] * ty[6 + oy]) * yp[L::Y_S];
       }
   }
-  if (row < ROWS) OUT[oy][lane] = acc;
+  double sum = acc;
+#pragma unroll
+  for (int k = 1; k < SPLIT; ++k) sum += __shfl(acc, (lane + k * PART) & 63, 64);
+  if (split == 0) OUT[oy][lane] = sum;
   __syncthreads();
-  if (oy == 0 && row < ROWS && I < g.n_nodes) {
+  if (oy == 0 && split == 0 && I < g.n_nodes) {
     const long d = (long)I * NB + c;
     rhs[d] = freem[d] ? OUT[0][lane] + OUT[1][lane] + OUT[2][lane] : 0.0;
   }
@@ -1047,7 +1062,9 @@ __global__ void __launch_bounds__(192) k_strip_residual(gm_grid g, const double*
 // of D, and the 15 sums a line fit in registers.  Bound by the LDS reads of the 36 candidates
 // (18 values a candidate and lane) and by the 15 wavefronts a CU that the pieces' LDS leaves:
 // pieces of 24, 40 and 56 FP64 rows took 407, 407 and 497 us against 378 with 32; 40 FP32 rows
-// 298 us.  One wavefront per row, lanes over its 25 blocks and one particle after the other,
+// 298 us.  8 rows with two lanes for a bin's particles and a line's whole range in one piece: 439
+// and 276 us (an eighth more particles staged, and twice the workgroups' start and output).  One
+// wavefront per row, lanes over its 25 blocks and one particle after the other,
 // took 2750 us FP64 and 2709 us FP32 (1,048,576 particles, 264,000 rows; 210 MB of matrix and
 // 201 MB of D); u-p with 11,628 rows 135 -> 69 us.
 template <bool COUPLED, typename TD, typename TV>
@@ -1194,9 +1211,9 @@ extern "C" int gm_node_residual(const gm_grid* g, const gm_bins* b, const double
   int n = g->n_nodes;
   int blk = gm_blocks(n, 128);
   if (g->dim == 2 && !coupled)
-    k_strip_residual<false><<<gm_blocks(n, 32), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
+    k_strip_residual<false><<<gm_blocks(n, RES_ROWS), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else if (g->dim == 2)
-    k_strip_residual<true><<<gm_blocks(n, 21), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
+    k_strip_residual<true><<<gm_blocks(n, RES_ROWS_UP), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else if (coupled)
     k_node_residual<3, true><<<blk, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else {

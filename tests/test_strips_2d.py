@@ -18,8 +18,8 @@ def _tables(x, lp, h):
         out(wa[0], wa[1]), on
 
 
-# grids and particle counts: fewer node rows than one strip, a strip's last row, remainders of
-# 7, 16, 21 and 32 rows, grid lines shorter and longer than a strip, no particles in most bins,
+# grids and particle counts: fewer node rows than one strip, a strip's last row, remainders of 5, 8,
+# 7 and 16 rows, grid lines shorter and longer than a strip, no particles in most bins,
 # and ranges of one and of several staged pieces (up to 60 particles in one bin)
 @pytest.mark.gpu
 @pytest.mark.parametrize('coupled', [False, True])
