@@ -182,7 +182,7 @@ class Multigrid:
             # exact coarsest solve: the inverse formed on the device, or, when its probe is off (a
             # singular operator, or one that needs pivoting across the whole matrix), on the host.
             # The host's LU alone took 4.5 ms for 602 dofs and 38 ms for 1890, to which its
-            # scatter and copies came; the device's takes 0.42 and 1.56 ms.
+            # scatter and copies came; the device's takes 0.37 and 1.48 ms.
             k = self._keep[-1]
             lv = self.levels[self.n_levels - 1]
             nb, n = self.nb, lv.n_nodes
