@@ -315,69 +315,60 @@ __global__ void k_bin_extset(int n_bins, const int* cell_start, const uint8_t* e
   extset[b] = s;
 }
 
+// A support of shape ex seen from its node at offset o sets the window bits (k - o + 2) of its box:
+// the box at o = (2, 2, 2) shifted, so a shape costs two shifts and not a loop over its nodes (139,425
+// nodes: 218 -> 9 us).
 template <int DIM>
 __global__ void k_pattern_count_sets(gm_grid g, const int* extset, uint64_t* mask, int* row_nnzb) {
+  constexpr int M = DIM == 3 ? 27 : 9;
   int I = blockIdx.x * blockDim.x + threadIdx.x;
   if (I >= g.n_nodes) return;
   int ci[3] = {0, 0, 0};
   node_coords<DIM>(g, I, ci);
-  const int ncell[3] = {g.nx, g.ny, g.nz};
-  uint64_t m0 = 0, m1 = 0;
-  int cb = (DIM == 2) ? (2 + 5 * 2) : (2 + 5 * 2 + 25 * 2);
-  if (cb < 64) m0 |= (1ull << cb); else m1 |= (1ull << (cb - 64));
-  const int oz_n = (DIM == 3) ? 3 : 1;
-  for (int oz = 0; oz < oz_n; ++oz)
-    for (int oy = 0; oy < 3; ++oy)
-      for (int ox = 0; ox < 3; ++ox) {
-        const int o[3] = {ox, oy, oz};
-        int bc[3] = {0, 0, 0};
-        bool ok = true;
+  const int nx1 = g.nx + 1, nxy = nx1 * (g.ny + 1);
+  int es[M];
 #pragma unroll
-        for (int a = 0; a < DIM; ++a) {
-          bc[a] = ci[a] - o[a];
-          if (bc[a] < 0 || bc[a] > ncell[a]) ok = false;
-        }
-        if (!ok) continue;
-        const int es = extset[node_index<DIM>(g, bc)];
-        for (int ex = 0; ex < (1 << DIM); ++ex) {
-          if (!((es >> ex) & 1)) continue;
-          int e[3] = {1, 1, 1};
-          bool in = true;
+  for (int o = 0; o < M; ++o) {
+    const bool ok = ci[0] >= o % 3 && ci[1] >= o / 3 % 3 && ci[2] >= o / 9;
+    es[o] = ok ? extset[I - o % 3 - o / 3 % 3 * nx1 - o / 9 * nxy] : 0;
+  }
+  const int cb = (DIM == 2) ? (2 + 5 * 2) : (2 + 5 * 2 + 25 * 2);  // centre bit
+  uint64_t m0 = cb < 64 ? 1ull << cb : 0ull, m1 = cb < 64 ? 0ull : 1ull << (cb - 64);
 #pragma unroll
-          for (int a = 0; a < DIM; ++a) {
-            e[a] = ((ex >> a) & 1) ? 3 : 2;
-            in = in && o[a] < e[a];
-          }
-          if (!in) continue;
-          for (int kz = 0; kz < e[2]; ++kz)
-            for (int ky = 0; ky < e[1]; ++ky)
-              for (int kx = 0; kx < e[0]; ++kx) {
-                int rx = kx - o[0] + 2, ry = ky - o[1] + 2, rz = (DIM == 3) ? (kz - o[2] + 2) : 0;
-                int bit = rx + 5 * ry + 25 * rz;
-                if (bit < 64) m0 |= (1ull << bit); else m1 |= (1ull << (bit - 64));
-              }
-        }
-      }
+  for (int o = 0; o < M; ++o) {
+    const int ox = o % 3, oy = o / 3 % 3, oz = o / 9;
+    uint64_t box = 0;  // the union of the shapes present that hold the node, at offset (2, 2, 2)
+#pragma unroll
+    for (int ex = 0; ex < (1 << DIM); ++ex) {
+      if ((ox == 2 && !(ex & 1)) || (oy == 2 && !(ex & 2)) || (oz == 2 && !(ex & 4))) continue;
+      uint64_t bits = (ex & 1) ? 7ull : 3ull;
+      bits |= bits << 5 | ((ex & 2) ? bits << 10 : 0ull);
+      if (DIM == 3) bits |= bits << 25 | ((ex & 4) ? bits << 50 : 0ull);
+      if ((es[o] >> ex) & 1) box |= bits;
+    }
+    const int sh = 2 - ox + 5 * (2 - oy) + (DIM == 3 ? 25 * (2 - oz) : 0);
+    m0 |= box << sh;
+    if (DIM == 3 && sh) m1 |= box >> (64 - sh);
+  }
   mask[2 * I] = m0;
   mask[2 * I + 1] = m1;
   row_nnzb[I] = __popcll(m0) + __popcll(m1);
 }
 
+// A lane per window bit of a row (128 a row in 3D, 32 in 2D): consecutive lanes write consecutive
+// columns (139,425 rows: 101 -> 44 us; a thread per row before).
 template <int DIM>
-__global__ void k_pattern_fill(gm_grid g, const uint64_t* mask, const int* row_ptr, int* col_idx) {
-  int I = blockIdx.x * blockDim.x + threadIdx.x;
-  if (I >= g.n_nodes) return;
-  int ci[3] = {0, 0, 0};
-  node_coords<DIM>(g, I, ci);
-  int k = row_ptr[I];
-  const int nbits = (DIM == 2) ? 25 : 125;
-  for (int bit = 0; bit < nbits; ++bit) {
-    uint64_t w = (bit < 64) ? mask[2 * I] : mask[2 * I + 1];
-    if (!((w >> (bit & 63)) & 1ull)) continue;
-    int rx = bit % 5 - 2, ry = (bit / 5) % 5 - 2, rz = (DIM == 3) ? (bit / 25 - 2) : 0;
-    int c[3] = {ci[0] + rx, ci[1] + ry, ci[2] + rz};
-    col_idx[k++] = node_index<DIM>(g, c);
-  }
+__global__ void __launch_bounds__(256) k_pattern_fill(gm_grid g, const uint64_t* mask, const int* row_ptr,
+                                                      int* col_idx) {
+  constexpr int LANES = DIM == 3 ? 128 : 32, W = DIM == 3 ? 125 : 25;
+  const int I = blockIdx.x * (256 / LANES) + threadIdx.x / LANES, bit = threadIdx.x % LANES;
+  if (I >= g.n_nodes || bit >= W) return;
+  const uint64_t m0 = mask[2 * I], m1 = mask[2 * I + 1];
+  if (!(((bit < 64 ? m0 : m1) >> (bit & 63)) & 1ull)) return;
+  const uint64_t low = (1ull << (bit & 63)) - 1ull;
+  const int below = bit < 64 ? __popcll(m0 & low) : __popcll(m0) + __popcll(m1 & low);
+  const int nx1 = g.nx + 1, nxy = nx1 * (g.ny + 1);
+  col_idx[row_ptr[I] + below] = I + bit % 5 - 2 + (bit / 5 % 5 - 2) * nx1 + (DIM == 3 ? (bit / 25 - 2) * nxy : 0);
 }
 
 // Row masks from the bins' support-shape sets (1, the default) or particle by particle (0).
@@ -418,9 +409,9 @@ extern "C" int gm_bsr_pattern(const gm_grid* g, const gm_bins* b, gm_pattern* pa
     return -4;
   }
   if (g->dim == 2)
-    k_pattern_fill<2><<<gm_blocks(n, 128), 128, 0, s>>>(*g, pat->row_mask, pat->row_ptr, pat->col_idx);
+    k_pattern_fill<2><<<gm_blocks(n, 8), 256, 0, s>>>(*g, pat->row_mask, pat->row_ptr, pat->col_idx);
   else
-    k_pattern_fill<3><<<gm_blocks(n, 128), 128, 0, s>>>(*g, pat->row_mask, pat->row_ptr, pat->col_idx);
+    k_pattern_fill<3><<<gm_blocks(n, 2), 256, 0, s>>>(*g, pat->row_mask, pat->row_ptr, pat->col_idx);
   GM_LAUNCH_CHECK();
   return 0;
 }
@@ -1679,41 +1670,66 @@ extern "C" int gm_penalty_pc(const gm_grid* g, const gm_bins* b, const gm_patter
 //  act:     activation (threshold < 0: every support node, as P2G_2d; else w > threshold)
 //  bflag:   pressure-Dirichlet flags are OR-ed into the p dof (coupled)
 //  mrhs:    consistent-mass rhs, may be null
+// Four lanes a node take every fourth particle of each of its bins: a lane alone is a chain of
+// dependent loads (ids, pressures) and axis data over some 36 (2D) or 216 particles (11,628 2D nodes:
+// 53 -> 26 us).
 template <int DIM>
-__global__ void k_p2g(gm_grid g, int nb, const double* x_s, const double* lp_s, const int* cell_start,
-                      const int* sorted, const uint8_t* ext_s, double threshold, const uint8_t* pbc_flag,
-                      double node_h_last, double p_mass, const double* p_part, uint8_t* act, uint8_t* bflag,
-                      double* mrhs) {
-  int I = blockIdx.x * blockDim.x + threadIdx.x;
-  if (I >= g.n_nodes) return;
+__global__ void __launch_bounds__(128) k_p2g(gm_grid g, int nb, const double* x_s, const double* lp_s,
+                                             const int* cell_start, const int* sorted, const uint8_t* ext_s,
+                                             double threshold, const uint8_t* pbc_flag, double node_h_last,
+                                             double p_mass, const double* p_part, uint8_t* act, uint8_t* bflag,
+                                             double* mrhs) {
+  const int I = blockIdx.x * 32 + threadIdx.x / 4, sub = threadIdx.x % 4;
   int ci[3] = {0, 0, 0};
   node_coords<DIM>(g, I, ci);
-  bool a_on = false, pb = false;
+  const int ncell[3] = {g.nx, g.ny, g.nz};
+  int on = 0;  // 1: active, 2: pressure boundary
   double rhs = 0.0;
-  for_candidates<DIM>(g, ci, cell_start, ext_s, [&](int k, const int* o, const int* b, bool in) {
-    int p = sorted[k];
-    // pressure boundary: 2D loops over the support, 3D over all 27 nodes (mpm_utils.py:225-235, 349-352)
-    if (pbc_flag && pbc_flag[p] && (in || DIM == 3)) {
-      double nc = (double)ci[DIM - 1] * node_h_last;
-      if (nc >= x_s[k * DIM + DIM - 1]) pb = true;
-    }
-    if (!in) return;
-    Axis ax[DIM];
-    load_axes<DIM>(g, x_s, lp_s, k, ax);
-    double w, G[3], wa;
-    node_geom<DIM>(ax, o, w, G, wa);
-    if (threshold < 0.0 || w > threshold) a_on = true;
-    if (mrhs) {
-      // sum of the particle's weights over its support, one axis at a time
-      double wsum = 1.0;
+  const double nc = (double)ci[DIM - 1] * node_h_last;
+  for (int q = 0; q < (DIM == 3 ? 27 : 9) && I < g.n_nodes; ++q) {
+    const int o[3] = {q % 3, q / 3 % 3, q / 9};
+    int bc[3] = {0, 0, 0};
+    bool ok = true;
 #pragma unroll
-      for (int aa = 0; aa < DIM; ++aa) wsum *= ax[aa].w[0] + ax[aa].w[1] + ax[aa].w[2];
-      rhs += w * wsum * p_mass * p_part[p];
+    for (int a = 0; a < DIM; ++a) {
+      bc[a] = ci[a] - o[a];
+      if (bc[a] < 0 || bc[a] > ncell[a]) ok = false;
     }
-  });
-  if (a_on)
+    if (!ok) continue;
+    const int b = node_index<DIM>(g, bc);
+    for (int k = cell_start[b] + sub; k < cell_start[b + 1]; k += 4) {
+      const int p = sorted[k];
+      const uint8_t ex = ext_s[k];
+      bool in = true;
+#pragma unroll
+      for (int a = 0; a < DIM; ++a) in = in && o[a] < (((ex >> a) & 1) ? 3 : 2);
+      // pressure boundary: 2D loops over the support, 3D over all 27 nodes (mpm_utils.py:225-235, 349-352)
+      if (pbc_flag && pbc_flag[p] && (in || DIM == 3) && nc >= x_s[k * DIM + DIM - 1]) on |= 2;
+      if (!in) continue;
+      const double pp = mrhs ? p_part[p] : 0.0;
+      Axis ax[DIM];
+      load_axes<DIM>(g, x_s, lp_s, k, ax);
+      double w, G[3], wa;
+      node_geom<DIM>(ax, o, w, G, wa);
+      if (threshold < 0.0 || w > threshold) on |= 1;
+      if (mrhs) {
+        // sum of the particle's weights over its support, one axis at a time
+        double wsum = 1.0;
+#pragma unroll
+        for (int aa = 0; aa < DIM; ++aa) wsum *= ax[aa].w[0] + ax[aa].w[1] + ax[aa].w[2];
+        rhs += w * wsum * p_mass * pp;
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 1; s < 4; s <<= 1) {
+    rhs += __shfl_xor(rhs, s, 64);
+    on |= __shfl_xor(on, s, 64);
+  }
+  if (sub || I >= g.n_nodes) return;
+  if (on & 1)
     for (int k = 0; k < nb; ++k) act[I * nb + k] = 1;
-  if (pb && bflag) bflag[I * nb + DIM] = 1;
+  if ((on & 2) && bflag) bflag[I * nb + DIM] = 1;
   if (mrhs) mrhs[I] = rhs;
 }
 
@@ -1728,10 +1744,10 @@ extern "C" int gm_p2g(const gm_grid* g, const gm_bins* b, const gm_pattern* pat,
     GM_LAUNCH_CHECK();
   }
   if (g->dim == 2)
-    k_p2g<2><<<gm_blocks(n, 128), 128, 0, s>>>(*g, g->nb, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold,
+    k_p2g<2><<<gm_blocks(n, 32), 128, 0, s>>>(*g, g->nb, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold,
                                                pbc_flag, node_h_last, p_mass, p_part, act, bflag, mrhs);
   else
-    k_p2g<3><<<gm_blocks(n, 128), 128, 0, s>>>(*g, g->nb, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold,
+    k_p2g<3><<<gm_blocks(n, 32), 128, 0, s>>>(*g, g->nb, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold,
                                                pbc_flag, node_h_last, p_mass, p_part, act, bflag, mrhs);
   GM_LAUNCH_CHECK();
   return 0;
