@@ -27,10 +27,23 @@
 #define GS_BLOCKS 1024  // workgroups (and partial norms) of the Gram-Schmidt update
 
 // ------------------------------------------------------------------ SpMV
+// A 3D grid's window pattern: rows whose mask is full hold the 125 nodes around theirs in order, so
+// their columns follow from the row (mask null: every row's columns are read): 4 bytes a block less,
+// and no load of x waits for one.  Solve of the 64 x 64 x 32-cell indentation (FP32 operator, FP16
+// smoother) 7.00 -> 6.83 ms; two blocks a lane in flight, four and eight take 1 and 2 % more.
+struct Window {
+  const uint64_t* mask;
+  int nx1, nxy;
+  __device__ __forceinline__ bool full(int row) const {
+    return mask && mask[2 * row] == ~0ull && mask[2 * row + 1] == (1ull << 61) - 1;
+  }
+  __device__ __forceinline__ int offset(int k) const { return k % 5 - 2 + (k / 5 % 5 - 2) * nx1 + (k / 25 - 2) * nxy; }
+};
+
 template <int NB, int G, typename TM, typename TX, typename TY, int T = SPMV_T>
 __global__ void __launch_bounds__(T) k_spmv(int n_rows, const int* row_ptr, const int* col_idx, const TM* vals,
                                             const TX* x, TY* y, const TY* w1, const TY* w2, double* part,
-                                            const double* gate) {
+                                            const double* gate, Window win) {
   if (gate && *gate != 0.0) return;  // a gated launch after its solve has converged
   const int rows_per_blk = T / G;
   int lr = threadIdx.x / G;
@@ -62,8 +75,9 @@ __global__ void __launch_bounds__(T) k_spmv(int n_rows, const int* row_ptr, cons
     for (; k < e; k += G) acc[0] += (double)vals[k] * (double)x[col_idx[k]];
   } else if (row < n_rows) {
     int s = row_ptr[row], e = row_ptr[row + 1];
+    const bool full = win.full(row);
     for (int k = s + lane; k < e; k += G) {
-      int c = col_idx[k];
+      int c = full ? row + win.offset(k - s) : col_idx[k];
       const TM* blk = vals + (long)k * NB * NB;
       double xv[NB];
 #pragma unroll
@@ -122,25 +136,25 @@ static constexpr int spmv_lanes(int nb) { return nb >= 4 ? 16 : (nb == 3 ? 8 : (
 template <int NB, typename TM, typename TX, typename TY>
 static void launch_spmv(int n_rows, const int* rp, const int* ci, const TM* v, const TX* x, TY* y, const TY* w1,
                         const TY* w2, double* part, hipStream_t s, int threads = 0,
-                        const double* gate = nullptr) {
+                        const double* gate = nullptr, const Window& win = Window{nullptr, 0, 0}) {
   const int G = spmv_lanes(NB);
   int t = part ? SPMV_T : (threads ? threads : g_spmv_threads[NB][sizeof(TM) == 4 ? 1 : 0]);
   switch (t) {
     case 64:
       k_spmv<NB, G, TM, TX, TY, 64><<<gm_blocks(n_rows, 64 / G), 64, 0, s>>>(n_rows, rp, ci, v, x, y, w1, w2, part,
-                                                                               gate);
+                                                                               gate, win);
       break;
     case 128:
       k_spmv<NB, G, TM, TX, TY, 128><<<gm_blocks(n_rows, 128 / G), 128, 0, s>>>(n_rows, rp, ci, v, x, y, w1, w2,
-                                                                                 part, gate);
+                                                                                 part, gate, win);
       break;
     case 512:
       k_spmv<NB, G, TM, TX, TY, 512><<<gm_blocks(n_rows, 512 / G), 512, 0, s>>>(n_rows, rp, ci, v, x, y, w1, w2,
-                                                                                 part, gate);
+                                                                                 part, gate, win);
       break;
     default:
       k_spmv<NB, G, TM, TX, TY, 256><<<gm_blocks(n_rows, 256 / G), 256, 0, s>>>(n_rows, rp, ci, v, x, y, w1, w2,
-                                                                                 part, gate);
+                                                                                 part, gate, win);
   }
 }
 
@@ -246,13 +260,14 @@ __global__ void __launch_bounds__(T) k_lo_convert_cached(int n_rows, const int* 
 // ends with the row's full product (butterfly reduction in a fixed order).
 template <int NB, int G, typename TM, typename TX>
 __device__ __forceinline__ void row_acc(int row, int lane, int n_rows, const int* row_ptr, const int* col_idx,
-                                        const TM* vals, const TX* x, double acc[NB]) {
+                                        const Window& win, const TM* vals, const TX* x, double acc[NB]) {
 #pragma unroll
   for (int r = 0; r < NB; ++r) acc[r] = 0.0;
   if (row < n_rows) {
     int s = row_ptr[row], e = row_ptr[row + 1];
+    const bool full = win.full(row);
     for (int k = s + lane; k < e; k += G) {
-      int c = col_idx[k];
+      int c = full ? row + win.offset(k - s) : col_idx[k];
       const TM* blk = vals + (long)k * NB * NB;
       double xv[NB];
 #pragma unroll
@@ -272,11 +287,36 @@ __device__ __forceinline__ void row_acc(int row, int lane, int n_rows, const int
 // The same from the FP16 copy: FP32 partial sums per (r, c), scaled after the reduction.
 template <int NB, int G>
 __device__ __forceinline__ void row_acc_lo(int row, int lane, int n_rows, const int* row_ptr, const int* col_idx,
-                                           const gm_half* lo, const float* scale, const float* x, double acc[NB]) {
+                                           const Window& win, const gm_half* lo, const float* scale, const float* x,
+                                           double acc[NB]) {
   float a[NB * NB];
 #pragma unroll
   for (int q = 0; q < NB * NB; ++q) a[q] = 0.0f;
-  if (row < n_rows) {
+  if (row < n_rows && win.full(row)) {
+    constexpr int U = 2, N = (125 + G - 1) / G;
+    const gm_half* base = lo + (long)row_ptr[row] * NB * NB;
+#pragma unroll
+    for (int u0 = 0; u0 < N; u0 += U) {
+      gm_half h[U][NB * NB];
+      float xv[U][NB];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = min(lane + (u0 + u) * G, 124);
+        const long c = row + win.offset(k);
+#pragma unroll
+        for (int q = 0; q < NB * NB; ++q) h[u][q] = base[(long)k * NB * NB + q];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) xv[u][j] = x[c * NB + j];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (lane + (u0 + u) * G < 125)
+#pragma unroll
+          for (int r = 0; r < NB; ++r)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) a[r * NB + j] += (float)h[u][r * NB + j] * xv[u][j];
+    }
+  } else if (row < n_rows) {
     int s = row_ptr[row], e = row_ptr[row + 1];
     int k = s + lane;
     // two blocks per step: both blocks' loads are issued before either is accumulated (the
@@ -337,16 +377,16 @@ __device__ __forceinline__ void row_acc_lo(int row, int lane, int n_rows, const 
 //   MODE 2 (Jacobi sweep):  out = x + omega Dinv (b - A x)      (out != x)
 // A is the level's matrix (TM) or, with LO, its FP16 copy (FP32 hierarchies).
 template <int NB, int G, int MODE, typename TM, typename T, bool LO>
-__global__ void __launch_bounds__(256) k_level(int n_rows, const int* row_ptr, const int* col_idx, const TM* vals,
-                                               const gm_half* lo, const float* scale, const T* x, const T* b,
+__global__ void __launch_bounds__(256) k_level(int n_rows, const int* row_ptr, const int* col_idx, Window win,
+                                               const TM* vals, const gm_half* lo, const float* scale, const T* x, const T* b,
                                                const T* dinv, double omega, T* out) {
   int row = blockIdx.x * (256 / G) + threadIdx.x / G;
   int lane = threadIdx.x % G;
   double acc[NB];
   if constexpr (LO)
-    row_acc_lo<NB, G>(row, lane, n_rows, row_ptr, col_idx, lo, scale, (const float*)x, acc);
+    row_acc_lo<NB, G>(row, lane, n_rows, row_ptr, col_idx, win, lo, scale, (const float*)x, acc);
   else
-    row_acc<NB, G, TM, T>(row, lane, n_rows, row_ptr, col_idx, vals, x, acc);
+    row_acc<NB, G, TM, T>(row, lane, n_rows, row_ptr, col_idx, win, vals, x, acc);
   if (row >= n_rows || lane != 0) return;
   double res[NB];
 #pragma unroll
@@ -1640,7 +1680,8 @@ struct JacobiPrec {
 template <int NB, typename TM, typename TV, typename Prec>
 static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, const TV* b, TV* x, TV* V, TV* z,
                       TV* w, const Prec& prec, double* part, double* dh, int m, double tol, int maxiter,
-                      int* iters_out, double* relres_out, hipStream_t st, TV* Zs = nullptr) {
+                      int* iters_out, double* relres_out, hipStream_t st, TV* Zs = nullptr,
+                      const Window& win = Window{nullptr, 0, 0}) {
   long n = (long)n_rows * NB;
   long ldv = n;
   int vb = dot_blocks(n);
@@ -1762,7 +1803,7 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
         TV* zj = Zs ? Zs + (long)j * ldv : z;
         int prc = prec.apply(vj, zj, q);
         if (prc) return prc;
-        launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, zj, w, nullptr, nullptr, nullptr, q);
+        launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, zj, w, nullptr, nullptr, nullptr, q, 0, nullptr, win);
         const int nchunk = chunks(j + 2), fc = fold ? nchunk : 0;
         double *h2 = dh + (m + 2), *sc = dh + nsl;
         k_gs_dots<TV><<<dim3(nchunk, j + 2), RED_T, 0, q>>>(n, j + 1, V, ldv, w, nchunk, part, nullptr, 0, sc);
@@ -2189,6 +2230,10 @@ inline Dims dims_of(const gm_mg_level& l) {
   return d;
 }
 
+inline Window window_of(const gm_mg_level& lv) {
+  return Window{lv.nz > 0 ? lv.row_mask : nullptr, lv.nx + 1, (lv.nx + 1) * (lv.ny + 1)};
+}
+
 struct Cycle {
   int dim, n_levels, nu_pre, nu_post, coarse_sweeps;
   double omega;
@@ -2233,19 +2278,20 @@ static void level_op(const gm_mg_level& lv, int l, const T* x, const T* b, const
                      hipStream_t st) {
   constexpr int G = spmv_lanes(NB);
   int blocks = gm_blocks(lv.n_nodes, 256 / G);
+  const Window win = window_of(lv);
   if constexpr (std::is_same<T, float>::value) {
     if (lv.vals_lo) {
       k_level<NB, G, MODE, float, float, true><<<blocks, 256, 0, st>>>(
-          lv.n_nodes, lv.row_ptr, lv.col_idx, nullptr, (const gm_half*)lv.vals_lo, lv.row_scale, x, b, dinv, omega,
+          lv.n_nodes, lv.row_ptr, lv.col_idx, win, nullptr, (const gm_half*)lv.vals_lo, lv.row_scale, x, b, dinv, omega,
           out);
       return;
     }
   }
   if (l == 0)
-    k_level<NB, G, MODE, T, T, false><<<blocks, 256, 0, st>>>(lv.n_nodes, lv.row_ptr, lv.col_idx, (const T*)lv.vals,
+    k_level<NB, G, MODE, T, T, false><<<blocks, 256, 0, st>>>(lv.n_nodes, lv.row_ptr, lv.col_idx, win, (const T*)lv.vals,
                                                                nullptr, nullptr, x, b, dinv, omega, out);
   else
-    k_level<NB, G, MODE, double, T, false><<<blocks, 256, 0, st>>>(lv.n_nodes, lv.row_ptr, lv.col_idx,
+    k_level<NB, G, MODE, double, T, false><<<blocks, 256, 0, st>>>(lv.n_nodes, lv.row_ptr, lv.col_idx, win,
                                                                     (const double*)lv.vals, nullptr, nullptr, x, b,
                                                                     dinv, omega, out);
 }
@@ -2492,18 +2538,19 @@ extern "C" int gm_gmres_mg(int dim, int nb, int fp32, int n_levels, const gm_mg_
   // the Krylov operator: op_vals (same pattern as level 0) when the hierarchy is built from
   // a modified copy of the system matrix, else level 0's own matrix
   const void* opv = op_vals ? op_vals : l0.vals;
+  const Window win = mg::window_of(l0);
 #define GM_GMG(D, B)                                                                                            \
   do {                                                                                                          \
     if (fp32) {                                                                                                 \
       mg::MGPrec<D, B, float> pc{cy, n};                                                                        \
       return gmres_impl<B, float, float>(l0.n_nodes, l0.row_ptr, l0.col_idx, (const float*)opv,                 \
                                          (const float*)b, (float*)x, (float*)V, (float*)z, (float*)w, pc, part, \
-                                         dh, m, tol, maxiter, iters, relres, s, (float*)Z);                     \
+                                         dh, m, tol, maxiter, iters, relres, s, (float*)Z, win);                \
     }                                                                                                           \
     mg::MGPrec<D, B, double> pc{cy, n};                                                                         \
     return gmres_impl<B, double, double>(l0.n_nodes, l0.row_ptr, l0.col_idx, (const double*)opv,                \
                                          (const double*)b, (double*)x, (double*)V, (double*)z, (double*)w, pc,  \
-                                         part, dh, m, tol, maxiter, iters, relres, s, (double*)Z);              \
+                                         part, dh, m, tol, maxiter, iters, relres, s, (double*)Z, win);         \
   } while (0)
   GM_MG_DISPATCH(GM_GMG);
 #undef GM_GMG
