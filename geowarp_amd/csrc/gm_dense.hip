@@ -222,7 +222,7 @@ extern "C" size_t gm_dense_inverse_work_bytes(int n) {
 extern "C" int gm_dense_inverse(int nb, int n_nodes, const int* row_ptr, const int* col_idx, const double* vals,
                                 double* inv, void* work, size_t work_bytes, double* err, hipStream_t s) {
   GM_REQUIRE(row_ptr && col_idx && vals && inv && work && err, "gm_dense_inverse: null argument");
-  GM_REQUIRE(nb >= 1 && n_nodes >= 1 && (long)nb * n_nodes <= 16384, "gm_dense_inverse: bad size");
+  GM_REQUIRE(nb >= 1 && n_nodes >= 1 && (long)nb * n_nodes <= 65536, "gm_dense_inverse: bad size");
   const int n = nb * n_nodes, nt = (n + DB - 1) / DB;
   GM_REQUIRE(work_bytes >= gm_dense_inverse_work_bytes(n), "gm_dense_inverse: workspace too small");
   double* other = (double*)work;

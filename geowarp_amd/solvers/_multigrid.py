@@ -37,6 +37,8 @@ def window_pattern(dim, cells):
 
 # largest relative error of the device inverse's probe (gm_dense_inverse) that is taken
 DENSE_TOL = 1e-8
+# dofs that gm_dense_inverse takes
+DENSE_MAX = 65536
 
 
 def _robust_inverse(A):
@@ -186,11 +188,12 @@ class Multigrid:
             k = self._keep[-1]
             lv = self.levels[self.n_levels - 1]
             nb, n = self.nb, lv.n_nodes
-            L.check(L.lib().gm_dense_inverse(nb, n, L.ptr(k['rp']), L.ptr(k['ci']), L.ptr(k['vals']),
-                                             L.ptr(self.cinv), L.ptr(self.cwork), self.cwork.numel(),
-                                             L.ptr(self.cerr), stream), 'gm_dense_inverse')
-            if self.cerr.item() <= DENSE_TOL:
-                return
+            if n * nb <= DENSE_MAX:
+                L.check(L.lib().gm_dense_inverse(nb, n, L.ptr(k['rp']), L.ptr(k['ci']), L.ptr(k['vals']),
+                                                 L.ptr(self.cinv), L.ptr(self.cwork), self.cwork.numel(),
+                                                 L.ptr(self.cerr), stream), 'gm_dense_inverse')
+                if self.cerr.item() <= DENSE_TOL:
+                    return
             rp = k['rp'].cpu().numpy().astype(np.int64)
             ci = k['ci'].cpu().numpy().astype(np.int64)
             v = k['vals'].double().cpu().numpy().reshape(-1, nb, nb)

@@ -361,7 +361,7 @@ int gm_bsr_transpose(int nb, int fp32, int n_rows, const int* row_ptr, const int
    n_nodes * 4^dim * nb * nb doubles. */
 int gm_mg_setup(int dim, int nb, int fp32, int n_levels, gm_mg_level* levels, void* ap_work, hipStream_t stream);
 
-/* Dense inverse (n x n FP64, row-major, n = nb * n_nodes <= 16384) of a block-CSR operator, the
+/* Dense inverse (n x n FP64, row-major, n = nb * n_nodes <= 65536) of a block-CSR operator, the
    hierarchy's coarsest, by Gauss-Jordan in blocks of 32 with pivoting inside the blocks.  *err
    (device) is set to max_i |A inv v - v|_i / |v_i| of a probe v_i = +-(the power of two next to sqrt|a_ii|), NaN or infinite
    when a pivot block is singular: the caller decides whether it will do (no counterpart in the
