@@ -944,9 +944,8 @@ int cu_count() {
 // the workgroups do not come out even over the CUs: the number of segments with the least
 // (rounds + 1/2) x (bins of a segment + 2), at least one round.  The half round is what the
 // lines without particles (which end at once) and the XCDs' shares make of the last one: whole
-// rounds instead pick 1, 3 and 3 segments for 21 x 17 x 13, 48 x 9 x 7 and 64 x 64 x 32 cells,
-// 249, 149 and 2268 us in FP32 where 2, 6 and 2 take 212, 117 and 2233.  (Some six particles a
-// bin are taken for granted.)
+// rounds instead pick 1 and 3 segments for 21 x 17 x 13 (FP64) and 48 x 9 x 7 cells (FP32), 249 and
+// 149 us where 2 and 6 take 212 and 117.  (Some six particles a bin are taken for granted.)
 int best_segments(int nbx, int lines, int n_p, int slots) {
   const double busy = std::max(1.0, std::min<double>(lines, n_p / (6.0 * nbx)));
   int best = 1;
