@@ -121,9 +121,12 @@ GM_DEV Axis gimp_axis(double x, double lp, double h, double inv_h) {
     double d0 = x - x0, d2 = x - x2;
     double a0 = h + lp - fabs(d0);
     double a2 = h + lp - fabs(d2);
-    // Every quotient has the denominator h lp or lp (times a power of two): one reciprocal of
-    // h lp serves them all, each quotient corrected by its own remainder (Markstein 1990), so
-    // that it is rounded as a division is.  Ten FP64 divisions took most of this function.
+    // Every quotient but the sign's has the denominator h lp or lp (times a power of two): one
+    // reciprocal of h lp serves them all, each quotient corrected by its own remainder (Markstein
+    // 1990), so that it is rounded as a division is.  Ten FP64 divisions took most of this
+    // function.  The sign d / |d| of an end node's gradient stays a product and a division: their
+    // two roundings are part of the value (every thirtieth F of the particle stage depends on
+    // them), and load steps are held to the last bit (see k_update_lp).
     const double hl = h * lp, r = 1.0 / hl, rl = r * h;
     auto div_hl = [&](double n) {
       const double q = n * r;
@@ -133,14 +136,12 @@ GM_DEV Axis gimp_axis(double x, double lp, double h, double inv_h) {
       const double q = n * rl;
       return fma(fma(-lp, q, n), rl, q);
     };
-    const double q0 = div_hl(a0), q2 = div_hl(a2);
-    const double s0 = d0 != 0.0 ? copysign(1.0, d0) : d0 / d0, s2 = d2 != 0.0 ? copysign(1.0, d2) : d2 / d2;
     a.w[0] = 0.25 * div_hl(a0 * a0);
-    a.g[0] = -0.5 * q0 * s0;
+    a.g[0] = -0.5 * div_hl(a0) * d0 / fabs(d0);
     a.w[1] = 1.0 - 0.5 * div_hl((x - x1) * (x - x1) + lp * lp);
     a.g[1] = -div_hl(x - x1);
     a.w[2] = 0.25 * div_hl(a2 * a2);
-    a.g[2] = -0.5 * q2 * s2;
+    a.g[2] = -0.5 * div_hl(a2) * d2 / fabs(d2);
     a.wa[0] = 0.25 * div_lp(a0);
     a.wa[1] = 0.5;
     a.wa[2] = 0.25 * div_lp(a2);

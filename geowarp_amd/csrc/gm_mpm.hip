@@ -1883,7 +1883,12 @@ extern "C" int gm_g2p(const gm_grid* g, int n, double* x, const double* lp, cons
   return 0;
 }
 
-// update_GIMP_lp_2d/3d (gimp.py:428-507)
+// update_GIMP_lp_2d/3d (gimp.py:428-507).  A domain that sticks out of the box is cut 1e-6 inside it,
+// a jump that a comparison decides.  In a wall cell x - min and lp0 |F col| are equal but for products
+// of shears, so far from the load the comparison hangs on the last digits of x and F, and a change of
+// rounding anywhere in the load step flips entries (64 x 64 x 32 cells, mixed form: the order of the
+// sums of any one kernel of the step, in one to five of 24 load paths).  Hence the kernels of the 3D
+// u-p step keep the order and the rounding of their sums.
 __global__ void k_update_lp(int n, int dim, const double* F_new, double* lp, double lp0, const double* x,
                             double mnx, double mxx, double mny, double mxy, double mnz, double mxz) {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
