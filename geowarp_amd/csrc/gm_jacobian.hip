@@ -9,23 +9,31 @@
 // stencil base node b) reach the same 3x3x3 nodes, so for every column dof c this
 // is a dense product (108 rows (I,r)) x (5 n_p) x (27 columns J): the matrix
 // cores take it 16x16x4 at a time, FP32 when the tangent is FP32 (mixed form),
-// FP64 otherwise.
-//   k_jac_line    a workgroup per segment of a bin line (fixed y, z): the products of its
-//                 bins one after another, summed over the line while they stay in the
+// FP64 otherwise.  Two forms, each a product kernel and a gather:
+//   k_jac_bin     a 256-lane workgroup per bin (or a persistent sweep over bins):
+//                 E_I for a group of particles in LDS, 14 output tiles of 16x16
+//                 over the 4 waves, the bin's 27 x 27 blocks written contiguously
+//                 to a workspace (n_nodes x 11664 values).
+//   k_jac_gather  one workgroup per block row I: every block (I, J) of the
+//                 pattern sums the <= 27 bins b = I - o holding both nodes in the
+//                 fixed order (oz, oy, ox); masks, sign and identity rows as in
+//                 the node-row kernels (k_jac_gather_staged: the same sums from
+//                 chunks staged in LDS).
+//   k_jac_line    (FP64) a workgroup per segment of a bin line (fixed y, z): the products of
+//                 its bins one after another, summed over the line while they stay in the
 //                 accumulators; every pair of nodes a line reaches is written once (405
-//                 blocks a bin where the bin itself has 729).
-//   k_jac_gather  one workgroup per block row I: every block (I, J) of the pattern sums
-//                 the <= 9 lines holding both nodes in the fixed order (oz, oy); masks,
-//                 sign and identity rows as in the node-row kernels.
-// Both steps are deterministic (fixed accumulation order).  The workspace holds n_nodes x
-// 6480 values, written once and read once per assembly.
-//   64 x 64 x 32 cells, 1,048,576 particles (MI355X), per assembly: FP32 2.23 + 1.05 ms
-//   (one workgroup per bin, 11664 values per node in the workspace: 2.84 + 1.56 ms), FP64
-//   4.0 + 1.83 ms (5.6 + 2.9).  k_jac_line: the products take 0.95 (FP32) and 1.3 ms (FP64),
-//   the stores of the line sums 0.7 and 1.95 (3.6 and 7.2 GB), and one follows the other in the
-//   product waves; the operand waves' FP64 arithmetic adds 0.4 and 0.2.  With the shape-function
-//   tables made by an operand wave rather than the last product wave FP32 took 2.60.
-//   k_jac_gather moves 4.7 GB (FP32) at 4.5 TB/s.
+//                 blocks a bin where the bin itself has 729; n_nodes x 6480 values).
+//   k_jac_line_gather  one workgroup per block row I: every block sums the <= 9 lines holding
+//                 both nodes in the fixed order (oz, oy).
+// Both forms are deterministic (fixed accumulation order), and bound by HBM on the workspace,
+// written and read once, and the matrix itself.
+//   FP32 takes bins at every size: a sum over a line would add up to three bin sums in FP32
+//   where the gather adds all of them in FP64, which moves the mixed form's Newton iterates
+//   (load steps are held to the last bit, see k_update_lp).  It would be faster on large grids:
+//   2.23 + 1.05 ms against 2.84 + 1.56 with 64 x 64 x 32 cells, 1,048,576 particles (MI355X).
+//   FP64 takes lines: 4.0 + 1.83 ms against 5.6 + 2.9 on that grid.  k_jac_line: the products take 1.3 ms, the stores of the line sums 1.95
+//   (7.2 GB), and one follows the other in the product waves; the operand waves' arithmetic
+//   adds 0.2.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -44,6 +52,11 @@ namespace {
 constexpr int NY = 17, NZ = 15;
 constexpr int Y_T = 9, Y_Q = 12, Y_M = 13, Y_S = 16;
 constexpr int Z_DU = 9, Z_P = 10, Z_PB = 11, Z_G = 12;
+constexpr long CB_BIN = 27L * 27L * 16L;  // values per bin: 27 x 27 blocks of 4 x 4
+// chunk of bin `bin`'s blocks (I_loc = o, J_loc = 0..26) in the workspace: bins one
+// after another, each its 27 chunks in I_loc order
+constexpr long CHUNK = 27L * 16L;
+__device__ __forceinline__ long chunk_at(int o, int bin) { return (long)bin * CB_BIN + o * CHUNK; }
 // Workspace of the line sums, per bin line (y, z) and node x of it (a grid node's share):
 // the pairs of a row node and a column node of the line whose smaller x is that node's, which
 // one step of k_jac_line completes together.  Parts: nine chunks A (row node (x, y + oy,
@@ -52,12 +65,11 @@ constexpr int Z_DU = 9, Z_P = 10, Z_PB = 11, Z_G = 12;
 // r.  A matrix-core lane ends with the four rows r of one (row node, column node, c), so
 // that a store instruction writes whole runs of neighbouring 16-byte vectors.
 constexpr long CHUNK_A = 4L * 27 * 4, CHUNK_B = 4L * 9 * 4;  // values
-constexpr int CHUNK = CHUNK_A + 2 * CHUNK_B;                 // a row node's values of a line
-constexpr long CB_NODE = 9L * CHUNK;                         // values per grid node
-__device__ __forceinline__ long chunk_a(int o9, int node) { return (long)node * CB_NODE + o9 * CHUNK_A; }
+constexpr long LINE_NODE = 9L * (CHUNK_A + 2 * CHUNK_B);     // values per grid node
+__device__ __forceinline__ long chunk_a(int o9, int node) { return (long)node * LINE_NODE + o9 * CHUNK_A; }
 // d = 1, 2: the distance of the row node
 __device__ __forceinline__ long chunk_b(int o9, int node, int d) {
-  return (long)node * CB_NODE + 9 * CHUNK_A + ((d - 1) * 9 + o9) * CHUNK_B;
+  return (long)node * LINE_NODE + 9 * CHUNK_A + ((d - 1) * 9 + o9) * CHUNK_B;
 }
 
 typedef float f4v __attribute__((ext_vector_type(4)));
@@ -102,14 +114,431 @@ __device__ __forceinline__ int zsel(int c, int beta) {
   return Z_G + beta - 1;
 }
 
-template <int V>
-struct Int {
-  static constexpr int value = V;
-};
+// shape-function component beta of stencil node J (x fastest) from the axis tables
+template <typename TC>
+__device__ __forceinline__ TC gcomp(const TC (*ax)[9], int J, int beta) {
+  const int jx = J % 3, jy = (J / 3) % 3, jz = J / 9;
+  if (beta == 4) return ax[0][6 + jx] * ax[1][6 + jy] * ax[2][6 + jz];
+  const TC wx = ax[0][jx], wy = ax[1][jy], wz = ax[2][jz];
+  if (beta == 0) return wx * wy * wz;
+  if (beta == 1) return ax[0][3 + jx] * wy * wz;
+  if (beta == 2) return wx * ax[1][3 + jy] * wz;
+  return wx * wy * ax[2][3 + jz];
+}
 
 constexpr int MAX_SEG = 61;  // bins of a line segment (with two before it and the end, one a lane)
 
 }  // namespace
+
+// Per-bin products.  Workspace cb[b] = 27 x 27 blocks (I_loc, J_loc), I_loc = o_x +
+// 3 o_y + 9 o_z with node = b + o.  A workgroup takes bins b = blockIdx.x, +gridDim.x,
+// ... (one bin when the grid has one workgroup per bin, a persistent sweep when it is
+// smaller) and each bin's particles PG at a time: the E table of a group in LDS, its
+// products accumulated in the matrix-core registers, the bin's 27 x 27 blocks stored
+// after its last group.  The global loads of the next group (of this bin or of the
+// next one) are issued before the products of the current group when PF is set, so
+// their latency hides behind the matrix cores (at the cost of the registers that hold
+// them), else at the top of the group.
+// K order: a K step of the MFMA is one shape-function component beta and four
+// particles (lane group l / 16 = particle): the five components of a quad of
+// particles, then the next quad, whatever PG is.  After the
+// K loop unrolls, every A and B operand address is a per-lane base plus an immediate,
+// and the (c, beta) products that vanish (u columns: no w term except the penalty
+// on u_z, no w_avg term) are not issued.  Every (PG, OCC, PF, grid) variant adds the
+// same products in the same order, so all of them write the same bits.
+template <typename TD, typename TC, int PG, int OCC, bool PF>
+__global__ void __launch_bounds__(256, OCC) k_jac_bin(gm_grid g, const double* x_s, const double* lp_s,
+                                                      const int* cell_start, int n_bins, const TD* D, TC* cb) {
+  static_assert(PG % 4 == 0, "particle groups are whole K steps");
+  constexpr int KST = 5 * PG / 4;  // K steps of 4 per group
+  constexpr int NI = 4 * NZ;       // (z, r) entries of a node row of E_p
+  // shape-function tables of a group, two buffers: with PF the next group's are
+  // computed (by wave 3, whose last row tile is empty) while the products run
+  __shared__ TC AXT_[2][PG][3][9];
+  // E_p[I][z][r] (r fastest), node rows 68 entries apart and particles 28 x 68 apart:
+  // the 32 (particle, I, r) entries half a wave reads at once fall in 32 distinct banks.
+  // Node row I = 27 is zero (the padding rows of the last row tile read it).
+  constexpr int EI = 68, EP = 28 * EI;
+  __shared__ TC E_[PG * EP];
+#define E(p, I, z, r) E_[(p) * EP + (I) * EI + (z) * 4 + (r)]
+  // B operand g_p[J][beta], J padded to 32 with zeros, particles 176 entries apart
+  constexpr int BB = 32, BP = 5 * BB + 16;
+  __shared__ TC BT_[PG * BP];
+#define BT(p, beta, J) BT_[(p) * BP + (beta) * BB + (J)]
+  int b = blockIdx.x, ks = 0, ke = 0;
+  for (; b < n_bins; b += gridDim.x) {  // first non-empty bin (uniform across the workgroup)
+    ks = cell_start[b];
+    ke = cell_start[b + 1];
+    if (ke > ks) break;
+  }
+  if (b >= n_bins) return;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform across the wave
+  for (int q = t; q < PG * NI; q += 256) E(q / NI, 27, (q % NI) >> 2, q & 3) = 0;  // never written again
+  typedef typename Mfma<TC>::acc ACC;
+  ACC acc[4][4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[s][c] = ACC{0, 0, 0, 0};
+  // output tiles tt = wave + 4 s: row tile mt = tt / 2 = wave / 2 + 2 s (16 rows (I, r)),
+  // column tile nt = tt % 2 = wave % 2 (16 columns J); waves 2 and 3 have no fourth
+  // tile (rows I >= 28)
+  const int lg = lane >> 4, rt = lane & 15;
+  const int r_l = Mfma<TC>::r_major ? (rt >> 2) : (rt & 3);
+  const int i_l = Mfma<TC>::r_major ? (rt & 3) : (rt >> 2);
+  int abase[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) abase[s] = lg * EP + min((wave >> 1) * 4 + 8 * s + i_l, 27) * EI + r_l;
+  const int bbase = lg * BP + (wave & 1) * 16 + rt;
+  constexpr int NQ = (PG * NI + 255) / 256;  // (p, z, r) items per thread
+  constexpr int GT0 = PF ? 192 : 0;           // first thread of the shape-function tables
+  static_assert(PG * 3 <= 64, "the tables of a group are one wave's work");
+  TC dv[NQ][5];
+  double xa = 0.0, la = 0.0;
+  // tangent entries of this thread's (p, z, r) items, position and domain size of
+  // particle (t - GT0) / 3 (axis (t - GT0) % 3) of the group starting at p0 (np particles)
+  auto load_group = [&](int p0, int np) {
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      const int q = t + 256 * j;
+      const int p = q / NI, zr = q % NI, z = zr >> 2, r = zr & 3;
+#pragma unroll
+      for (int i = 0; i < 5; ++i) dv[j][i] = (TC)0;
+      if (q < PG * NI && p < np) {
+        const TD* Dp = D + (long)(p0 + p) * NY * NZ;
+        if (r < 3) {
+          dv[j][0] = (TC)Dp[(0 * 3 + r) * NZ + z];
+          dv[j][1] = (TC)Dp[(1 * 3 + r) * NZ + z];
+          dv[j][2] = (TC)Dp[(2 * 3 + r) * NZ + z];
+          dv[j][3] = (TC)Dp[(Y_T + r) * NZ + z];
+        } else {
+          const TC dS = (TC)Dp[Y_S * NZ + z];
+          dv[j][0] = (TC)Dp[(Y_M + 0) * NZ + z];
+          dv[j][1] = (TC)Dp[(Y_M + 1) * NZ + z];
+          dv[j][2] = (TC)Dp[(Y_M + 2) * NZ + z];
+          dv[j][3] = (TC)Dp[Y_Q * NZ + z] + dS;
+          dv[j][4] = -dS;
+        }
+      }
+    }
+    xa = 0.0;
+    la = 0.0;
+    if (t >= GT0 && t < GT0 + PG * 3 && (t - GT0) / 3 < np) {
+      xa = x_s[(long)(p0 + (t - GT0) / 3) * 3 + (t - GT0) % 3];
+      la = lp_s[(long)(p0 + (t - GT0) / 3) * 3 + (t - GT0) % 3];
+    }
+  };
+  // shape-function tables of the group whose positions are in xa / la (np particles)
+  auto axis_tables = [&](int buf, int np) {
+    if (t >= GT0 && t < GT0 + PG * 3) {
+      const int p = (t - GT0) / 3, a = (t - GT0) % 3;
+      if (p < np) {
+        const Axis ax = gimp_axis(xa, la, g.h[a], g.inv_h[a]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          AXT_[buf][p][a][i] = (TC)ax.w[i];
+          AXT_[buf][p][a][3 + i] = (TC)ax.g[i];
+          AXT_[buf][p][a][6 + i] = (TC)ax.wa[i];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) AXT_[buf][p][a][i] = (TC)0;
+      }
+    }
+  };
+  int p0 = ks, cur = 0;
+  if (PF) {
+    load_group(p0, min(PG, ke - p0));
+    axis_tables(0, min(PG, ke - p0));
+  }
+  while (true) {
+    const int np = min(PG, ke - p0);
+    if (!PF) load_group(p0, np);
+    __syncthreads();  // the previous group's LDS reads are done (and, with PF, this one's tables written)
+    if (!PF) {
+      axis_tables(cur, np);
+      __syncthreads();
+    }
+    const TC(*AXT)[3][9] = AXT_[cur];
+    for (int q = t; q < PG * 5 * BB; q += 256) {
+      const int p = q / (5 * BB), beta = (q / BB) % 5, J = q % BB;
+      BT(p, beta, J) = (J < 27) ? gcomp<TC>(AXT[p], J, beta) : (TC)0;
+    }
+    // E_p[I][z][r] = (L_I D_p)[r][z]: u rows sum_b dw/dx_b D[(b,r)] + w D[T_r];
+    // the pressure row w D[Q] + sum_b dw/dx_b D[M_b] + (w - w_avg) D[S]
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      const int q = t + 256 * j;
+      if (q >= PG * NI) break;
+      const int p = q / NI, zr = q % NI, z = zr >> 2, r = zr & 3;
+      const TC d0 = dv[j][0], d1 = dv[j][1], d2 = dv[j][2], dw = dv[j][3], dwa = dv[j][4];
+      // sum-factorised over the tensor-product axes: with u = gx d0 + wx dw, v = wx d1,
+      // q = wx d2, a = wax dwa per x node, E = wz (wy u + gy v) + gz (wy q) + waz (way a)
+      TC wx[3], gx[3], ax[3], wy[3], gy[3], ay[3], wz[3], gz[3], az[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        wx[i] = AXT[p][0][i];
+        gx[i] = AXT[p][0][3 + i];
+        ax[i] = AXT[p][0][6 + i];
+        wy[i] = AXT[p][1][i];
+        gy[i] = AXT[p][1][3 + i];
+        ay[i] = AXT[p][1][6 + i];
+        wz[i] = AXT[p][2][i];
+        gz[i] = AXT[p][2][3 + i];
+        az[i] = AXT[p][2][6 + i];
+      }
+#pragma unroll
+      for (int ix = 0; ix < 3; ++ix) {
+        const TC u = gx[ix] * d0 + wx[ix] * dw, v = wx[ix] * d1, qx = wx[ix] * d2, a = ax[ix] * dwa;
+#pragma unroll
+        for (int iy = 0; iy < 3; ++iy) {
+          const TC U = wy[iy] * u + gy[iy] * v, Q = wy[iy] * qx, A2 = ay[iy] * a;
+#pragma unroll
+          for (int iz = 0; iz < 3; ++iz) E(p, ix + 3 * iy + 9 * iz, z, r) = wz[iz] * U + gz[iz] * Q + az[iz] * A2;
+        }
+      }
+    }
+    // the next group: the rest of this bin, else the first of the next non-empty bin
+    int nb = b, nks = ks, nke = ke, np0 = p0 + PG;
+    const bool bin_done = np0 >= ke;
+    if (bin_done) {
+      for (nb = b + gridDim.x; nb < n_bins; nb += gridDim.x) {
+        nks = cell_start[nb];
+        nke = cell_start[nb + 1];
+        if (nke > nks) break;
+      }
+      np0 = nks;
+    }
+    const bool more = nb < n_bins;
+    if (PF && more) load_group(np0, min(PG, nke - np0));
+    __syncthreads();  // E and B tables complete
+    // particles past np have all-zero axis tables, hence zero B
+#pragma unroll
+    for (int kst = 0; kst < KST; ++kst) {
+      const int beta = kst % 5, pb = (kst / 5) * 4;  // constants once unrolled
+      const TC bk = BT_[bbase + pb * BP + beta * BB];
+      // the step's A operands are read before its products are issued
+      TC av[4][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int z = zsel(c, beta);
+          av[s][c] = (z == ZERO) ? (TC)0 : E_[abase[s] + pb * EP + z * 4];  // z resolved at compile time
+        }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (s == 3 && wave >= 2) break;  // wave-uniform: no fourth tile
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (zsel(c, beta) != ZERO) acc[s][c] = Mfma<TC>::step(av[s][c], bk, acc[s][c]);
+      }
+    }
+    if (bin_done) {
+      // lane holds rows r = 0..3 of node I_loc = 4 mt + lane / 16 in column J_loc =
+      // 16 nt + lane % 16: one whole 4 x 4 block
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int mt = (wave >> 1) + 2 * s, nt = wave & 1;
+        const int I = mt * 4 + (lane >> 4), J = nt * 16 + (lane & 15);
+        if (I < 27 && J < 27) {
+          TC* o = cb + chunk_at(I, b) + J * 16;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o[r * 4 + c] = acc[s][c][r];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[s][c] = ACC{0, 0, 0, 0};
+      }
+    }
+    if (!more) break;
+    if (PF) {
+      cur ^= 1;
+      axis_tables(cur, min(PG, nke - np0));  // read after the next barrier
+    }
+    b = nb;
+    ks = nks;
+    ke = nke;
+    p0 = np0;
+  }
+}
+
+#undef E
+#undef BT
+
+// One workgroup per block row I, four lanes per block (one per block row r).  The
+// row's 27 candidate bins (b = I - o, -1 when outside the grid or empty) are read
+// once into LDS.
+template <typename TC, typename TV>
+__global__ void __launch_bounds__(512) k_jac_gather(gm_grid g, const int* cell_start, const TC* cb,
+                                                    const uint8_t* freem, const int* row_ptr,
+                                                    const uint64_t* row_mask, TV* vals) {
+  __shared__ int SLOT_BIT[125];
+  __shared__ int BIN[27];
+  const int I = blockIdx.x, t = threadIdx.x;
+  const uint64_t m0 = row_mask[2 * I], m1 = row_mask[2 * I + 1];
+  const int nx1 = g.nx + 1, nxy = (g.nx + 1) * (g.ny + 1);
+  const int ci[3] = {I % nx1, (I / nx1) % (g.ny + 1), I / nxy};
+  if (t < 125) {
+    const uint64_t w = (t < 64) ? m0 : m1;
+    const int sh = t & 63;
+    if ((w >> sh) & 1ull) {
+      const int below = (t < 64) ? __popcll(m0 & ((1ull << sh) - 1ull))
+                                 : __popcll(m0) + __popcll(m1 & ((1ull << sh) - 1ull));
+      SLOT_BIT[below] = t;
+    }
+  } else if (t >= 128 && t < 128 + 27) {
+    const int o = t - 128, ox = o % 3, oy = (o / 3) % 3, oz = o / 9;
+    const int bc[3] = {ci[0] - ox, ci[1] - oy, ci[2] - oz};
+    int bn = -1;
+    if (bc[0] >= 0 && bc[0] <= g.nx && bc[1] >= 0 && bc[1] <= g.ny && bc[2] >= 0 && bc[2] <= g.nz) {
+      bn = bc[0] + bc[1] * nx1 + bc[2] * nxy;
+      if (cell_start[bn + 1] == cell_start[bn]) bn = -1;
+    }
+    BIN[o] = bn;
+  }
+  __syncthreads();
+  const int nnz = __popcll(m0) + __popcll(m1);
+  const int slot = t >> 2, r = t & 3;
+  if (slot >= nnz) return;
+  const int bit = SLOT_BIT[slot];
+  const int d[3] = {bit % 5 - 2, (bit / 5) % 5 - 2, bit / 25 - 2};
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int o = 0; o < 27; ++o) {
+    const int kx = d[0] + o % 3, ky = d[1] + (o / 3) % 3, kz = d[2] + o / 9;
+    const int bn = BIN[o];
+    if (bn >= 0 && kx >= 0 && kx < 3 && ky >= 0 && ky < 3 && kz >= 0 && kz < 3) {
+      const TC* src = cb + chunk_at(o, bn) + (kx + 3 * ky + 9 * kz) * 16 + r * 4;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[c] += (double)src[c];
+    }
+  }
+  const int Jn = I + d[0] + d[1] * nx1 + d[2] * nxy;
+  const bool diag = (Jn == I);
+  const bool fr = freem[I * 4 + r];
+  TV* out = vals + (long)(row_ptr[I] + slot) * 16 + r * 4;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const bool fc = freem[Jn * 4 + c];
+    double v = (fr && fc) ? -s[c] : 0.0;
+    if (diag && r == c && !fr) v = 1.0;
+    out[c] = (TV)v;
+  }
+}
+
+// The same sums with coalesced reads: one workgroup per block row I stages the row's
+// <= 27 bin chunks (bin I - o, I_loc = o: 27 blocks, contiguous) in LDS
+// with whole 16-byte vector loads, OB chunks at a time, and every (block, row r) item
+// then adds its <= 27 contributions from LDS in the same order (o = 0..26) as
+// k_jac_gather: both write the same bits.
+template <typename TC, typename TV, int OB>
+__global__ void __launch_bounds__(256, 3) k_jac_gather_staged(gm_grid g, const int* cell_start, const TC* cb,
+                                                           const uint8_t* freem, const int* row_ptr,
+                                                           const uint64_t* row_mask, TV* vals) {
+  static_assert(27 % OB == 0, "chunk rounds cover o = 0..26");
+  constexpr int CH = 27 * 16;          // values per chunk
+  constexpr int CV = CH * sizeof(TC) / 16;  // 16-byte vectors per chunk
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  __shared__ int SLOT_BIT[125];
+  __shared__ int BIN[27];
+  __shared__ u4 ST[OB][CV];
+  const int I = blockIdx.x, t = threadIdx.x;
+  const uint64_t m0 = row_mask[2 * I], m1 = row_mask[2 * I + 1];
+  const int nx1 = g.nx + 1, nxy = (g.nx + 1) * (g.ny + 1);
+  const int ci[3] = {I % nx1, (I / nx1) % (g.ny + 1), I / nxy};
+  if (t < 125) {
+    const uint64_t w = (t < 64) ? m0 : m1;
+    const int sh = t & 63;
+    if ((w >> sh) & 1ull) {
+      const int below = (t < 64) ? __popcll(m0 & ((1ull << sh) - 1ull))
+                                 : __popcll(m0) + __popcll(m1 & ((1ull << sh) - 1ull));
+      SLOT_BIT[below] = t;
+    }
+  } else if (t >= 128 && t < 128 + 27) {
+    const int o = t - 128, ox = o % 3, oy = (o / 3) % 3, oz = o / 9;
+    const int bc[3] = {ci[0] - ox, ci[1] - oy, ci[2] - oz};
+    int bn = -1;
+    if (bc[0] >= 0 && bc[0] <= g.nx && bc[1] >= 0 && bc[1] <= g.ny && bc[2] >= 0 && bc[2] <= g.nz) {
+      bn = bc[0] + bc[1] * nx1 + bc[2] * nxy;
+      if (cell_start[bn + 1] == cell_start[bn]) bn = -1;
+    }
+    BIN[o] = bn;
+  }
+  __syncthreads();
+  const int nnz = __popcll(m0) + __popcll(m1);
+  // items (slot, r) = (it / 4, it % 4), it = t and t + 256
+  int dd[2][3];
+  bool live[2];
+  double s[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int it = t + 256 * h;
+    live[h] = it < 4 * nnz;
+    const int bit = live[h] ? SLOT_BIT[it >> 2] : 62;
+    dd[h][0] = bit % 5 - 2;
+    dd[h][1] = (bit / 5) % 5 - 2;
+    dd[h][2] = bit / 25 - 2;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s[h][c] = 0.0;
+  }
+#pragma unroll 1
+  for (int o0 = 0; o0 < 27; o0 += OB) {
+    if (o0) __syncthreads();  // the previous round's LDS reads are done
+    // all of a thread's loads are issued before its first LDS store
+    constexpr int NJ = (OB * CV + 255) / 256;
+    u4 tmp[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int q = t + 256 * j;
+      tmp[j] = u4{0u, 0u, 0u, 0u};
+      if (q < OB * CV) {
+        const int oo = q / CV, f = q % CV;
+        const int bn = BIN[o0 + oo];
+        if (bn >= 0) tmp[j] = reinterpret_cast<const u4*>(cb + chunk_at(o0 + oo, bn))[f];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int q = t + 256 * j;
+      if (q < OB * CV) ST[q / CV][q % CV] = tmp[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!live[h]) continue;
+      const int r = (t + 256 * h) & 3;
+#pragma unroll 3
+      for (int oo = 0; oo < OB; ++oo) {
+        const int o = o0 + oo;
+        const int kx = dd[h][0] + o % 3, ky = dd[h][1] + (o / 3) % 3, kz = dd[h][2] + o / 9;
+        if (BIN[o] >= 0 && kx >= 0 && kx < 3 && ky >= 0 && ky < 3 && kz >= 0 && kz < 3) {
+          const TC* src = reinterpret_cast<const TC*>(&ST[oo][0]) + (kx + 3 * ky + 9 * kz) * 16 + r * 4;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) s[h][c] += (double)src[c];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (!live[h]) continue;
+    const int it = t + 256 * h, slot = it >> 2, r = it & 3;
+    const int Jn = I + dd[h][0] + dd[h][1] * nx1 + dd[h][2] * nxy;
+    const bool diag = (Jn == I);
+    const bool fr = freem[I * 4 + r];
+    TV* out = vals + (long)(row_ptr[I] + slot) * 16 + r * 4;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const bool fc = freem[Jn * 4 + c];
+      double v = (fr && fc) ? -s[h][c] : 0.0;
+      if (diag && r == c && !fr) v = 1.0;
+      out[c] = (TV)v;
+    }
+  }
+}
 
 // Line sums.  A workgroup takes the bins of one segment [xs, xe) of a bin line (fixed y, z)
 // in ascending x.  The nodes x, x + 1, x + 2 that a bin reaches lie in the three slots
@@ -119,30 +548,23 @@ constexpr int MAX_SEG = 61;  // bins of a line segment (with two before it and t
 // node is x: 405 of 729 blocks) are stored and cleared.  Pairs that bins before xs reach as
 // well belong to this segment when min(row x, column x) >= xs; the sweep starts two bins
 // early to have their whole sum.
-// A bin's particles are taken four at a time (a group).  The first CW waves hold the
-// accumulators and do nothing but products and stores.  The others, in teams of four waves,
-// prepare E_p and the B operand of one coming group each in the other half of the LDS
-// buffers, stage the tangent rows and shape-function tables of the groups after those and
-// load the rows of the next ones: one barrier for CW / 4 groups, and neither the tables nor
-// the loads are in the matrix cores' way.
-//   FP32: 8 product waves (two tiles each) and two teams.  A bin's products are summed from
-//     zero in one set of accumulators and added to the line's sums in another, so that the
-//     line's longer sum has one rounding a bin more and no longer chains (the matrix stays
-//     as near the 64-bit one as with bin sums added in FP64).
-//   FP64: 4 product waves (four tiles each) and one team, for the operands' size in LDS.
-// The operands are formed in FP64 and rounded once.
+// A bin's particles are taken four at a time (a group).  The first four waves hold the
+// accumulators (four tiles each) and do nothing but products and stores.  The other four
+// prepare E_p and the B operand of the coming group in the other half of the LDS buffers,
+// stage the tangent rows and shape-function tables of the group after it and load the rows of
+// the next ones: one barrier a group, and neither the tables nor the loads are in the matrix
+// cores' way.
 // K order: a K step of the MFMA is one shape-function component beta and the four
 // particles (lane group l / 16 = particle).  After the
 // K loop unrolls, every A and B operand address is a per-lane base plus an immediate,
 // and the (c, beta) products that vanish (u columns: no w term except the penalty
 // on u_z, no w_avg term) are not issued.  Every segment length adds the same products in
 // the same order, so all of them write the same bits.
-template <typename TD, typename TC, int CW>
-__global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const double* x_s, const double* lp_s,
-                                                               const int* cell_start, int n_p, int seg_len,
-                                                               int n_seg, const TD* D, TC* cb) {
-  constexpr int TEAMS = CW / 4, TILES = 16 / CW;
-  constexpr bool BIN_SUMS = sizeof(TC) == 4;
+__global__ void __launch_bounds__(512, 2) k_jac_line(gm_grid g, const double* x_s, const double* lp_s,
+                                                     const int* cell_start, int n_p, int seg_len, int n_seg,
+                                                     const double* D, double* cb) {
+  constexpr int CW = 4;             // product waves
+  constexpr int TILES = 16 / CW;
   constexpr int PG = 4;             // particles of a group: one quad of K steps
   constexpr int NI = 4 * NZ;        // (z, r) entries of a node row of E_p
   // shape-function tables of the sweep's particles, a ring filled a batch at a time
@@ -150,15 +572,15 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
   __shared__ double AXT_[RING][3][9];
   // tangent rows of a group (particles are in bin order, so a group's rows are contiguous)
   constexpr int DROW = NY * NZ;
-  __shared__ TD DR_[TEAMS][2][PG * DROW];
+  __shared__ double DR_[2][PG * DROW];
   // E_p[I][z][r] (r fastest), node rows 68 entries apart and particles 1840: the 64
   // (particle, I, r) entries a wave reads at once fall in 64 distinct banks.  (The padding
   // rows of the last row tile read row 26; they are never stored.)
   constexpr int EI = 68, EP = 27 * EI + 4;
-  __shared__ TC E_[TEAMS][2][PG * EP];
+  __shared__ double E_[2][PG * EP];
   // B operand g_p[J][beta], J padded to 32 with zeros, particles 176 entries apart
   constexpr int BB = 32, BP = 5 * BB + 16;
-  __shared__ TC BT_[TEAMS][2][PG * BP];
+  __shared__ double BT_[2][PG * BP];
   const int line = blockIdx.x / n_seg;  // y + (ny + 1) z
   const int lb = line * (g.nx + 1);     // the line's first bin (and node)
   const int xs = (blockIdx.x % n_seg) * seg_len, xe = min(xs + seg_len, g.nx + 1);
@@ -189,11 +611,6 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
     }
     return q;
   };
-  auto next_round = [&](Group q) {
-#pragma unroll
-    for (int k = 0; k < TEAMS; ++k) q = next(q);
-    return q;
-  };
   Group cur{x0, 0, 0};
   seek(cur);
   // shape-function tables of particles [tabs, tabs + BATCH) of the sweep: 48 lanes of the last
@@ -209,7 +626,7 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
     xa = x_s[at];
     la = lp_s[at];
   };
-  // q: the last group of a round (none: the sweep ends in that round)
+  // the tables of group q (none: the sweep ends before it)
   auto tables_for = [&](const Group& q) {
     if ((q.x < xe ? min(q.p0 + PG, q.ke) - ps : n_sweep) <= tabs) return;  // uniform
     if (tl >= 0 && tl < 3 * BATCH) {
@@ -227,20 +644,18 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
   };
   if (wave < CW) {
     // ---------------------------------------------------------------- products
-    typedef typename Mfma<TC>::acc ACC;
-    ACC acc[TILES][4], sum[TILES][4];  // (sum: BIN_SUMS only)
+    d4v acc[TILES][4];
 #pragma unroll
     for (int s = 0; s < TILES; ++s)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[s][c] = sum[s][c] = ACC{0, 0, 0, 0};
+      for (int c = 0; c < 4; ++c) acc[s][c] = d4v{0, 0, 0, 0};
     // output tiles w + CW s: row tile mt = w / 2 + CW / 2 s (16 rows (I, r)), column tile
     // nt = w % 2 (16 columns J); the last waves have no last tile (rows I >= 28).  Node index
     // I = 9 slot + oy + 3 oz, J likewise.
     const int w = wave;
     const bool last = (w >> 1) + (CW >> 1) * (TILES - 1) < 7;
     const int lg = lane >> 4, rt = lane & 15;
-    const int r_l = Mfma<TC>::r_major ? (rt >> 2) : (rt & 3);
-    const int i_l = Mfma<TC>::r_major ? (rt & 3) : (rt >> 2);
+    const int r_l = rt >> 2, i_l = rt & 3;  // r-major tiles
     int abase[TILES];
 #pragma unroll
     for (int s = 0; s < TILES; ++s)
@@ -256,89 +671,68 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
       const int J = (w & 1) * 16 + (l & 15), jslot = J / 9, jyz = J % 9;
 #pragma unroll
       for (int s = 0; s < TILES; ++s) {
-        ACC* leave = BIN_SUMS ? sum[s] : acc[s];
         const int I = ((w >> 1) + (CW >> 1) * s) * 4 + (l >> 4), islot = I / 9, iyz = I - 9 * islot;
         if (I < 27 && J < 27 && (islot == q || jslot == q)) {
           const int di = islot >= q ? islot - q : islot - q + 3, dj = jslot >= q ? jslot - q : jslot - q + 3;
           if (B >= xs && B + di <= g.nx) {
-            TC* o = cb + (di == 0 ? chunk_a(iyz, lb + B) + (dj * 9 + jyz) * 4 : chunk_b(iyz, lb + B, di) + jyz * 4);
+            double* o = cb + (di == 0 ? chunk_a(iyz, lb + B) + (dj * 9 + jyz) * 4 : chunk_b(iyz, lb + B, di) + jyz * 4);
             const int plane = di == 0 ? 27 * 4 : 9 * 4;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) *reinterpret_cast<ACC*>(o + c * plane) = leave[c];
+            for (int c = 0; c < 4; ++c) *reinterpret_cast<d4v*>(o + c * plane) = acc[s][c];
           }
 #pragma unroll
-          for (int c = 0; c < 4; ++c) leave[c] = ACC{0, 0, 0, 0};
+          for (int c = 0; c < 4; ++c) acc[s][c] = d4v{0, 0, 0, 0};
         }
       }
     };
-    Group gt = cur;  // the last group of the round whose tables come next
+    Group gt = cur;  // the group whose tables come next
     if (wave == CW - 1) {
-#pragma unroll
-      for (int k = 1; k < TEAMS; ++k) gt = next(gt);
       load_tables(0);
       tables_for(gt);
-      gt = next_round(gt);
+      gt = next(gt);
       tables_for(gt);
     }
     __syncthreads();
     __syncthreads();
     for (int buf = 0; cur.x < xe; buf ^= 1) {
       if (wave == CW - 1) {
-        gt = next_round(gt);
+        gt = next(gt);
         tables_for(gt);
       }
-#pragma unroll 1
-      for (int k = 0; k < TEAMS && cur.x < xe; ++k) {
-        // particles past the bin's last have zero B; a tile's operands are read before its products
-        const TC *E = E_[k][buf], *BT = BT_[k][buf];
-        TC b[5];
+      // particles past the bin's last have zero B; a tile's operands are read before its products
+      const double *E = E_[buf], *BT = BT_[buf];
+      double b[5];
 #pragma unroll
-        for (int beta = 0; beta < 5; ++beta) b[beta] = BT[bbase + beta * BB];
-        auto products = [&](auto tile) {
-          constexpr int s = decltype(tile)::value;
-          TC a[4][5];
+      for (int beta = 0; beta < 5; ++beta) b[beta] = BT[bbase + beta * BB];
 #pragma unroll
-          for (int beta = 0; beta < 5; ++beta)
+      for (int s = 0; s < TILES; ++s) {
+        if (s == TILES - 1 && !last) break;  // wave-uniform
+        double a[4][5];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-              if (zsel(c, beta) != ZERO) a[c][beta] = E[abase[s] + zsel(c, beta) * 4];
+        for (int beta = 0; beta < 5; ++beta)
 #pragma unroll
-          for (int beta = 0; beta < 5; ++beta)
+          for (int c = 0; c < 4; ++c)
+            if (zsel(c, beta) != ZERO) a[c][beta] = E[abase[s] + zsel(c, beta) * 4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)  // (c, beta) resolved at compile time
-              if (zsel(c, beta) != ZERO) acc[s][c] = Mfma<TC>::step(a[c][beta], b[beta], acc[s][c]);
-        };
-        if constexpr (TILES == 4) {
-          products(Int<0>{});
-          products(Int<1>{});
-        }
-        products(Int<TILES - 2>{});
-        if (last) products(Int<TILES - 1>{});  // wave-uniform
-        const Group nxt = next(cur);
-        if (nxt.x != cur.x) {  // the bin's last group
-          if (BIN_SUMS) {
+        for (int beta = 0; beta < 5; ++beta)
 #pragma unroll
-            for (int s = 0; s < TILES; ++s)
-#pragma unroll
-              for (int c = 0; c < 4; ++c) {
-                sum[s][c] += acc[s][c];
-                acc[s][c] = ACC{0, 0, 0, 0};
-              }
-          }
-          // up to three steps clear every pair the sweep has touched
-          for (int B = cur.x; B < min(min(nxt.x, cur.x + 3), xe); ++B) flush(B);
-        }
-        cur = nxt;
+          for (int c = 0; c < 4; ++c)  // (c, beta) resolved at compile time
+            if (zsel(c, beta) != ZERO) acc[s][c] = Mfma<double>::step(a[c][beta], b[beta], acc[s][c]);
       }
+      const Group nxt = next(cur);
+      // after the bin's last group; up to three steps clear every pair the sweep has touched
+      if (nxt.x != cur.x)
+        for (int B = cur.x; B < min(min(nxt.x, cur.x + 3), xe); ++B) flush(B);
+      cur = nxt;
       __syncthreads();
     }
     return;
   }
   // ------------------------------------------------------------------ operands
-  const int team = (wave - CW) >> 2, t = (threadIdx.x - 64 * CW) & 255;
-  constexpr int VD = 16 / sizeof(TD);  // tangent values per load
+  const int t = threadIdx.x - 64 * CW;
+  constexpr int VD = 2;  // tangent values per load
   constexpr int ND = (PG * DROW + 256 * VD - 1) / (256 * VD);
-  typedef TD dvec __attribute__((ext_vector_type(16 / sizeof(TD)), aligned(sizeof(TD))));
+  typedef double dvec __attribute__((ext_vector_type(2), aligned(8)));
   // tangent rows of a group: addresses clamped rather than loads skipped, so that the loads
   // of two groups stay in flight (a skipped load leaves the count of those in flight unknown)
   dvec even[ND], odd[ND];
@@ -357,9 +751,9 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
       const int back = (int)max(k0 + k - ((long)n_p * DROW - VD), 0L);
 #pragma unroll
       for (int i = 0; i < VD; ++i) {
-        TD v = from[j][i];
-        if (back > 0) v = i + back < VD ? from[j][min(i + back, VD - 1)] : (TD)0;
-        if (k + i < PG * DROW) DR_[team][buf][k + i] = k0 + k + i < lim ? v : (TD)0;
+        double v = from[j][i];
+        if (back > 0) v = i + back < VD ? from[j][min(i + back, VD - 1)] : 0.0;
+        if (k + i < PG * DROW) DR_[buf][k + i] = k0 + k + i < lim ? v : 0.0;
       }
     }
   };
@@ -368,16 +762,16 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
     // B operand: threads (J, particle)
     if (t < PG * 32) {
       const int p = t >> 5, Jb = t & 31;
-      TC* B = BT_[team][buf] + p * BP + Jb;
+      double* B = BT_[buf] + p * BP + Jb;
       const double(*AX)[9] = AXT_[(q.p0 - ps + p) % RING];
       if (Jb < 27 && p < np) {
         const int js = Jb / 9, sx = js >= rot ? js - rot : js - rot + 3, jy = Jb % 3, jz = (Jb / 3) % 3;
         const double wx = AX[0][sx], wy = AX[1][jy], wz = AX[2][jz];
-        B[0] = (TC)(wx * wy * wz);
-        B[BB] = (TC)(AX[0][3 + sx] * wy * wz);
-        B[2 * BB] = (TC)(wx * AX[1][3 + jy] * wz);
-        B[3 * BB] = (TC)(wx * wy * AX[2][3 + jz]);
-        B[4 * BB] = (TC)(AX[0][6 + sx] * AX[1][6 + jy] * AX[2][6 + jz]);
+        B[0] = (wx * wy * wz);
+        B[BB] = (AX[0][3 + sx] * wy * wz);
+        B[2 * BB] = (wx * AX[1][3 + jy] * wz);
+        B[3 * BB] = (wx * wy * AX[2][3 + jz]);
+        B[4 * BB] = (AX[0][6 + sx] * AX[1][6 + jy] * AX[2][6 + jz]);
       } else {
 #pragma unroll
         for (int beta = 0; beta < 5; ++beta) B[beta * BB] = 0;
@@ -387,10 +781,10 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
     // the pressure row w D[Q] + sum_b dw/dx_b D[M_b] + (w - w_avg) D[S]
     if (t < PG * NI) {
       const int p = t / NI, zr = t % NI, z = zr >> 2, r = zr & 3;
-      const TD* Dp = DR_[team][buf] + p * DROW + z;
+      const double* Dp = DR_[buf] + p * DROW + z;
       const int k0 = r < 3 ? r : Y_M, dk = r < 3 ? 3 : 1;
       const double d0 = Dp[k0 * NZ], d1 = Dp[(k0 + dk) * NZ], d2 = Dp[(k0 + 2 * dk) * NZ];
-      const double dS = r < 3 ? 0.0 : (double)Dp[Y_S * NZ];
+      const double dS = r < 3 ? 0.0 : Dp[Y_S * NZ];
       const double dw = Dp[(r < 3 ? Y_T + r : Y_Q) * NZ] + dS, dwa = -dS;
       // sum-factorised over the tensor-product axes: with u = gx d0 + wx dw, v = wx d1,
       // q = wx d2, a = wax dwa per x node, E = wz (wy u + gy v) + gz (wy q) + waz (way a)
@@ -407,48 +801,45 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
       }
 #pragma unroll
       for (int ix = 0; ix < 3; ++ix) {
-        TC* Eo = E_[team][buf] + p * EP + zr + 9 * EI * (ix + rot >= 3 ? ix + rot - 3 : ix + rot);
+        double* Eo = E_[buf] + p * EP + zr + 9 * EI * (ix + rot >= 3 ? ix + rot - 3 : ix + rot);
         const double wx = AX[0][ix], u = AX[0][3 + ix] * d0 + wx * dw, v = wx * d1, qx = wx * d2, a = AX[0][6 + ix] * dwa;
 #pragma unroll
         for (int iy = 0; iy < 3; ++iy) {
           const double U = wy[iy] * u + gy[iy] * v, Q = wy[iy] * qx, A2 = ay[iy] * a;
 #pragma unroll
-          for (int iz = 0; iz < 3; ++iz) Eo[(iy + 3 * iz) * EI] = (TC)(wz[iz] * U + gz[iz] * Q + az[iz] * A2);
+          for (int iz = 0; iz < 3; ++iz) Eo[(iy + 3 * iz) * EI] = (wz[iz] * U + gz[iz] * Q + az[iz] * A2);
         }
       }
     }
   };
-  // round i: the groups TEAMS i + team; `cur` stays the round's first group
-  Group g0 = cur;
-  for (int k = 0; k < team; ++k) g0 = next(g0);
-  Group g1 = next_round(g0), g2 = next_round(g1), g3 = next_round(g2);
+  Group g0 = cur, g1 = next(g0), g2 = next(g1), g3 = next(g2);
   load_group(g0, even);
   load_group(g1, odd);
   stage_group(g0, 0, even);
   load_group(g2, even);
   __syncthreads();
-  if (g0.x < xe) operands(g0, 0);
+  operands(g0, 0);
   stage_group(g1, 1, odd);
   load_group(g3, odd);
   __syncthreads();
-  // while the products of round i run: the operands of i + 1, the rows and tables of i + 2,
+  // while the products of group i run: the operands of i + 1, the rows and tables of i + 2,
   // and the loads of i + 3 and i + 4 on their way
   while (cur.x < xe) {
     if (g1.x < xe) operands(g1, 1);
     stage_group(g2, 0, even);
-    const Group g4 = next_round(g3);
+    const Group g4 = next(g3);
     load_group(g4, even);
     __syncthreads();
-    cur = next_round(cur);
+    cur = next(cur);
     if (cur.x >= xe) break;
     if (g2.x < xe) operands(g2, 0);
     stage_group(g3, 1, odd);
     g1 = g3;
     g2 = g4;
-    g3 = next_round(g4);
+    g3 = next(g4);
     load_group(g3, odd);
     __syncthreads();
-    cur = next_round(cur);
+    cur = next(cur);
   }
 }
 
@@ -456,11 +847,10 @@ __global__ void __launch_bounds__(128 * CW, CW / 2) k_jac_line(gm_grid g, const 
 // the <= 9 line sums of its four rows, all loads issued before the first is added.  Both
 // the reads (runs of 16-byte vectors) and the writes (the row's blocks, through LDS) are
 // coalesced; bound by HBM on the workspace and the matrix.
-template <typename TC, typename TV, int T>
-__global__ void __launch_bounds__(T) k_jac_gather(gm_grid g, const int* cell_start, const TC* cb,
-                                                  const uint8_t* freem, const int* row_ptr,
-                                                  const uint64_t* row_mask, TV* vals) {
-  typedef typename Mfma<TC>::acc V4;
+template <typename TV, int T>
+__global__ void __launch_bounds__(T) k_jac_line_gather(gm_grid g, const int* cell_start, const double* cb,
+                                                       const uint8_t* freem, const int* row_ptr,
+                                                       const uint64_t* row_mask, TV* vals) {
   __shared__ int NODE[9], MASK[9];
   __shared__ __align__(16) TV OUT[125 * 16];
   const int I = blockIdx.x, t = threadIdx.x;
@@ -490,12 +880,11 @@ __global__ void __launch_bounds__(T) k_jac_gather(gm_grid g, const int* cell_sta
   const int slot = bit < 64 ? __popcll(m0 & ((1ull << (bit & 63)) - 1ull))
                             : __popcll(m0) + __popcll(m1 & ((1ull << (bit & 63)) - 1ull));
   __syncthreads();
-  // column dofs a thread has in flight: all of them in FP64 (1.95 -> 1.83 ms), one in FP32 (1.06; all 1.09)
-  constexpr int UC = sizeof(TC) == 8 ? 4 * 128 / T : 1;
-#pragma unroll UC
+  // all column dofs of a thread in flight (1.95 -> 1.83 ms)
+#pragma unroll
   for (int c0 = 0; c0 < 4 * 128 / T; ++c0) {
     const int c = (t >> 7) + c0 * (T / 128);
-    V4 v[9];
+    d4v v[9];
     bool on[9];
 #pragma unroll
     for (int o = 0; o < 9; ++o) {
@@ -503,13 +892,13 @@ __global__ void __launch_bounds__(T) k_jac_gather(gm_grid g, const int* cell_sta
       on[o] = live && ky >= 0 && ky < 3 && kz >= 0 && kz < 3 && ((MASK[o] >> dx) & 1);
       const long at = dx >= 2 ? chunk_a(o, n) + (c * 27 + (dx - 2) * 9 + k) * 4
                               : chunk_b(o, n + dx - 2, 2 - dx) + (c * 9 + k) * 4;
-      v[o] = *reinterpret_cast<const V4*>(cb + (on[o] ? at : 0L));
+      v[o] = *reinterpret_cast<const d4v*>(cb + (on[o] ? at : 0L));
     }
     double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int o = 0; o < 9; ++o)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s[r] += on[o] ? (double)v[o][r] : 0.0;
+      for (int r = 0; r < 4; ++r) s[r] += on[o] ? v[o][r] : 0.0;
     if (live) {  // masks, sign, identity rows
       const int Jn = I + (dx - 2) + dy * nx1 + dz * nxy;
       const bool diag = (Jn == I), fc = freem[Jn * 4 + c];
@@ -916,13 +1305,21 @@ extern "C" int gm_p2g_binned(const gm_grid* g, const gm_bins* b, double threshol
 
 extern "C" size_t gm_node_jacobian_work_bytes(const gm_grid* g, int tangent_fp32) {
   if (!g) return 0;
-  return (size_t)g->n_nodes * (size_t)CB_NODE * (tangent_fp32 ? sizeof(float) : sizeof(double));
+  return (size_t)g->n_nodes * (size_t)CB_BIN * (tangent_fp32 ? sizeof(float) : sizeof(double));
 }
 
 // ------------------------------------------------------------ variants and their tuner
+// Product variants of the per-bin form (particles per group, workgroups per CU, grid):
+//   FP32 tangent: 0 (8, 2, one per bin), 1 (8, 2, persistent), 2 (4, 4, persistent), 3 (4, 3, persistent)
+//   FP64 tangent: 0 (4, 2, one per bin), 1 (4, 2, persistent), 2 (8, 1, one per bin), 3 (8, 1, persistent)
+// "persistent": one workgroup per resident slot (CUs x workgroups per CU), each
+// sweeping bins blockIdx.x + k gridDim.x, with the next group's loads issued before
+// the current group's products; "one per bin": loads at the top of each group.  Gather
+// variants: 0 (per-lane reads from the workspace), 1 (all 27 chunks of a row staged in
+// LDS at once; 9 at a time in FP64), 2 (9 at a time; 3 in FP64).
 // Variants of the line sums: 0 the number of segments of a line that best_segments picks,
-// 1 twice and 2 three times as many, 3 one segment (as few as MAX_SEG allows).  Gather
-// variants: 128, 256 or 512 threads a row.  Every variant writes the same bits.
+// 1 twice and 2 three times as many, 3 one segment (as few as MAX_SEG allows); their gather's:
+// 128, 256 or 512 threads a row.  Every variant of a form writes the same bits.
 namespace {
 constexpr int N_BIN_VARIANTS = 4, N_GATHER_VARIANTS = 3;
 int g_bin_variant[2] = {0, 0};     // [tangent_fp32]
@@ -944,8 +1341,8 @@ int cu_count() {
 // the workgroups do not come out even over the CUs: the number of segments with the least
 // (rounds + 1/2) x (bins of a segment + 2), at least one round.  The half round is what the
 // lines without particles (which end at once) and the XCDs' shares make of the last one: whole
-// rounds instead pick 1 and 3 segments for 21 x 17 x 13 (FP64) and 48 x 9 x 7 cells (FP32), 249 and
-// 149 us where 2 and 6 take 212 and 117.  (Some six particles a bin are taken for granted.)
+// rounds instead pick 1 segment for 21 x 17 x 13 cells, 249 us where 2 take 212.  (Some six
+// particles a bin are taken for granted.)
 int best_segments(int nbx, int lines, int n_p, int slots) {
   const double busy = std::max(1.0, std::min<double>(lines, n_p / (6.0 * nbx)));
   int best = 1;
@@ -961,26 +1358,51 @@ int best_segments(int nbx, int lines, int n_p, int slots) {
   return best;
 }
 
+// the form of an assembly: FP32 sums per bin, FP64 along lines of bins
+bool line_sums(const gm_grid*, const gm_bins*, int fp32) { return !fp32; }
+
 int launch_bins(const gm_grid* g, const gm_bins* b, const void* D, int fp32, int variant, void* work,
                 hipStream_t s) {
   const int n = g->n_nodes;
   const int cus = cu_count();
   GM_REQUIRE(cus > 0, "gm_jacobian_bins: no device properties");
-  const int nbx = g->nx + 1, lines = n / nbx;
-  const int slots = cus;  // one workgroup per CU (the operand buffers in LDS)
-  int n_seg = best_segments(nbx, lines, b->n_particles, slots);
-  if (variant == 1) n_seg *= 2;
-  if (variant == 2) n_seg *= 3;
-  if (variant == 3) n_seg = 1;
-  n_seg = std::min(std::max(n_seg, (nbx + MAX_SEG - 1) / MAX_SEG), nbx);
-  const int len = (nbx + n_seg - 1) / n_seg;
-  const unsigned wgs = (unsigned)lines * n_seg;
-  if (fp32)
-    k_jac_line<float, float, 8><<<wgs, 1024, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->n_particles, len, n_seg,
-                                                  (const float*)D, (float*)work);
-  else
-    k_jac_line<double, double, 4><<<wgs, 512, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->n_particles, len,
-                                                   n_seg, (const double*)D, (double*)work);
+  if (line_sums(g, b, fp32)) {
+    const int nbx = g->nx + 1, lines = n / nbx;
+    int n_seg = best_segments(nbx, lines, b->n_particles, cus);  // one workgroup per CU (the operand buffers in LDS)
+    if (variant == 1) n_seg *= 2;
+    if (variant == 2) n_seg *= 3;
+    if (variant == 3) n_seg = 1;
+    n_seg = std::min(std::max(n_seg, (nbx + MAX_SEG - 1) / MAX_SEG), nbx);
+    const int len = (nbx + n_seg - 1) / n_seg;
+    k_jac_line<<<(unsigned)lines * n_seg, 512, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->n_particles, len, n_seg,
+                                                       (const double*)D, (double*)work);
+    GM_LAUNCH_CHECK();
+    return 0;
+  }
+#define GM_BIN(TT, PG, OCC, PERSIST)                                                                     \
+  if (PERSIST)                                                                                           \
+    k_jac_bin<TT, TT, PG, OCC, true><<<std::min(n, cus * OCC), 256, 0, s>>>(*g, b->x_s, b->lp_s,          \
+                                                                        b->cell_start, n, (const TT*)D, \
+                                                                        (TT*)work);                     \
+  else                                                                                                   \
+    k_jac_bin<TT, TT, PG, OCC, false><<<n, 256, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, n, (const TT*)D, \
+                                                      (TT*)work)
+  if (fp32) {
+    switch (variant) {
+      case 0: GM_BIN(float, 8, 2, false); break;
+      case 1: GM_BIN(float, 8, 2, true); break;
+      case 2: GM_BIN(float, 4, 4, true); break;
+      default: GM_BIN(float, 4, 3, true); break;
+    }
+  } else {
+    switch (variant) {
+      case 0: GM_BIN(double, 4, 2, false); break;
+      case 1: GM_BIN(double, 4, 2, true); break;
+      case 2: GM_BIN(double, 8, 1, false); break;
+      default: GM_BIN(double, 8, 1, true); break;
+    }
+  }
+#undef GM_BIN
   GM_LAUNCH_CHECK();
   return 0;
 }
@@ -988,16 +1410,31 @@ int launch_bins(const gm_grid* g, const gm_bins* b, const void* D, int fp32, int
 int launch_gather(const gm_grid* g, const gm_bins* b, const gm_pattern* pat, int fp32, int variant,
                   const void* work, const uint8_t* freem, void* vals, int vals_fp32, hipStream_t s) {
   const int n = g->n_nodes;
-#define GM_GATHER_T(TCC, TVV, T)                                                                               \
-  k_jac_gather<TCC, TVV, T><<<n, T, 0, s>>>(*g, b->cell_start, (const TCC*)work, freem, pat->row_ptr,          \
+#define GM_LINES(TVV, T)                                                                                        \
+  k_jac_line_gather<TVV, T><<<n, T, 0, s>>>(*g, b->cell_start, (const double*)work, freem, pat->row_ptr,        \
                                             pat->row_mask, (TVV*)vals)
-#define GM_GATHER(TCC, TVV)                          \
-  do {                                               \
-    if (variant == 0) GM_GATHER_T(TCC, TVV, 128);    \
-    else if (variant == 1) GM_GATHER_T(TCC, TVV, 256); \
-    else GM_GATHER_T(TCC, TVV, 512);                 \
-  } while (0)
-  if (fp32) {
+#define GM_GATHER(TCC, TVV)                                                                                      \
+  if (variant == 0)                                                                                              \
+    k_jac_gather<TCC, TVV><<<n, 512, 0, s>>>(*g, b->cell_start, (const TCC*)work, freem, pat->row_ptr,         \
+                                             pat->row_mask, (TVV*)vals);                                       \
+  else if (variant == 1)                                                                                         \
+    k_jac_gather_staged<TCC, TVV, sizeof(TCC) == 4 ? 27 : 9><<<n, 256, 0, s>>>(                                 \
+        *g, b->cell_start, (const TCC*)work, freem, pat->row_ptr, pat->row_mask, (TVV*)vals);                  \
+  else                                                                                                           \
+    k_jac_gather_staged<TCC, TVV, sizeof(TCC) == 4 ? 9 : 3><<<n, 256, 0, s>>>(                                  \
+        *g, b->cell_start, (const TCC*)work, freem, pat->row_ptr, pat->row_mask, (TVV*)vals)
+  if (line_sums(g, b, fp32)) {
+    if (variant == 0) {
+      if (vals_fp32) GM_LINES(float, 128);
+      else GM_LINES(double, 128);
+    } else if (variant == 1) {
+      if (vals_fp32) GM_LINES(float, 256);
+      else GM_LINES(double, 256);
+    } else {
+      if (vals_fp32) GM_LINES(float, 512);
+      else GM_LINES(double, 512);
+    }
+  } else if (fp32) {
     if (vals_fp32) GM_GATHER(float, float);
     else GM_GATHER(float, double);
   } else {
@@ -1005,7 +1442,7 @@ int launch_gather(const gm_grid* g, const gm_bins* b, const gm_pattern* pat, int
     else GM_GATHER(double, double);
   }
 #undef GM_GATHER
-#undef GM_GATHER_T
+#undef GM_LINES
   GM_LAUNCH_CHECK();
   return 0;
 }

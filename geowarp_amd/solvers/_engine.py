@@ -105,10 +105,10 @@ class Engine:
         self.penalty = None
         self.penalty_pc = True
         self.vals_pc = None
-        # node Jacobian and residual of the 3D u-p form: 'bins' (per-bin sums -- the Jacobian's
-        # as products on the matrix cores -- into a workspace of up to n_nodes x 6480 values,
-        # then a fixed-order gather) or 'rows' (one workgroup or thread per node row, no
-        # workspace)
+        # node Jacobian and residual of the 3D u-p form: 'bins' (sums per bin, or of FP64
+        # Jacobians on larger grids per line of bins -- the Jacobian's as products on the matrix
+        # cores -- into a workspace of up to n_nodes x 11664 values, then a fixed-order gather)
+        # or 'rows' (one workgroup or thread per node row, no workspace)
         self.jacobian_kernel = os.environ.get('GM_JACOBIAN_KERNEL', 'bins')
         # 3D u-p P2G (flags and consistent-mass right-hand side): per particle bin, then a
         # fixed-order gather per node (True), or one thread per node over its candidates

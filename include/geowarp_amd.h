@@ -103,27 +103,33 @@ int gm_node_jacobian(const gm_grid* g, const gm_bins* bins, const gm_pattern* pa
                      const uint8_t* freem, void* vals, int vals_fp32, int coupled, hipStream_t stream);
 
 /* The same matrix for the 3D u-p form (the reference's qc3d:285-321 coloured
-   reverse sweeps), assembled on the matrix cores per line of particle bins along
-   x: the line's sums of its node blocks go to the workspace `work` (at least
-   gm_node_jacobian_work_bytes(g, tangent_fp32) bytes: n_nodes x 6480 values
-   of the tangent's precision), then every block of the pattern sums the lines
-   that hold both of its nodes in a fixed order.  Arithmetic in the tangent's
+   reverse sweeps), assembled on the matrix cores: the sums of each particle bin's 27 x 27
+   node blocks (FP64 on larger grids: of each line of bins along x) go to the workspace
+   `work` (at least gm_node_jacobian_work_bytes(g, tangent_fp32) bytes: n_nodes x 11664
+   values of the tangent's precision), then every block of the pattern sums the bins (lines)
+   that hold both of its nodes in a fixed order, in FP64.  Arithmetic in the tangent's
    precision; -1 for another form or a smaller workspace. */
 size_t gm_node_jacobian_work_bytes(const gm_grid* g, int tangent_fp32);
 int gm_node_jacobian_binned(const gm_grid* g, const gm_bins* bins, const gm_pattern* pat, const void* D,
                             int tangent_fp32, const uint8_t* freem, void* vals, int vals_fp32, void* work,
                             size_t work_bytes, hipStream_t stream);
 /* Its two phases, callable separately (gm_node_jacobian_binned is the pair): the
-   line sums into `work`, and the per-block gather from `work` into vals. */
+   products into `work`, and the per-block gather from `work` into vals; both with the same
+   grid and bins. */
 int gm_jacobian_bins(const gm_grid* g, const gm_bins* bins, const void* D, int tangent_fp32, void* work,
                      size_t work_bytes, hipStream_t stream);
 int gm_jacobian_gather(const gm_grid* g, const gm_bins* bins, const gm_pattern* pat, int tangent_fp32,
                        const void* work, const uint8_t* freem, void* vals, int vals_fp32, hipStream_t stream);
 /* The same phases with an explicit kernel variant (the two above use the one the
-   tuner below chose for the tangent's precision, else variant 0).  Line-sum variants
-   0-3: the number of segments of a bin line (0: from the grid and the number of
-   compute units, 1: twice, 2: three times as many, 3: the fewest).  Gather variants
-   0, 1, 2: 128, 256 or 512 threads per block row.
+   tuner below chose for the tangent's precision, else variant 0).  Per-bin variants
+   0-3 (particles per group, workgroups per CU, grid): FP32 (8, 2, one per bin),
+   (8, 2, persistent), (4, 4, persistent), (4, 3, persistent); FP64 (4, 2, one per
+   bin), (4, 2, persistent), (8, 1, one per bin), (8, 1, persistent).  Gather
+   variants 0 (per-lane reads of the workspace), 1 and 2 (bin chunks staged in LDS,
+   27 or 9 at a time in FP32, 9 or 3 in FP64).  Line sums: variants 0-3 the number of
+   segments of a bin line (0: from the grid and the number of compute units, 1: twice,
+   2: three times as many, 3: the fewest), gather variants 0, 1, 2: 128, 256 or 512
+   threads per block row.
    Every variant writes the same bits; -1 for a variant out of range. */
 int gm_jacobian_bins_variant(const gm_grid* g, const gm_bins* bins, const void* D, int tangent_fp32, int variant,
                              void* work, size_t work_bytes, hipStream_t stream);

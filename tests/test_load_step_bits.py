@@ -34,3 +34,53 @@ def test_gimp_end_gradients_round_like_the_quotients(n):
         d = x - (lo + k) * h
         ref = -((h + lp) - np.abs(d)) / (2.0 * h * lp) * d / np.abs(d)
         assert np.array_equal(g[:, k][wide], ref[wide]), k
+
+
+def _engine(cells, n, seed, crowd=0):
+    """An engine with random particles on a grid of half-unit cells, `crowd` of them in one cell."""
+    import torch
+    from geowarp_amd.solvers._engine import Engine
+    rng = np.random.default_rng(seed)
+    lp = rng.uniform(0.05, 0.25, (n, 3))
+    x = rng.uniform(0, 1, (n, 3)) * np.array(cells) * 0.5
+    x[:crowd] = 0.6 + 0.02 * rng.random((crowd, 3))
+    x = np.clip(x, lp + 1e-3, np.array(cells) * 0.5 - lp - 1e-3)
+    eng = Engine(3, True, cells, (0.5, 0.5, 0.5))
+    X, LP = (torch.as_tensor(np.ascontiguousarray(a), device=eng.dev) for a in (x, lp))
+    eng.begin_step(X, LP)
+    return eng, X, LP, rng
+
+
+def _binned(eng, D, fp32, vals_fp32=False):
+    """Binned Jacobian for tangent rows D (bin order), the workspace full of NaN before."""
+    import torch
+    from geowarp_amd import _lib as L
+    from geowarp_amd.solvers._engine import _stream
+    lib = L.lib()
+    g, b, pat = L.ctypes.byref(eng.grid), L.ctypes.byref(eng.bins), L.ctypes.byref(eng.pattern)
+    need = int(lib.gm_node_jacobian_work_bytes(g, int(fp32)))
+    w = torch.full((need,), 255, dtype=torch.uint8, device=eng.dev)
+    vals = torch.full((eng.nnzb * 16,), float('nan'), dtype=torch.float32 if vals_fp32 else torch.float64,
+                      device=eng.dev)
+    L.check(lib.gm_node_jacobian_binned(g, b, pat, L.ptr(D), int(fp32), L.ptr(eng.freem), L.ptr(vals),
+                                        int(vals_fp32), L.ptr(w), need, _stream()), 'gm_node_jacobian_binned')
+    return vals
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('cells,n,crowd', [((3, 4, 5), 300, 40), ((20, 5, 4), 3000, 0), ((70, 3, 3), 5000, 30)])
+def test_fp32_jacobian_adds_the_bin_sums_in_fp64(cells, n, crowd):
+    """The mixed form's matrix adds FP32 sums over a bin's particles in FP64: assembled from the bins of
+    even x and from those of odd x (the other particles' tangent zero) the two add up to the whole, to
+    the round-off of 27 FP64 additions."""
+    import torch
+    eng, X, LP, rng = _engine(cells, n, n, crowd)
+    eng.freem.fill_(1)
+    D = torch.as_tensor(rng.standard_normal((n, 255)).astype(np.float32), device=eng.dev)
+    base = torch.repeat_interleave(torch.arange(eng.n_nodes, device=eng.dev),
+                                   (eng.cell_start[1:eng.n_nodes + 1] - eng.cell_start[:eng.n_nodes]).long())
+    even = (base % (cells[0] + 1) % 2 == 0).to(torch.float32)[:, None]
+    whole, a, b = (_binned(eng, (D * m).contiguous(), True) for m in (torch.ones_like(even), even, 1 - even))
+    err = float((whole - (a + b)).abs().max() / whole.abs().max())
+    print(cells, n, 'even + odd bins against all', err)
+    assert float(a.abs().max()) > 0 and float(b.abs().max()) > 0 and err < 1e-14
