@@ -31,7 +31,8 @@
 //   where the gather adds all of them in FP64, which moves the mixed form's Newton iterates
 //   (load steps are held to the last bit, see k_update_lp).  It would be faster on large grids:
 //   2.23 + 1.05 ms against 2.84 + 1.56 with 64 x 64 x 32 cells, 1,048,576 particles (MI355X).
-//   FP64 takes lines: 4.0 + 1.83 ms against 5.6 + 2.9 on that grid.  k_jac_line: the products take 1.3 ms, the stores of the line sums 1.95
+//   FP64 takes lines where they are the faster form (line_sums): 4.0 + 1.83 ms against 5.6 +
+//   2.9 on that grid.  k_jac_line: the products take 1.3 ms, the stores of the line sums 1.95
 //   (7.2 GB), and one follows the other in the product waves; the operand waves' arithmetic
 //   adds 0.2.
 #include <hip/hip_runtime.h>
@@ -1358,8 +1359,14 @@ int best_segments(int nbx, int lines, int n_p, int slots) {
   return best;
 }
 
-// the form of an assembly: FP32 sums per bin, FP64 along lines of bins
-bool line_sums(const gm_grid*, const gm_bins*, int fp32) { return !fp32; }
+// FP64 assemblies take the line sums when there are lines enough for the CUs: from 24,000
+// particles (at some eight a cell) on more than 7000 nodes.  Products and gather against the
+// per-bin form's: 16 x 16 x 8 cells 167 and 146 us, 56 x 6 x 5 161 and 118, 24 x 12 x 8 (18,432
+// particles) 178 and 175, 48 x 9 x 7 (24,192) 238 and 237, 20 x 16 x 10 231 and 255, 9 x 48 x 7 202
+// and 252, 33 x 29 x 15 776 and 1034.
+bool line_sums(const gm_grid* g, const gm_bins* b, int fp32) {
+  return !fp32 && g->n_nodes > 7000 && b->n_particles >= 24000;
+}
 
 int launch_bins(const gm_grid* g, const gm_bins* b, const void* D, int fp32, int variant, void* work,
                 hipStream_t s) {

@@ -84,3 +84,35 @@ def test_fp32_jacobian_adds_the_bin_sums_in_fp64(cells, n, crowd):
     err = float((whole - (a + b)).abs().max() / whole.abs().max())
     print(cells, n, 'even + odd bins against all', err)
     assert float(a.abs().max()) > 0 and float(b.abs().max()) > 0 and err < 1e-14
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('cells,n', [((30, 20, 14), 23999), ((30, 20, 14), 24000), ((24, 19, 13), 25000),
+                                     ((9, 70, 11), 24100), ((130, 8, 6), 30000)])
+def test_fp64_jacobian_either_side_of_the_line_sums(cells, n):
+    """The binned FP64 matrix equals the node-row one to the round-off of a differently ordered sum: with
+    the particles or the nodes just too few for the line sums, and with enough (lines of one segment and
+    of several); all variants write the same bits and every entry."""
+    import torch
+    from geowarp_amd import _lib as L
+    from geowarp_amd.solvers._engine import _stream
+    eng, X, LP, rng = _engine(cells, n, 1, 200)
+    eng.freem.copy_(torch.as_tensor((rng.random(eng.n_nodes * 4) < 0.9).astype(np.uint8), device=eng.dev))
+    D = torch.as_tensor(rng.standard_normal((n, 255)), device=eng.dev)
+    b = _binned(eng, D, False)
+    lib = L.lib()
+    g, bn, pat = L.ctypes.byref(eng.grid), L.ctypes.byref(eng.bins), L.ctypes.byref(eng.pattern)
+    a = torch.empty_like(b)
+    L.check(lib.gm_node_jacobian(g, bn, pat, L.ptr(D), 0, L.ptr(eng.freem), L.ptr(a), 0, 1, _stream()), 'rows')
+    rel = float((a - b).norm() / a.norm())
+    print(cells, n, 'nodes', eng.n_nodes, 'bins against rows', rel)
+    assert rel < 1e-13  # a few hundred terms of 1e-16
+    need = int(lib.gm_node_jacobian_work_bytes(g, 0))
+    w, vals = torch.empty(need, dtype=torch.uint8, device=eng.dev), torch.empty_like(b)
+    for v in range(4):
+        w.fill_(255)
+        vals.fill_(float('nan'))
+        L.check(lib.gm_jacobian_bins_variant(g, bn, L.ptr(D), 0, v, L.ptr(w), need, _stream()), 'bins')
+        L.check(lib.gm_jacobian_gather_variant(g, bn, pat, 0, v % 3, L.ptr(w), L.ptr(eng.freem), L.ptr(vals), 0,
+                                               _stream()), 'gather')
+        assert torch.equal(vals, b), v
