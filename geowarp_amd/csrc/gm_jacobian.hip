@@ -920,22 +920,20 @@ __global__ void __launch_bounds__(T) k_jac_line_gather(gm_grid g, const int* cel
 }
 
 // ================================================================== residual (3D u-p)
-// r_I = sum_p L_I Y_p per bin (node I_loc of the bin's 3x3x3 box), then per node the fixed-order sum over the <= 27 bins holding it.
-// A wave per bin: tables and rows of Y staged in its LDS together, five particles at a time, twelve
-// lanes each: one per (iz, dof) with the sums of its nine (ix, iy) in registers, added over the
-// five at the end.  A bin without particles writes zeros, so that the gather has nothing to look
-// up before its 27 loads.  Bound by the LDS reads (26 a lane for nine sums; a lane per (iy, iz,
-// dof) takes 20 for three and 227 us) and by HBM in the gather.  1,048,576 particles, 139,425
-// nodes: 150 + 45 us (224 + 60 with a lane per node reading Y from memory, and a gather that
-// looked at every bin before its load); 756 bins: 10 us (26).
-constexpr int RES_PB = 10, RES_G = 5;
+// r_I = sum_p L_I Y_p per bin (node I_loc of the bin's 3x3x3 box, its particles in bin order), then
+// per node the fixed-order sum over the <= 27 bins holding it.
+// A wave per bin: tables and rows of Y staged in its LDS together; two lanes a node take two dofs
+// each and walk the particles one after the other (a load step depends on the order, see
+// k_update_lp).  A bin without particles writes zeros, so that the gather has nothing to look up
+// before its 27 loads.  Bound by the LDS reads (18 and 22 a lane and particle).  With the gather,
+// 64 x 64 x 32 cells 222 us, 33 x 29 x 15 33, 12 x 9 x 7 12; with a lane per node reading Y from
+// memory, and a gather that looked at every bin first, 233, 43 and 27; with the particles shared
+// out to five groups of lanes, whose sums are added at the end, 194, 28 and 12, in another order.
+constexpr int RES_PB = 10;
 __global__ void __launch_bounds__(256) k_res_bin(gm_grid g, const double* x_s, const double* lp_s,
                                                  const int* cell_start, const double* Y, double* cb) {
-  __shared__ union {
-    struct {
-      double ax[RES_PB][3][9], y[RES_PB * NY];
-    };
-    double red[RES_G][108];
+  __shared__ struct {
+    double ax[RES_PB][3][9], y[RES_PB * NY];
   } sh[4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.x * 4 + wave;
@@ -946,12 +944,13 @@ __global__ void __launch_bounds__(256) k_res_bin(gm_grid g, const double* x_s, c
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  const int grp = lane / 12, c = lane % 12 & 3, iz = lane % 12 >> 2;
-  // the dof's rows of Y: (b = 0, 1, 2) of P or m, body force or mass balance
-  const int y0 = c < 3 ? c : Y_M, dy = c < 3 ? 3 : 1, yt = c < 3 ? Y_T + c : Y_Q;
-  double r[9];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) r[i] = 0.0;
+  const int node = min(lane >> 1, 26), ix = node % 3, iy = node / 3 % 3, iz = node / 9;
+  const bool odd = lane & 1;  // dofs 0 and 1, or 2 and 3 (the pressure's)
+  const int c = odd ? 2 : 0;
+  // the second dof's terms, in their order: three gradients and the body force, or a gradient, the
+  // mass balance, two gradients and the PPP term
+  const int q0 = odd ? Y_M : 1, q1 = odd ? Y_Q : 4, q2 = odd ? Y_M + 1 : 7, q3 = odd ? Y_M + 2 : Y_T + 1;
+  double r0 = 0.0, r1 = 0.0;
   for (int p0 = ks; p0 < ke; p0 += RES_PB) {
     const int np = min(RES_PB, ke - p0);
     sync();
@@ -972,31 +971,19 @@ __global__ void __launch_bounds__(256) k_res_bin(gm_grid g, const double* x_s, c
       }
     }
     sync();
-    for (int p = grp; p < np && grp < RES_G; p += RES_G) {
+    for (int p = 0; p < np; ++p) {
       const double *X = S_.ax[p][0], *V = S_.ax[p][1], *W = S_.ax[p][2], *yp = S_.y + p * NY;
-      const double wz = W[iz], S = c < 3 ? 0.0 : yp[Y_S];
-      // r = gx (P0 wy wz) + wx (P1 gy wz + wy (P2 gz + T wz)) - wax way (waz S)
-      const double u = yp[y0] * wz, v = yp[y0 + dy] * wz, t = yp[y0 + 2 * dy] * W[3 + iz] + (yp[yt] + S) * wz;
-      const double a = W[6 + iz] * S;
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double uj = V[j] * u, vj = V[3 + j] * v + V[j] * t, aj = V[6 + j] * a;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) r[3 * j + i] += X[3 + i] * uj + X[i] * vj - X[6 + i] * aj;
-      }
+      const double wx = X[ix], wy = V[iy], wz = W[iz], w = wx * wy * wz;
+      const double G0 = X[3 + ix] * wy * wz, G1 = wx * V[3 + iy] * wz, G2 = wx * wy * W[3 + iz];
+      const double wa = X[6 + ix] * V[6 + iy] * W[6 + iz];
+      r0 += fma(w, yp[Y_T + c], fma(G2, yp[6 + c], fma(G1, yp[3 + c], G0 * yp[c])));
+      const double t = fma(odd ? G2 : w, yp[q3], fma(odd ? G1 : G2, yp[q2], fma(odd ? w : G1, yp[q1], G0 * yp[q0])));
+      r1 += odd ? fma(w - wa, yp[Y_S], t) : t;
     }
   }
-  sync();
-  if (grp < RES_G)
-#pragma unroll
-    for (int i = 0; i < 9; ++i) S_.red[grp][(iz * 9 + i) * 4 + c] = r[i];
-  sync();
-#pragma unroll
-  for (int q = lane; q < 108; q += 64) {
-    double s = S_.red[0][q];
-#pragma unroll
-    for (int k = 1; k < RES_G; ++k) s += S_.red[k][q];
-    cb[(long)b * 108 + q] = s;
+  if (lane < 54) {
+    cb[((long)b * 27 + node) * 4 + c] = r0;
+    cb[((long)b * 27 + node) * 4 + c + 1] = r1;
   }
 }
 

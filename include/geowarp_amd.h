@@ -88,7 +88,7 @@ int gm_node_residual(const gm_grid* g, const gm_bins* bins, const double* Y, con
                      int coupled, hipStream_t stream);
 
 /* The same residual for the 3D u-p form (mpm_utils.py:1020-1294) summed per particle
-   bin (the 27 nodes of each bin) into `work` (at least
+   bin (the 27 nodes of each bin, its particles in bin order) into `work` (at least
    gm_residual_work_bytes(g): n_nodes x 108 doubles), then per node over the <= 27 bins
    holding it in a fixed order; masked like gm_node_residual. */
 size_t gm_residual_work_bytes(const gm_grid* g);

@@ -116,3 +116,47 @@ def test_fp64_jacobian_either_side_of_the_line_sums(cells, n):
         L.check(lib.gm_jacobian_gather_variant(g, bn, pat, 0, v % 3, L.ptr(w), L.ptr(eng.freem), L.ptr(vals), 0,
                                                _stream()), 'gather')
         assert torch.equal(vals, b), v
+
+
+def _sum_by_bins(eng, terms, nb, add=lambda acc, t: acc + t):
+    """Nodal sums of per-particle terms (bin order, n x n_nodes x nb): over a bin's particles in their
+    order, then over the bins that hold a node in the order of its place in them (x fastest)."""
+    nx1, ny1 = eng.grid.nx + 1, eng.grid.ny + 1
+    start = eng.cell_start.cpu().numpy()
+    bins = np.zeros((eng.n_nodes, eng.n_nodes, nb))
+    for b in range(eng.n_nodes):
+        for k in range(start[b], start[b + 1]):
+            bins[b] = add(bins[b], terms[k])
+    i = np.arange(eng.n_nodes)
+    c = np.stack([i % nx1, i // nx1 % ny1, i // (nx1 * ny1)], 1)
+    out = np.zeros((eng.n_nodes, nb))
+    for o in range(27):
+        d = np.array([o % 3, o // 3 % 3, o // 9])
+        on = (c >= d).all(1)
+        out[on] += bins[i[on] - d @ np.array([1, nx1, nx1 * ny1]), i[on]]
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('cells,n,crowd', [((3, 3, 3), 1, 0), ((3, 4, 5), 70, 35), ((5, 2, 3), 90, 0)])
+def test_binned_residual_adds_particles_in_bin_order(cells, n, crowd):
+    """The residual of all particles is the sum, in bin order, of what each of them gives alone (its row of Y
+    the only one that is not zero), bit for bit."""
+    import torch
+    eng, X, LP, rng = _engine(cells, n, n + 1, crowd)
+    eng.freem.fill_(1)
+    Y = torch.as_tensor(rng.standard_normal((n, eng.NY)), device=eng.dev)
+
+    def residual(rows):
+        eng.Y.view(-1)[:n * eng.NY].copy_(rows.reshape(-1))
+        eng._bins_workspace(1 << 20).fill_(255)
+        eng.residual(X, LP)
+        return eng.rhs.cpu().numpy().reshape(eng.n_nodes, 4).copy()
+
+    one = torch.zeros_like(Y)
+    terms = []
+    for k in range(n):
+        one.zero_()
+        one[k] = Y[k]
+        terms.append(residual(one))
+    assert np.array_equal(residual(Y), _sum_by_bins(eng, terms, 4))
