@@ -1167,74 +1167,71 @@ extern "C" int gm_mass_binned(const gm_grid* g, const gm_bins* b, const gm_patte
 // w_I m_p p_p sum_J w_J, activation when w_I > threshold inside the particle's support,
 // pressure boundary over all 27 nodes when the node lies at or above a flagged
 // particle); per node, a fixed-order pass over the <= 27 bins holding it.
-// A wave per bin, its particles' weights, right-hand-side factors and flags staged in LDS together;
-// two half waves take every other particle.  Bins without particles write zeros, so that the gather
-// has nothing to look up.  1,048,576 particles, 139,425 nodes: 85 + 35 us (164 + 41 with each lane
-// reading ids, flags and pressures one after the other, and a gather that looked at every bin).
+// Half a wave per bin, its particles' weights, pressures and flags staged in LDS together; a lane a
+// node walks the particles one after the other (a load step depends on the order, see k_update_lp).
+// Bins without particles write zeros, so that the gather has nothing to look up.  P2G with the
+// active mask, 64 x 64 x 32 cells: 92 us; a wave per bin whose halves take every other particle
+// 112, in another order; a wave per bin reading ids, flags and pressures one after the other, and a
+// gather that looked at every bin, 183.
 __global__ void __launch_bounds__(256) k_p2g_bin(gm_grid g, const double* x_s, const double* lp_s,
                                                  const int* cell_start, const int* sorted, const uint8_t* ext_s,
                                                  double threshold, const uint8_t* pbc_flag, double node_h_last,
                                                  double p_mass, const double* p_part, double* cb, uint8_t* cf) {
-  constexpr int PB = 16;
+  constexpr int PB = 10;
   __shared__ struct {
-    double w[PB][3][3], m[PB], z[PB];
+    double w[PB][3][3], sum[PB], pr[PB], z[PB];
     uint8_t ext[PB];
-  } sh[4];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b = blockIdx.x * 4 + wave;
-  if (b >= g.n_nodes) return;  // the whole wave
-  auto& S = sh[wave];
-  const int ks = cell_start[b], ke = cell_start[b + 1];
+  } sh[8];
+  const int t = threadIdx.x & 31, half = threadIdx.x >> 5;
+  const int b = blockIdx.x * 8 + half;
+  auto& S = sh[half];
+  const int ks = b < g.n_nodes ? cell_start[b] : 0, n = b < g.n_nodes ? cell_start[b + 1] - ks : 0;
   auto sync = [] {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  const int t = lane & 31, half = lane >> 5;
   const int ox = t % 3, oy = (t / 3) % 3, oz = min(t / 9, 2);  // lanes 27 to 31 of a half: not stored
   const int nxy = (g.nx + 1) * (g.ny + 1);
   const double node_z = (double)(b / nxy + oz) * node_h_last;
   double rhs = 0.0;
   int on = 0;  // 1: active, 2: pressure boundary
-  for (int p0 = ks; p0 < ke; p0 += PB) {
-    const int np = min(PB, ke - p0);
+  const int most = max(n, __shfl_xor(n, 32, 64));  // the same rounds for both halves
+  for (int i0 = 0; i0 < most; i0 += PB) {
+    const int np = min(PB, n - i0), p0 = ks + i0;  // (np <= 0: this half is through)
     sync();
-    double z = INFINITY, pm = 0.0;  // height of a flagged particle, m_p p_p
-    if (lane < np) {
-      const int k = p0 + lane, pid = sorted[k];
-      if (pbc_flag && pbc_flag[pid]) z = x_s[(long)k * 3 + 2];
-      if (p_part) pm = p_mass * p_part[pid];
-      S.ext[lane] = ext_s[k];
-      S.z[lane] = z;
+    if (t < np) {
+      const int k = p0 + t, pid = sorted[k];
+      S.z[t] = pbc_flag && pbc_flag[pid] ? x_s[(long)k * 3 + 2] : INFINITY;  // height of a flagged particle
+      S.pr[t] = p_part ? p_part[pid] : 0.0;
+      S.ext[t] = ext_s[k];
     }
-    if (lane < 3 * np) {
-      const int a = lane % 3;
-      const Axis ax = gimp_axis(x_s[(long)p0 * 3 + lane], lp_s[(long)p0 * 3 + lane], g.h[a], g.inv_h[a]);
+    if (t < 3 * np) {
+      const int a = t % 3;
+      const Axis ax = gimp_axis(x_s[(long)p0 * 3 + t], lp_s[(long)p0 * 3 + t], g.h[a], g.inv_h[a]);
 #pragma unroll
-      for (int i = 0; i < 3; ++i) S.w[lane / 3][a][i] = ax.w[i];
+      for (int i = 0; i < 3; ++i) S.w[t / 3][a][i] = ax.w[i];
     }
     sync();
-    if (lane < np) {
-      double wsum = 1.0;
+    if (t < np) {
+      double sum = 1.0;
 #pragma unroll
-      for (int a = 0; a < 3; ++a) wsum *= S.w[lane][a][0] + S.w[lane][a][1] + S.w[lane][a][2];
-      S.m[lane] = wsum * pm;
+      for (int a = 0; a < 3; ++a) sum *= S.w[t][a][0] + S.w[t][a][1] + S.w[t][a][2];
+      S.sum[t] = sum;
     }
     sync();
-    for (int p = half; p < np; p += 2) {
+    for (int p = 0; p < np; ++p) {
       if (node_z >= S.z[p]) on |= 2;
       const uint8_t ex = S.ext[p];
       const bool in = ox < ((ex & 1) ? 3 : 2) && oy < ((ex & 2) ? 3 : 2) && oz < ((ex & 4) ? 3 : 2);
       if (!in) continue;
       const double w = S.w[p][0][ox] * S.w[p][1][oy] * S.w[p][2][oz];
       if (threshold < 0.0 || w > threshold) on |= 1;
-      if (p_part) rhs += w * S.m[p];
+      if (p_part) rhs = fma(w * S.sum[p] * p_mass, S.pr[p], rhs);
     }
   }
-  rhs += __shfl_xor(rhs, 32, 64);
-  on |= __shfl_xor(on, 32, 64);
-  if (lane < 27) {
-    cb[(long)b * 27 + lane] = rhs;
-    cf[(long)b * 27 + lane] = (uint8_t)on;
+  if (t < 27 && b < g.n_nodes) {
+    cb[(long)b * 27 + t] = rhs;
+    cf[(long)b * 27 + t] = (uint8_t)on;
   }
 }
 
@@ -1283,7 +1280,7 @@ extern "C" int gm_p2g_binned(const gm_grid* g, const gm_bins* b, double threshol
   if (n == 0) return 0;
   double* cb = (double*)work;
   uint8_t* cf = (uint8_t*)(cb + (size_t)n * 27);
-  k_p2g_bin<<<gm_blocks(n, 4), 256, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold, pbc_flag,
+  k_p2g_bin<<<gm_blocks(n, 8), 256, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->sorted, b->ext_s, threshold, pbc_flag,
                              node_h_last, p_mass, mrhs ? p_part : nullptr, cb, cf);
   GM_LAUNCH_CHECK();
   k_p2g_gather<<<gm_blocks(n, 256), 256, 0, s>>>(*g, cb, cf, act, bflag, mrhs);

@@ -160,3 +160,28 @@ def test_binned_residual_adds_particles_in_bin_order(cells, n, crowd):
         one[k] = Y[k]
         terms.append(residual(one))
     assert np.array_equal(residual(Y), _sum_by_bins(eng, terms, 4))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('cells,n,crowd', [((3, 3, 3), 1, 0), ((3, 4, 5), 70, 35), ((5, 2, 3), 90, 0)])
+def test_binned_p2g_adds_particles_in_bin_order(cells, n, crowd):
+    """The mass projection's right-hand side: w_I m sum_J w_J (a particle alone, of unit pressure) times the
+    particle's pressure, added with one rounding, in bin order, then the bins in theirs; bit for bit."""
+    from fractions import Fraction
+    import torch
+    eng, X, LP, rng = _engine(cells, n, n + 2, crowd)
+    order = eng.sorted[:n].long()
+    p = torch.as_tensor(rng.standard_normal(n), device=eng.dev)
+
+    def rhs(pp):
+        eng._bins_workspace(1 << 20).fill_(255)
+        return eng.p2g(X, LP, 0.0, None, 0.5, 0.37, pp, mass=True).cpu().numpy().copy()
+
+    one = torch.zeros_like(p)
+    terms = []
+    for k in range(n):
+        one.zero_()
+        one[order[k]] = 1.0
+        terms.append((rhs(one)[:, None], float(p[order[k]])))
+    fma = np.vectorize(lambda a, b, c: float(Fraction(a) * Fraction(b) + Fraction(c)) if a else c)
+    assert np.array_equal(rhs(p), _sum_by_bins(eng, terms, 1, lambda acc, t: fma(t[0], t[1], acc))[:, 0])
