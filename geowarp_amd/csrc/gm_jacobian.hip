@@ -1032,8 +1032,7 @@ extern "C" int gm_node_residual_binned(const gm_grid* g, const gm_bins* b, const
 // registers.  A stencil line's candidates lie in consecutive bins, so their weights are one range
 // of particles, staged C at a time: weight-major, and particles eight apart next to each other, so
 // that the rows of a wave read different banks.  The waves' sums are added in LDS in order.
-// Bound by those LDS reads (8 a particle and lane in 3D).  1,048,576 particles, 139,425 rows:
-// 414 us, against 1110 for products per bin, stored (764 MB) and summed over 27 bins;
+// Bound by those LDS reads (8 a particle and lane in 3D).  1,048,576 particles, 139,425 rows: 414 us;
 // 11,628 2D rows: 12 us, against 110 for a thread a row adding to its entries in memory.  Pieces of
 // 64, 128 and 192 particles: 510, 478 and 493 us (what a lane waits for its bins in longer ranges
 // against the wavefronts their LDS leaves); strips of 10 rows with two lanes for a bin's particles: 403.
@@ -1135,7 +1134,7 @@ __global__ void __launch_bounds__(192) k_mass_strip(gm_grid g, const double* x_s
   }
 }
 
-// the consistent mass of a grid's pattern (declared in gm_common.h; gm_p2g uses it as well)
+// the consistent mass of a grid's pattern (declared in gm_common.h; for gm_p2g)
 void gm::launch_mass(const gm_grid& g, const gm_bins& b, const gm_pattern& pat, double p_mass, double* mvals,
                      hipStream_t s) {
   const int blocks = gm_blocks(g.n_nodes, MASS_ROWS);
@@ -1145,8 +1144,91 @@ void gm::launch_mass(const gm_grid& g, const gm_bins& b, const gm_pattern& pat, 
     k_mass_strip<2><<<blocks, 192, 0, s>>>(g, b.x_s, b.lp_s, b.cell_start, p_mass, pat.row_ptr, pat.row_mask, mvals);
 }
 
-// (the workspace is not used any more; callers keep passing the bytes asked for)
-extern "C" size_t gm_mass_work_bytes(const gm_grid* g) { return g ? sizeof(double) : 0; }
+// ------------------------------------------------------------------ consistent mass per bin (3D)
+// The same matrix in the order that the 3D u-p step depends on (see k_update_lp): per bin the 27 x 27
+// products of its particles, in bin order, then per row the fixed-order sum over the bins holding
+// both nodes.  The products are formed from a table of the particles' 27 node weights.  With the
+// right-hand side, 64 x 64 x 32 cells 890 us, 33 x 29 x 15 82, 12 x 9 x 7 20; the strips 410, 101 and
+// 59; products from the axis weights 1140, 122 and 28.
+__global__ void __launch_bounds__(256) k_mass_bin(gm_grid g, const double* x_s, const double* lp_s,
+                                                  const int* cell_start, double p_mass, double* cb) {
+  constexpr int PB = 32;
+  __shared__ double A[PB][3][3], W[PB][27];
+  const int b = blockIdx.x;
+  const int ks = cell_start[b], ke = cell_start[b + 1];
+  if (ks == ke) return;  // uniform across the workgroup
+  const int t = threadIdx.x;
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (int p0 = ks; p0 < ke; p0 += PB) {
+    const int np = min(PB, ke - p0);
+    __syncthreads();
+    if (t < 3 * np) {
+      const int a = t % 3;
+      const Axis ax = gimp_axis(x_s[(long)p0 * 3 + t], lp_s[(long)p0 * 3 + t], g.h[a], g.inv_h[a]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) A[t / 3][a][i] = ax.w[i];
+    }
+    __syncthreads();
+    for (int q = t; q < 27 * np; q += 256) {
+      const int p = q / 27, i = q % 27;
+      W[p][i] = A[p][0][i % 3] * A[p][1][i / 3 % 3] * A[p][2][i / 9];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int q = min(t + 256 * j, 728), I = q / 27, J = q % 27;
+      for (int p = 0; p < np; ++p) acc[j] = fma(W[p][I] * W[p][J], p_mass, acc[j]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    if (t + 256 * j < 729) cb[(long)b * 729 + t + 256 * j] = acc[j];
+}
+
+__global__ void __launch_bounds__(128) k_mass_gather(gm_grid g, const int* cell_start, const double* cb,
+                                                     const int* row_ptr, const uint64_t* row_mask, double* mvals) {
+  __shared__ int SLOT_BIT[125];
+  __shared__ int BIN[27];
+  const int I = blockIdx.x, t = threadIdx.x;
+  const uint64_t m0 = row_mask[2 * I], m1 = row_mask[2 * I + 1];
+  const int nx1 = g.nx + 1, nxy = (g.nx + 1) * (g.ny + 1);
+  const int ci[3] = {I % nx1, (I / nx1) % (g.ny + 1), I / nxy};
+  if (t < 125) {
+    const uint64_t w = (t < 64) ? m0 : m1;
+    const int sh = t & 63;
+    if ((w >> sh) & 1ull) {
+      const int below = (t < 64) ? __popcll(m0 & ((1ull << sh) - 1ull))
+                                 : __popcll(m0) + __popcll(m1 & ((1ull << sh) - 1ull));
+      SLOT_BIT[below] = t;
+    }
+  }
+  if (t < 27) {
+    const int ox = t % 3, oy = (t / 3) % 3, oz = t / 9;
+    const int bc[3] = {ci[0] - ox, ci[1] - oy, ci[2] - oz};
+    int bn = -1;
+    if (bc[0] >= 0 && bc[0] <= g.nx && bc[1] >= 0 && bc[1] <= g.ny && bc[2] >= 0 && bc[2] <= g.nz) {
+      bn = bc[0] + bc[1] * nx1 + bc[2] * nxy;
+      if (cell_start[bn + 1] == cell_start[bn]) bn = -1;
+    }
+    BIN[t] = bn;
+  }
+  __syncthreads();
+  const int nnz = __popcll(m0) + __popcll(m1);
+  if (t >= nnz) return;
+  const int bit = SLOT_BIT[t];
+  const int d[3] = {bit % 5 - 2, (bit / 5) % 5 - 2, bit / 25 - 2};
+  double s = 0.0;
+#pragma unroll
+  for (int o = 0; o < 27; ++o) {
+    const int kx = d[0] + o % 3, ky = d[1] + (o / 3) % 3, kz = d[2] + o / 9;
+    const int bn = BIN[o];
+    if (bn >= 0 && kx >= 0 && kx < 3 && ky >= 0 && ky < 3 && kz >= 0 && kz < 3)
+      s += cb[(long)bn * 729 + o * 27 + (kx + 3 * ky + 9 * kz)];
+  }
+  mvals[row_ptr[I] + t] = s;
+}
+
+extern "C" size_t gm_mass_work_bytes(const gm_grid* g) { return g ? (size_t)g->n_nodes * 729 * sizeof(double) : 0; }
 
 extern "C" int gm_mass_binned(const gm_grid* g, const gm_bins* b, const gm_pattern* pat, double p_mass,
                               double* mvals, void* work, size_t work_bytes, hipStream_t s) {
@@ -1155,7 +1237,9 @@ extern "C" int gm_mass_binned(const gm_grid* g, const gm_bins* b, const gm_patte
   GM_REQUIRE(work_bytes >= gm_mass_work_bytes(g), "gm_mass_binned: workspace smaller than gm_mass_work_bytes");
   const int n = g->n_nodes;
   if (n == 0) return 0;
-  gm::launch_mass(*g, *b, *pat, p_mass, mvals, s);
+  k_mass_bin<<<n, 256, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, p_mass, (double*)work);
+  GM_LAUNCH_CHECK();
+  k_mass_gather<<<n, 128, 0, s>>>(*g, b->cell_start, (const double*)work, pat->row_ptr, pat->row_mask, mvals);
   GM_LAUNCH_CHECK();
   return 0;
 }

@@ -159,9 +159,9 @@ int gm_stage_de_3d(int n, const int* sorted, const double* F_old, const double* 
                 const double* pen_force, const double* Y, double p_vol, double E, double* dY, hipStream_t stream);
 
 /* 3D consistent-mass matrix M_IJ = sum_p m w_I w_J (mpm_utils.py:327-383) in the
-   pattern, gathered by strips of node rows in a fixed order (as gm_p2g does with mvals);
-   gm_p2g_binned then fills the activation flags and the right-hand side.  `work`: at least
-   gm_mass_work_bytes(g) bytes, which no kernel uses any more. */
+   pattern, assembled per particle bin into `work` (at least gm_mass_work_bytes(g):
+   n_nodes x 729 doubles) and gathered per row in a fixed order; gm_p2g then
+   leaves mvals null and fills only the activation flags and the right-hand side. */
 size_t gm_mass_work_bytes(const gm_grid* g);
 int gm_mass_binned(const gm_grid* g, const gm_bins* bins, const gm_pattern* pat, double p_mass, double* mvals,
                    void* work, size_t work_bytes, hipStream_t stream);

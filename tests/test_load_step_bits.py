@@ -185,3 +185,38 @@ def test_binned_p2g_adds_particles_in_bin_order(cells, n, crowd):
         terms.append((rhs(one)[:, None], float(p[order[k]])))
     fma = np.vectorize(lambda a, b, c: float(Fraction(a) * Fraction(b) + Fraction(c)) if a else c)
     assert np.array_equal(rhs(p), _sum_by_bins(eng, terms, 1, lambda acc, t: fma(t[0], t[1], acc))[:, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('cells,n,crowd', [((3, 3, 3), 1, 0), ((3, 4, 4), 50, 40), ((4, 2, 3), 60, 0)])
+def test_binned_mass_adds_particles_in_bin_order(cells, n, crowd):
+    """The consistent mass (particle mass a power of two) is the sum, in bin order and then over the bins in
+    theirs, of what each particle gives alone, bit for bit."""
+    import torch
+    from geowarp_amd import _lib
+    from geowarp_amd.solvers._engine import Engine, _stream
+    eng, X, LP, rng = _engine(cells, n, n + 3, crowd)
+
+    def mass(e, x, lp):
+        if e.mvals is not None:
+            e.mvals.fill_(float('nan'))
+        e._bins_workspace(1 << 20).fill_(255)
+        e.p2g(x, lp, 0.0, None, 0.5, 0.5, torch.zeros(len(x), dtype=torch.float64, device=e.dev), mass=True)
+        rp, ci = e.row_ptr[:e.n_nodes + 1].cpu().numpy(), e.col_idx[:e.nnzb].cpu().numpy()
+        M = np.zeros((e.n_nodes, e.n_nodes))
+        M[np.repeat(np.arange(e.n_nodes), np.diff(rp)), ci] = e.mvals[:e.nnzb].cpu().numpy()
+        return M
+
+    terms = []
+    for k in eng.sorted[:n].tolist():
+        one = Engine(3, True, cells, (0.5, 0.5, 0.5))
+        one.begin_step(X[k:k + 1].contiguous(), LP[k:k + 1].contiguous())
+        terms.append(mass(one, X[k:k + 1].contiguous(), LP[k:k + 1].contiguous()))
+    assert np.array_equal(mass(eng, X, LP), _sum_by_bins(eng, terms, eng.n_nodes))
+    # gm_p2g's own mass (strips of rows) sums the same terms in another order
+    L, lib = _lib, _lib.lib()
+    vals = torch.full_like(eng.mvals[:eng.nnzb], float('nan'))
+    L.check(lib.gm_p2g(L.ctypes.byref(eng.grid), L.ctypes.byref(eng.bins), L.ctypes.byref(eng.pattern), 0.0, None, 0.5,
+                       0.5, None, L.ptr(eng.act), L.ptr(eng.bflag), L.ptr(vals), None, _stream()), 'gm_p2g')
+    err = float((vals - eng.mvals[:eng.nnzb]).abs().max() / vals.abs().max())
+    assert err < 1e-14, err
