@@ -40,7 +40,8 @@ struct Window {
   __device__ __forceinline__ int offset(int k) const { return k % 5 - 2 + (k / 5 % 5 - 2) * nx1 + (k / 25 - 2) * nxy; }
 };
 
-template <int NB, int G, typename TM, typename TX, typename TY, int T = SPMV_T>
+// GRID: scalar rows with a window (an instance of its own: its registers cost the other products)
+template <int NB, int G, typename TM, typename TX, typename TY, int T = SPMV_T, bool GRID = false>
 __global__ void __launch_bounds__(T) k_spmv(int n_rows, const int* row_ptr, const int* col_idx, const TM* vals,
                                             const TX* x, TY* y, const TY* w1, const TY* w2, double* part,
                                             const double* gate, Window win) {
@@ -58,6 +59,25 @@ __global__ void __launch_bounds__(T) k_spmv(int n_rows, const int* row_ptr, cons
     // one-entry-at-a-time order
     const int s = row_ptr[row], e = row_ptr[row + 1];
     int k = s + lane;
+    if (GRID && win.full(row)) {
+      // (125 entries: the last step of four is cut short by the lane's count)
+      constexpr int N = (125 + G - 1) / G;
+#pragma unroll
+      for (int u0 = 0; u0 < N; u0 += 4) {
+        TM v[4];
+        double xv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int q = min(lane + (u0 + u) * G, 124);
+          v[u] = vals[s + q];
+          xv[u] = (double)x[row + win.offset(q)];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (lane + (u0 + u) * G < 125) acc[0] = fma((double)v[u], xv[u], acc[0]);
+      }
+      k = e;
+    }
     for (; k + 3 * G < e; k += 4 * G) {
       int c[4];
       TM v[4];
@@ -138,6 +158,12 @@ static void launch_spmv(int n_rows, const int* rp, const int* ci, const TM* v, c
                         const TY* w2, double* part, hipStream_t s, int threads = 0,
                         const double* gate = nullptr, const Window& win = Window{nullptr, 0, 0}) {
   const int G = spmv_lanes(NB);
+  if constexpr (NB == 1)
+    if (win.mask) {
+      k_spmv<NB, G, TM, TX, TY, SPMV_T, true><<<gm_blocks(n_rows, SPMV_T / G), SPMV_T, 0, s>>>(
+          n_rows, rp, ci, v, x, y, w1, w2, part, gate, win);
+      return;
+    }
   int t = part ? SPMV_T : (threads ? threads : g_spmv_threads[NB][sizeof(TM) == 4 ? 1 : 0]);
   switch (t) {
     case 64:
@@ -934,18 +960,18 @@ __global__ void __launch_bounds__(PCG_WIDE) k_pcg_alpha(const double* part, int 
 }
 
 // x += alpha p, r -= alpha q, z = Dinv r; per-workgroup partials of r.z and r.r.
-// pq_parts > 0: alpha is formed here, by every workgroup, from that many partial sums of p.q
-// (pq), with the rules of k_pcg_alpha; workgroup 0 stores it.
-template <int NB, typename TM, typename TV>
+// ALPHA: alpha is formed here, by every workgroup, from pq_parts partial sums of p.q (pq), with the
+// rules of k_pcg_alpha; workgroup 0 stores it.
+template <int NB, typename TM, typename TV, bool ALPHA>
 __global__ void __launch_bounds__(RED_T) k_pcg_xr(int n_rows, const double* pq, int pq_parts, double* sc, TV* x, TV* r,
                                                   const TV* p, const TV* q, const TM* dinv, TV* z, double* part) {
   __shared__ double a[RED_T], c[RED_T];
   if (sc[C_DONE] != 0.0) {
-    if (pq_parts && blockIdx.x == 0 && threadIdx.x == 0) sc[C_GATE] = 1.0;
+    if (ALPHA && blockIdx.x == 0 && threadIdx.x == 0) sc[C_GATE] = 1.0;
     return;
   }
   double alpha;
-  if (pq_parts) {
+  if constexpr (ALPHA) {
     double u = 0.0;
     for (int i = threadIdx.x; i < pq_parts; i += RED_T) u += pq[i];
     u = block_sum(u, a);
@@ -1016,20 +1042,18 @@ __global__ void __launch_bounds__(RED_T) k_pcg_p(long n, const double* part, int
     p[i] = (TV)((double)z[i] + beta * (double)p[i]);
 }
 
-// y = A x of a scalar matrix in a grid's window pattern (at most 5^DIM entries a row, in window
+// y = A x of a scalar matrix in a 2D grid's window pattern (at most 25 entries a row, in window
 // order), and the workgroups' partial sums of x.y.  The columns of a full row follow from its
 // number, so col_idx is read only for the rows the boundary cuts and no load of x waits for one.
-// G lanes a row, its entries and x loaded together.  Bound by HBM: 139,425 rows of 125 take 33 us
-// for 139 MB, 36 us with the columns read.  A workgroup takes several steps of rows so that p.q
-// comes as 1024 partial sums, few enough for every workgroup of the update to add up: a launch
-// (k_pcg_alpha, 4.6 us) less an iteration.  One step a workgroup: 31 us, but 16 for the update
-// (16 -> 6.5).  The next rows' entries loaded a step ahead: 49 us, for the registers they take.
+// Eight lanes a row, its entries and x loaded together.  A workgroup takes several steps of rows so
+// that p.q comes as 1024 partial sums, few enough for every workgroup of the update to add up: a
+// launch (k_pcg_alpha, 4.6 us) less an iteration.  18,943 rows, 48 iterations: the projection 1.42 ->
+// 1.34 ms.  (3D keeps the launches and the order of sums of gm_pcg, see k_update_lp.)
 constexpr int WIN_T = 512, WIN_BLOCKS = 1024;
-template <int DIM>
-__global__ void __launch_bounds__(WIN_T) k_window_mv(int n_rows, int nx1, int nxy, const int* rp, const int* ci,
+__global__ void __launch_bounds__(WIN_T) k_window_mv(int n_rows, int nx1, const int* rp, const int* ci,
                                                      const double* vals, const double* x, double* y, double* part,
                                                      const double* gate) {
-  constexpr int W = DIM == 3 ? 125 : 25, G = DIM == 3 ? 16 : 8, U = (W + G - 1) / G;
+  constexpr int W = 25, G = 8, U = (W + G - 1) / G;
   __shared__ double sh[WIN_T / 64];
   if (gate && *gate != 0.0) return;  // a gated launch after its solve has converged
   const int lane = threadIdx.x % G;
@@ -1037,7 +1061,7 @@ __global__ void __launch_bounds__(WIN_T) k_window_mv(int n_rows, int nx1, int nx
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int k = min(lane + G * u, W - 1);
-    off[u] = k % 5 - 2 + (k / 5 % 5 - 2) * nx1 + (DIM == 3 ? (k / 25 - 2) * nxy : 0);
+    off[u] = k % 5 - 2 + (k / 5 - 2) * nx1;
   }
   double d = 0.0;
   for (int row = blockIdx.x * (WIN_T / G) + threadIdx.x / G; row < n_rows; row += gridDim.x * (WIN_T / G)) {
@@ -1090,7 +1114,7 @@ __global__ void k_rowsum_inv(int n_rows, const int* rp, const TM* vals, TM* dinv
 template <int NB, typename TM, typename TV>
 static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, const TV* b, TV* x, gm_krylov_ws* ws,
                     double tol, int maxiter, int check_every, int options, int* iters_out, double* relres_out,
-                    hipStream_t st, const gm_grid* window = nullptr) {
+                    hipStream_t st, const gm_grid* window = nullptr, const Window& win = Window{nullptr, 0, 0}) {
   const bool lumped = options & 1, warm = options & 2;
   long n = (long)n_rows * NB;
   TV *r = (TV*)ws->r, *p = (TV*)ws->p, *q = (TV*)ws->v, *z = (TV*)ws->z;
@@ -1098,24 +1122,20 @@ static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, co
   double* sc = ws->sc;
   double* part = ws->part;
   const int rb = gm_blocks(n_rows, 256);
-  // window: the pattern is the grid's; p.q comes as WIN_BLOCKS partial sums at most and the
+  // window: the pattern is the 2D grid's; p.q comes as WIN_BLOCKS partial sums at most and the
   // update forms alpha itself, its own partial pairs behind them (workspace: 2048 values)
   const int db = std::min(window ? 512 : 1024, gm_blocks(n_rows, RED_T));
   const int sb = spmv_blocks(n_rows, NB);
-  const int wb = std::min(WIN_BLOCKS, gm_blocks(n_rows, WIN_T / (window && window->dim == 3 ? 16 : 8)));
+  const int wb = std::min(WIN_BLOCKS, gm_blocks(n_rows, WIN_T / 8));
   double* xpart = window ? part + WIN_BLOCKS : part;
   auto mv = [&](const TV* in, TV* out, double* pq, const double* gate) {
     if constexpr (NB == 1 && sizeof(TM) == 8 && sizeof(TV) == 8) {
       if (window) {
-        const int nx1 = window->nx + 1, nxy = nx1 * (window->ny + 1);
-        if (window->dim == 3)
-          k_window_mv<3><<<wb, WIN_T, 0, st>>>(n_rows, nx1, nxy, rp, ci, vals, in, out, pq, gate);
-        else
-          k_window_mv<2><<<wb, WIN_T, 0, st>>>(n_rows, nx1, nxy, rp, ci, vals, in, out, pq, gate);
+        k_window_mv<<<wb, WIN_T, 0, st>>>(n_rows, window->nx + 1, rp, ci, vals, in, out, pq, gate);
         return;
       }
     }
-    launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, in, out, pq ? in : nullptr, nullptr, pq, st, 0, gate);
+    launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, in, out, pq ? in : nullptr, nullptr, pq, st, 0, gate, win);
   };
   if (NB == 1 && lumped)
     k_rowsum_inv<TM><<<rb, 256, 0, st>>>(n_rows, rp, vals, dinv);
@@ -1150,8 +1170,12 @@ static int pcg_impl(int n_rows, const int* rp, const int* ci, const TM* vals, co
     const int nrun = std::min(check_every, maxiter - it);
     for (int k = 0; k < nrun; ++k) {
       mv(p, q, part, sc + C_DONE);
-      if (!window) k_pcg_alpha<<<1, PCG_WIDE, 0, st>>>(part, sb, sc);
-      k_pcg_xr<NB, TM, TV><<<db, RED_T, 0, st>>>(n_rows, part, window ? wb : 0, sc, x, r, p, q, dinv, z, xpart);
+      if (window) {
+        k_pcg_xr<NB, TM, TV, true><<<db, RED_T, 0, st>>>(n_rows, part, wb, sc, x, r, p, q, dinv, z, xpart);
+      } else {
+        k_pcg_alpha<<<1, PCG_WIDE, 0, st>>>(part, sb, sc);
+        k_pcg_xr<NB, TM, TV, false><<<db, RED_T, 0, st>>>(n_rows, nullptr, 0, sc, x, r, p, q, dinv, z, xpart);
+      }
       k_pcg_p<TV><<<gm_blocks(n, RED_T), RED_T, 0, st>>>(n, xpart, db, sc, z, p, thr2);
     }
     GM_LAUNCH_CHECK();
@@ -1203,8 +1227,13 @@ extern "C" int gm_pcg_window(const gm_grid* g, const gm_pattern* pat, const doub
   GM_REQUIRE(g->dim == 2 || g->dim == 3, "gm_pcg_window: dim must be 2 or 3");
   GM_REQUIRE((long)(g->nx + 1) * (g->ny + 1) * (g->dim == 3 ? g->nz + 1 : 1) == g->n_nodes,
              "gm_pcg_window: n_nodes does not match the grid");
+  // 3D: columns of full rows from the grid where the product is long enough to be bound by memory
+  // (the projection with 171,396 rows 4.17 -> 3.75 ms, 48,600 2.15 -> 2.03; 24,548 1.65 -> 1.76)
+  const int nx1 = g->nx + 1;
+  const Window win{g->dim == 3 && g->n_nodes > 32768 ? pat->row_mask : nullptr, nx1, nx1 * (g->ny + 1)};
   return pcg_impl<1, double, double>(g->n_nodes, pat->row_ptr, pat->col_idx, vals, b, x, ws, tol, maxiter,
-                                     check_every < 1 ? 1 : check_every, options, iters, relres, s, g);
+                                     check_every < 1 ? 1 : check_every, options, iters, relres, s,
+                                     g->dim == 2 ? g : nullptr, win);
 }
 
 // y = A x  (A in FP64 or FP32, x and y in FP64 or FP32; FP64 accumulation)

@@ -243,8 +243,9 @@ int gm_pcg(int nb, int fp32, int n_rows, const int* row_ptr, const int* col_idx,
            double* relres, hipStream_t stream);
 
 /* gm_pcg (nb = 1, FP64) for a matrix in the grid's own node pattern, as gm_p2g and
-   gm_p2g_binned write the consistent mass: the columns of the rows whose window is complete
-   follow from the grid, so only the others' are read, and an iteration takes three launches. */
+   gm_mass_binned write the consistent mass: the columns of the rows whose window is complete
+   follow from the grid, so only the others' are read.  3D: the same bits as gm_pcg; 2D: sums in
+   another order, and three launches an iteration. */
 int gm_pcg_window(const gm_grid* g, const gm_pattern* pat, const double* vals, const double* b, double* x,
                   gm_krylov_ws* ws, double tol, int maxiter, int check_every, int options, int* iters, double* relres,
                   hipStream_t stream);

@@ -220,3 +220,31 @@ def test_binned_mass_adds_particles_in_bin_order(cells, n, crowd):
                        0.5, None, L.ptr(eng.act), L.ptr(eng.bflag), L.ptr(vals), None, _stream()), 'gm_p2g')
     err = float((vals - eng.mvals[:eng.nnzb]).abs().max() / vals.abs().max())
     assert err < 1e-14, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('options', [0, 3])
+@pytest.mark.parametrize('cells', [(2, 3, 2), (4, 4, 4), (13, 9, 11), (41, 30, 28)])
+def test_mass_cg_sums_as_the_general_cg(cells, options):
+    """gm_pcg_window in 3D, which takes the columns of complete rows from the grid, gives the bits of gm_pcg."""
+    import torch
+    from geowarp_amd import _lib as L
+    from geowarp_amd.solvers._engine import _stream
+    eng, X, LP, rng = _engine(cells, 8 * int(np.prod(cells)), 5)
+    n, lib = eng.n_nodes, L.lib()
+    p = torch.as_tensor(rng.standard_normal(len(X)), device=eng.dev)
+    b = eng.p2g(X, LP, 0.0, None, 0.5, 0.7, p, mass=True)
+    L.check(lib.gm_fix_empty_diag(n, L.ptr(eng.row_ptr), L.ptr(eng.col_idx), L.ptr(eng.mvals), L.ptr(b), _stream()),
+            'gm_fix_empty_diag')
+    ws, out = eng.workspace(1, False), []
+    for window in (False, True):
+        it, rr, x = L.c_int(0), L.c_double(0.0), torch.full_like(b, 0.1)
+        tail = (L.ptr(eng.mvals), L.ptr(b), L.ptr(x), L.ctypes.byref(ws), 1e-10, 4000, 16, options,
+                L.ctypes.byref(it), L.ctypes.byref(rr), _stream())
+        if window:
+            L.check(lib.gm_pcg_window(L.ctypes.byref(eng.grid), L.ctypes.byref(eng.pattern), *tail), 'window')
+        else:
+            L.check(lib.gm_pcg(1, 0, n, L.ptr(eng.row_ptr), L.ptr(eng.col_idx), *tail), 'general')
+        out.append((x, it.value, rr.value))
+    print(cells, options, out[0][1:], out[1][1:])
+    assert torch.equal(out[0][0], out[1][0]) and out[0][1:] == out[1][1:]
