@@ -448,16 +448,17 @@ static void launch_lo_convert(int n_rows, const int* rp, const TM* vals, gm_half
 static int spmv_blocks(int n_rows, int nb) { return gm_blocks(n_rows, SPMV_T / spmv_lanes(nb)); }
 
 // ------------------------------------------------------------------ reductions
-// sum over the workgroup (RED_T threads) in a fixed order; every thread gets it
+// sum over the workgroup (RED_T threads) in the order of the trees below (halves onto each other);
+// every thread gets it
 __device__ __forceinline__ double block_sum(double s, double* sh) {
+  static_assert(RED_T == 256, "four waves");
+  __syncthreads();
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  const int l = threadIdx.x & 63;
+  s = (sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  s = sh[0];
-#pragma unroll
-  for (int i = 1; i < RED_T / 64; ++i) s += sh[i];
   return s;
 }
 
@@ -1381,67 +1382,85 @@ extern "C" int gm_fix_empty_diag(int n_rows, const int* row_ptr, const int* col_
 // is solved on the host, which reads one column of H per iteration.
 // x <- x + M^{-1} V y at the end of every cycle; restart from r = b - A x.
 
-// Gram-Schmidt of one Arnoldi step in five to seven launches (k_gs_dots, [k_gs_fin,] k_gs_axpy,
-// the same again for the second pass, k_gs_scale).  Launches of small systems take 2.5 us each
-// whatever they do, so what follows a pass rides on it: w.w on the first pass's products, the new
-// norm on the update, the second-pass decision and the final norm on the kernels that need them,
-// the column of H on the scaling.  One launch a quantity took 14 and a copy: 41 us a step on
-// 5,600 dofs (29 steps) against 17 us, 90 against 40 us on 557,700 dofs in FP32.
+// Gram-Schmidt of one Arnoldi step in five launches (small systems) or eight (k_gs_dots, [k_gs_fin,]
+// k_gs_axpy, the same again for the second pass, [k_gs_norm,] k_gs_scale).  Launches of small systems
+// take 2.5 us each whatever they do, so what follows a pass rides on it: w.w on the first pass's
+// products, the new norm on the update, the second-pass decision and the final norm on the kernels
+// that need them, the column of H on the scaling.  One launch a quantity took 14 and a copy: 41 us a
+// step on 5,600 dofs (29 steps) against 17 us, 90 against 44 us on 557,700 dofs in FP32.  The long
+// vectors' sums keep the partition and the order of those launches (see k_update_lp in gm_mpm.hip).
 
-// the partial sums of ||w||^2 that k_gs_axpy left, added in a fixed order
+// the partial sums of ||w||^2 that k_gs_axpy or k_gs_norm left, added in a fixed order
 __device__ __forceinline__ double norm_of_parts(const double* npart, int np, double* sh) {
   double s = 0.0;
   for (int c = threadIdx.x; c < np; c += RED_T) s += npart[c];
   return block_sum(s, sh);
 }
 
-// part[i * nchunk + c]: partial dots of w with basis vectors V[0..k) and, in the first pass
-// (npart null), with itself (i = k).  The second pass first takes the selective
-// reorthogonalisation test (Daniel, Gragg, Kaufman & Stewart 1976) on the norm after the first
-// pass, sc[0], and before it, sc[1]: sc[2] = 1 when the pass removed more than half of ||w||^2 or
-// a norm is NaN; else the pass is left out.
+// part[i * nchunk + c]: partial dots of w with basis vectors V[0..k), nchunk workgroups each, and in
+// the first pass (ww given) wpart: of w with itself, the workgroups after those.  The second pass
+// (ww null) first takes the selective reorthogonalisation test (Daniel, Gragg, Kaufman & Stewart
+// 1976) on the norm after the first pass, whose np partial sums are in wpart, and before it, sc[1]:
+// sc[0] the former, sc[2] = 1 when the pass removed more than half of ||w||^2 or a norm is NaN; else
+// the pass is left out.
 template <typename TV>
 __global__ void __launch_bounds__(RED_T) k_gs_dots(long n, int k, const TV* V, long ldv, const TV* w, int nchunk,
-                                                   double* part, const double* npart, int np, double* sc) {
-  __shared__ double sh[RED_T / 64];
-  if (npart) {
-    const double after = norm_of_parts(npart, np, sh);
+                                                   double* part, double* ww, const double* wpart, int np, double* sc) {
+  __shared__ double sh[RED_T];
+  if (!ww) {
+    const double after = norm_of_parts(wpart, np, sh);
     const bool second = !(after >= 0.5 * sc[1]);
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
       sc[0] = after;
       sc[2] = second ? 1.0 : 0.0;
     }
     if (!second) return;
   }
-  const int i = blockIdx.y;
-  const TV* vi = i < k ? V + (long)i * ldv : w;
+  const bool self = (int)blockIdx.x >= nchunk * k;
+  const int c = self ? (int)blockIdx.x - nchunk * k : (int)blockIdx.x % nchunk;
+  const int chunks = self ? (int)gridDim.x - nchunk * k : nchunk;
+  const TV* vi = self ? w : V + (long)(blockIdx.x / nchunk) * ldv;
   double s = 0.0;
-  for (long r = blockIdx.x * (long)RED_T + threadIdx.x; r < n; r += (long)nchunk * RED_T)
-    s += (double)vi[r] * (double)w[r];
+  for (long r = c * (long)RED_T + threadIdx.x; r < n; r += (long)chunks * RED_T) s += (double)vi[r] * (double)w[r];
   s = block_sum(s, sh);
-  if (threadIdx.x == 0) part[(long)i * nchunk + blockIdx.x] = s;
+  if (threadIdx.x == 0) (self ? ww[c] : part[blockIdx.x]) = s;
 }
 
-// h[i] = sum_c part[i * nchunk + c] for i < k, *ww that of i = k (one block each, fixed order)
+// h[i] = sum_c part[i * nchunk + c] for i < k, *ww the sum of the np partial sums wpart (i = k; one
+// block each, fixed order)
 __global__ void __launch_bounds__(RED_T) k_gs_fin(const double* gate, int k, int nchunk, const double* part, double* h,
-                                                  double* ww) {
+                                                  const double* wpart, int np, double* ww) {
   if (gate && *gate == 0.0) return;
-  __shared__ double sh[RED_T / 64];
-  const int i = blockIdx.x;
+  __shared__ double sh[RED_T];
+  const int i = blockIdx.x, n = i < k ? nchunk : np;
+  const double* p = i < k ? part + (long)i * nchunk : wpart;
   double s = 0.0;
-  for (int c = threadIdx.x; c < nchunk; c += RED_T) s += part[(long)i * nchunk + c];
+  for (int c = threadIdx.x; c < n; c += RED_T) s += p[c];
   s = block_sum(s, sh);
   if (threadIdx.x == 0) (i < k ? h[i] : *ww) = s;
 }
 
+// npart: the workgroups' partial sums of ||w||^2
+template <typename TV>
+__global__ void __launch_bounds__(RED_T) k_gs_norm(const double* gate, long n, const TV* w, double* npart) {
+  __shared__ double sh[RED_T];
+  if (*gate == 0.0) return;
+  double s = 0.0;
+  for (long r = blockIdx.x * (long)RED_T + threadIdx.x; r < n; r += (long)gridDim.x * RED_T)
+    s += (double)w[r] * (double)w[r];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) npart[blockIdx.x] = s;
+}
+
 // w -= sum_i V_i h_i, and the partial sums of the new ||w||^2 (npart, one a block).  A row a
 // thread, four independent partial sums over the basis vectors so that four loads are in flight.
-// nchunk > 0: h (and ww, when given) are summed here from part, in every block; block 0 stores them.
+// nchunk > 0: h (and ww, when given, behind it) are summed here from part, in every block; block 0
+// stores them.
 template <typename TV>
 __global__ void __launch_bounds__(RED_T) k_gs_axpy(const double* gate, long n, int k, const TV* V, long ldv,
                                                    const double* part, int nchunk, double* h, double* ww, TV* w,
                                                    double* npart) {
-  __shared__ double hs[GS_MAX], sh[RED_T / 64];
+  __shared__ double hs[GS_MAX], sh[RED_T];
   if (gate && *gate == 0.0) return;
   for (int i = threadIdx.x; i < k + (nchunk && ww ? 1 : 0); i += RED_T) {
     double s = 0.0;
@@ -1479,7 +1498,7 @@ template <typename TV>
 __global__ void __launch_bounds__(RED_T) k_gs_scale(long n, int k, const TV* w, const double* npart, int np,
                                                     const double* h, const double* h2, const double* sc, TV* v,
                                                     double* host, int stride) {
-  __shared__ double sh[RED_T / 64];
+  __shared__ double sh[RED_T];
   const bool second = sc[2] != 0.0;
   const double q = second ? norm_of_parts(npart, np, sh) : sc[0];
   const double s = (q > 0.0) ? 1.0 / sqrt(q) : 0.0;
@@ -1718,12 +1737,13 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
   const int cap = std::max(64 * (m + 1), 2048);
   double* npart = part + (cap - GS_BLOCKS);
   const int ab = (int)std::min<long>(GS_BLOCKS, gm_blocks(n, RED_T));
-  // chunks of a product with one basis vector: 256 fill the chip.  Up to 64 k entries at most 16,
-  // of at least 1024 entries each: few enough for every block of the update to add them up itself
+  // chunks of a product with one of k basis vectors: 256 fill the chip.  Up to 64 k entries at most
+  // 16, of at least 1024 entries each: few enough for every block of the update to add them up itself
   // (fold), which saves the launch of k_gs_fin; above, the blocks are many and it costs more
   const bool fold = n <= 65536;
-  auto chunks = [&](int cols) {
-    return std::max(1, std::min(fold ? (int)std::min<long>(16, n / 1024) : 256, (cap - GS_BLOCKS) / cols));
+  auto chunks = [&](int k) {
+    if (fold) return std::max(1, std::min((int)std::min<long>(16, n / 1024), (cap - GS_BLOCKS) / (k + 1)));
+    return std::max(1, std::min(std::min(256, 64 * (m + 1) / k), (cap - GS_BLOCKS) / k));
   };
   GM_HIP(hipMemsetAsync(x, 0, sizeof(TV) * n, st));
   // ||b||
@@ -1833,16 +1853,20 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
         int prc = prec.apply(vj, zj, q);
         if (prc) return prc;
         launch_spmv<NB, TM, TV, TV>(n_rows, rp, ci, vals, zj, w, nullptr, nullptr, nullptr, q, 0, nullptr, win);
-        const int nchunk = chunks(j + 2), fc = fold ? nchunk : 0;
+        const int k = j + 1, nchunk = chunks(k), fc = fold ? nchunk : 0;
         double *h2 = dh + (m + 2), *sc = dh + nsl;
-        k_gs_dots<TV><<<dim3(nchunk, j + 2), RED_T, 0, q>>>(n, j + 1, V, ldv, w, nchunk, part, nullptr, 0, sc);
-        if (!fold) k_gs_fin<<<j + 2, RED_T, 0, q>>>(nullptr, j + 1, nchunk, part, dh, sc + 1);
-        k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(nullptr, n, j + 1, V, ldv, part, fc, dh, sc + 1, w, npart);
-        k_gs_dots<TV><<<dim3(nchunk, j + 1), RED_T, 0, q>>>(n, j + 1, V, ldv, w, nchunk, part, npart, ab, sc);
-        if (!fold) k_gs_fin<<<j + 1, RED_T, 0, q>>>(sc + 2, j + 1, nchunk, part, h2, nullptr);
-        k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(sc + 2, n, j + 1, V, ldv, part, fc, h2, nullptr, w, npart);
-        k_gs_scale<TV><<<vb, RED_T, 0, q>>>(n, j + 1, w, npart, ab, dh, h2, sc, vj1,
-                                               host + (j & 1) * half, m + 2);
+        // w.w: chunks behind the products' for the update to add up, or those of the norms
+        const int wc = fold ? nchunk : ab;
+        double* wpart = fold ? part + k * nchunk : npart;
+        k_gs_dots<TV><<<nchunk * k + wc, RED_T, 0, q>>>(n, k, V, ldv, w, nchunk, part, wpart, nullptr, 0, sc);
+        if (!fold) k_gs_fin<<<k + 1, RED_T, 0, q>>>(nullptr, k, nchunk, part, dh, wpart, wc, sc + 1);
+        k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(nullptr, n, k, V, ldv, part, fc, dh, sc + 1, w, npart);
+        k_gs_dots<TV><<<nchunk * k, RED_T, 0, q>>>(n, k, V, ldv, w, nchunk, part, nullptr, npart, ab, sc);
+        if (!fold) k_gs_fin<<<k, RED_T, 0, q>>>(sc + 2, k, nchunk, part, h2, nullptr, 0, nullptr);
+        k_gs_axpy<TV><<<ab, RED_T, 0, q>>>(sc + 2, n, k, V, ldv, part, fc, h2, nullptr, w, npart);
+        const int nb2 = fold ? ab : 256;  // partial sums of the second pass's norm
+        if (!fold) k_gs_norm<TV><<<nb2, RED_T, 0, q>>>(sc + 2, n, w, npart);
+        k_gs_scale<TV><<<vb, RED_T, 0, q>>>(n, k, w, npart, nb2, dh, h2, sc, vj1, host + (j & 1) * half, m + 2);
         GM_LAUNCH_CHECK();
         return 0;
       };
@@ -2237,7 +2261,8 @@ __global__ void __launch_bounds__(256) k_dense_mv(int n, const double* Minv, con
       v[u] = (double)b[j];
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s += j0 + 64 * u < n ? m[u] * v[u] : 0.0;
+    for (int u = 0; u < 8; ++u)
+      if (j0 + 64 * u < n) s = fma(m[u], v[u], s);  // (entry by entry: the sum of one at a time)
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);

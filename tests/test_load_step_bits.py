@@ -248,3 +248,75 @@ def test_mass_cg_sums_as_the_general_cg(cells, options):
         out.append((x, it.value, rr.value))
     print(cells, options, out[0][1:], out[1][1:])
     assert torch.equal(out[0][0], out[1][0]) and out[0][1:] == out[1][1:]
+
+
+def _tree(v):
+    """Sum over the last axis, 256 long, halves added onto each other."""
+    while v.shape[-1] > 1:
+        v = v[..., :v.shape[-1] // 2] + v[..., v.shape[-1] // 2:]
+    return v[..., 0]
+
+
+def _dot(a, b, chunks):
+    """Sum of FP32 products in FP64: chunks of 256 threads in turn, a tree over each chunk's threads, then
+    256 threads over the chunks and a tree."""
+    def strided(v, width):
+        v = np.pad(v, (0, -len(v) % width)).reshape(-1, width)
+        s = np.zeros(width)
+        for row in v:
+            s = s + row
+        return s
+    part = _tree(strided(a.astype(np.float64) * b.astype(np.float64), chunks * 256).reshape(chunks, 256))
+    return _tree(strided(part, 256))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n', [65537, 131072, 300001])
+@pytest.mark.parametrize('near', [False, True])
+def test_gmres_sums_of_long_vectors(n, near):
+    """One step of FP32 GMRES on a system of more than 65,536 unknowns: its residual estimate from sums in
+    the stated order (products with a basis vector in 256 chunks, norms in up to 1024, that of a second
+    pass in 256), bit for bit.  near: the first pass removes almost all of w and a second one follows."""
+    import torch
+    from geowarp_amd import _lib as L
+    from geowarp_amd.solvers._engine import _stream
+    rng = np.random.default_rng(n)
+    f32 = np.float32
+    lower, upper = ((rng.random(n) * (1e-3 if near else 3.0)).astype(f32) for _ in range(2))
+    lower[0] = upper[-1] = 0.0
+    diag = np.where(rng.random(n) < 0.5, f32(1), f32(2))  # (its inverse is exact)
+    b = rng.standard_normal(n).astype(f32)
+    i = np.arange(n)
+    cols = np.stack([i - 1, i, i + 1], 1)
+    ok = (cols >= 0) & (cols < n)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device='cuda')  # noqa: E731
+    rp, ci = t(np.r_[0, ok.sum(1).cumsum()].astype(np.int32)), t(cols[ok].astype(np.int32))
+    vals, B = t(np.stack([lower, diag, upper], 1)[ok]), t(b)
+    m = 12
+    x, z, w, dinv = (torch.zeros(n, dtype=torch.float32, device='cuda') for _ in range(4))
+    V = torch.zeros(m + 1, n, dtype=torch.float32, device='cuda')
+    part = torch.zeros(2048, dtype=torch.float64, device='cuda')
+    dh = torch.zeros(3 * (m + 2), dtype=torch.float64, device='cuda')
+    its, rel = L.c_int(0), L.c_double(0.0)
+    L.check(L.lib().gm_gmres(1, 1, n, L.ptr(rp), L.ptr(ci), L.ptr(vals), L.ptr(B), L.ptr(x), L.ptr(V), L.ptr(z),
+                             L.ptr(w), L.ptr(dinv), L.ptr(part), L.ptr(dh), m, 1e-12, 1, L.ctypes.byref(its),
+                             L.ctypes.byref(rel), _stream()), 'gm_gmres')
+    f64 = lambda a: a.astype(np.float64)  # noqa: E731
+    nv = min(1024, -(-n // 256))  # chunks of a norm
+    beta = np.sqrt(_dot(b, b, nv))
+    v = (f64(b) * (1.0 / beta)).astype(f32)
+    y = f64(v / diag)
+    q = np.r_[0.0, y, 0.0]
+    u = (f64(lower) * q[:-2] + f64(diag) * y + f64(upper) * q[2:]).astype(f32)
+    h, before = _dot(v, u, 256), _dot(u, u, nv)
+    u = (f64(u) - h * f64(v)).astype(f32)
+    after = _dot(u, u, nv)
+    assert (after < 0.5 * before) == near
+    if near:
+        h2 = _dot(v, u, 256)
+        u = (f64(u) - h2 * f64(v)).astype(f32)
+        h, after = h + h2, _dot(u, u, 256)
+    hn = np.sqrt(after)
+    want = abs(-(hn / np.sqrt(h * h + hn * hn)) * beta) / beta
+    print(n, near, rel.value, want)
+    assert its.value == 1 and rel.value == want
