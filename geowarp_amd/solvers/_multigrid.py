@@ -133,9 +133,10 @@ class Multigrid:
         nc = self.levels[len(dims) - 1].n_nodes * self.nb
         self.dense = len(dims) > 1 and nc <= max_dense
         self.cinv = torch.zeros(nc * nc, dtype=torch.float64, device=dev) if self.dense else None
-        if self.dense:
-            # workspace of the device inverse and the error of its probe
-            self.cwork = torch.zeros(int(L.lib().gm_dense_inverse_work_bytes(nc)), dtype=torch.uint8, device=dev)
+        # workspace of the device inverse (written before it is read) and the error of its probe
+        self.cwork = self.cerr = None
+        if self.dense and nc <= DENSE_MAX:
+            self.cwork = torch.empty(int(L.lib().gm_dense_inverse_work_bytes(nc)), dtype=torch.uint8, device=dev)
             self.cerr = torch.zeros(1, dtype=torch.float64, device=dev)
         self.levels[len(dims) - 1].dense_inv = self.cinv.data_ptr() if self.dense else None
 
@@ -188,7 +189,7 @@ class Multigrid:
             k = self._keep[-1]
             lv = self.levels[self.n_levels - 1]
             nb, n = self.nb, lv.n_nodes
-            if n * nb <= DENSE_MAX:
+            if self.cwork is not None:
                 L.check(L.lib().gm_dense_inverse(nb, n, L.ptr(k['rp']), L.ptr(k['ci']), L.ptr(k['vals']),
                                                  L.ptr(self.cinv), L.ptr(self.cwork), self.cwork.numel(),
                                                  L.ptr(self.cerr), stream), 'gm_dense_inverse')

@@ -76,3 +76,43 @@ def test_dense_inverse_reports_an_operator_it_cannot_invert(kind):
     err = _inverse(2, v, rp, ci)[1]
     print(kind, err)
     assert not err <= DENSE_TOL
+
+
+def _coarsest(mgh):
+    """Dense copy of a hierarchy's coarsest operator."""
+    k, lv, nb = mgh._keep[-1], mgh.levels[mgh.n_levels - 1], mgh.nb
+    rp, ci = k['rp'].cpu().numpy().astype(int), k['ci'].cpu().numpy().astype(int)
+    v = k['vals'].double().cpu().numpy().reshape(-1, nb, nb)
+    A = np.zeros((lv.n_nodes, nb, lv.n_nodes, nb))
+    A[np.repeat(np.arange(lv.n_nodes), np.diff(rp)), :, ci, :] = v
+    return A.reshape(lv.n_nodes * nb, lv.n_nodes * nb)
+
+
+def _solved(problem, precision, **kw):
+    """A solver after a load step with multigrid, and its hierarchy."""
+    import harness as H
+    import geowarp_amd.solvers as gs
+    from geowarp_amd import problems as P
+    if problem == 'bar':
+        cfg = P.bar_nh(n_cells_x=12, n_cells_y=40)
+        cfg['iteration_dict'].update(precision=precision, tol=1e-8)
+    else:
+        cfg = P.indent3d(n_cells=(8, 8, 6), dx=0.125, total_steps=10, depth=0.02, footing=0.5, precision=precision,
+                         material='Neo-Hookean', footing_start='surface', penalty_form='physical')
+    cfg['iteration_dict']['krylov'] = 'mg'
+    s = H.make(gs, cfg)
+    s.advance_one_step(0, cfg['total_steps'])
+    return s, s.engine.multigrid(precision == 'mixed')[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('problem', ['bar', 'indent'])
+def test_host_inverse_beyond_the_device_limit(monkeypatch, problem):
+    """A coarsest operator larger than the device inverse takes: inverted on the host, and no workspace of
+    its square held."""
+    from geowarp_amd.solvers import _multigrid as MG
+    monkeypatch.setattr(MG, 'DENSE_MAX', 10)
+    s, mgh = _solved(problem, 'fp64')
+    A, n = _coarsest(mgh), mgh.levels[mgh.n_levels - 1].n_nodes * mgh.nb
+    assert mgh.dense and n > 10 and mgh.cwork is None and mgh.cerr is None
+    assert np.array_equal(mgh.cinv.cpu().numpy().reshape(n, n), MG._robust_inverse(A))
