@@ -133,9 +133,12 @@ class Multigrid:
         nc = self.levels[len(dims) - 1].n_nodes * self.nb
         self.dense = len(dims) > 1 and nc <= max_dense
         self.cinv = torch.zeros(nc * nc, dtype=torch.float64, device=dev) if self.dense else None
-        # workspace of the device inverse (written before it is read) and the error of its probe
+        # workspace of the device inverse (written before it is read) and the error of its probe.  The
+        # 3D mixed form inverts on the host where it keeps its coarse operators across load steps: the
+        # steps are held to the last bit (k_update_lp in gm_mpm.hip; with the device inverse's other
+        # roundings 12 entries in 24 load paths flipped), and the inverse is rare.
         self.cwork = self.cerr = None
-        if self.dense and nc <= DENSE_MAX:
+        if self.dense and nc <= DENSE_MAX and not (self.fp32 and self.dim == 3 and eng.mg_lag == 2):
             self.cwork = torch.empty(int(L.lib().gm_dense_inverse_work_bytes(nc)), dtype=torch.uint8, device=dev)
             self.cerr = torch.zeros(1, dtype=torch.float64, device=dev)
         self.levels[len(dims) - 1].dense_inv = self.cinv.data_ptr() if self.dense else None
@@ -182,8 +185,9 @@ class Multigrid:
             if not coarse:
                 return
         if self.dense:
-            # exact coarsest solve: the inverse formed on the device, or, when its probe is off (a
-            # singular operator, or one that needs pivoting across the whole matrix), on the host.
+            # exact coarsest solve: the inverse formed on the device, or on the host: where the device's
+            # is not wanted (see cwork), and when its probe is off (a singular operator, or one that needs
+            # pivoting across the whole matrix).
             # The host's LU alone took 4.5 ms for 602 dofs and 38 ms for 1890, to which its
             # scatter and copies came; the device's takes 0.37 and 1.48 ms.
             k = self._keep[-1]

@@ -320,3 +320,15 @@ def test_gmres_sums_of_long_vectors(n, near):
     want = abs(-(hn / np.sqrt(h * h + hn * hn)) * beta) / beta
     print(n, near, rel.value, want)
     assert its.value == 1 and rel.value == want
+
+
+@pytest.mark.gpu
+def test_mixed_3d_hierarchy_keeps_the_host_inverse():
+    """The coarsest operator of the 3D mixed form's hierarchy, which is kept across load steps, is inverted by
+    LU on the host, bit for bit."""
+    from test_dense_inverse import _coarsest, _solved
+    from geowarp_amd.solvers import _multigrid as MG
+    s, mgh = _solved('indent', 'mixed')
+    A = _coarsest(mgh)
+    assert mgh.dense and mgh.fp32
+    assert np.array_equal(mgh.cinv.cpu().numpy().reshape(A.shape), MG._robust_inverse(A))
