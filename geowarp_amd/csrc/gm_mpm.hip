@@ -22,6 +22,9 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "gm_common.h"
 #include "gm_device.h"
 #include "gm_types.h"
@@ -456,6 +459,17 @@ struct WaveRows {
       if (l < n && e < w) base[l * stride + e] = tile[l * (W | 1) + e];
     }
   }
+  // the same with P >= W lanes a row, a power of two: the steps differ by constants, where flush has a
+  // place of its own for every step, W registers that the tangent's terms need
+  template <int W, int P, int STRIDE>
+  __device__ __forceinline__ void flush_padded(T* base, int w) {
+    const int l0 = lane / P, e = lane % P;
+    const T* t = tile + l0 * (W | 1) + e;
+    const int at = l0 * STRIDE + e;
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+      if (l0 + i * (64 / P) < n && e < w) (base + i * (64 / P) * STRIDE)[at] = t[i * (64 / P) * (W | 1)];
+  }
   // rows by index: the loads, then the exchange
   template <int W>
   __device__ __forceinline__ void load(const T* base, int row, T* t) {
@@ -479,16 +493,24 @@ struct WaveRows {
   }
 };
 
+// f(0), f(1), ...: the rows of the tangent, unrolled whatever their size
+template <typename F, int... I>
+__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
 // One particle a lane, an instance a material (MAT): the return maps of the others would cost it
 // registers.  The per-particle arrays and the rows of Y and D pass through LDS (WaveRows); D is
 // formed row by row, R rows a pass of the tile (1 and 4 FP32 rows a pass: 658 and 763 us where 2
 // take 672).  Bound by the memory traffic of those rows.  1,048,576 particles, a lane writing its
 // own rows and D by columns before: 3D u-p Neo-Hookean 334 -> 265 us without the tangent, 1282 ->
 // 672 with FP32 and 2404 -> 1024 with FP64 rows of D; 2D J2 220 -> 149 and 340 -> 229 us; 37,128
-// particles of 3D Drucker-Prager 151 -> 73 us.  A few thousand particles take the latency of one
-// wavefront either way (25 and 29 us).
+// particles of 3D Drucker-Prager 151 -> 73 us.  6,048 particles take the latency of one wavefront,
+// 29 us (30).  Neo-Hookean rows sum the terms of the full product that are not zero, in its order and
+// with its roundings (see k_update_lp).  Two waves a SIMD: with the register or two more that the
+// compiler takes otherwise, one fits, and the stage without the tangent takes 352 us.
 template <int DIM, bool COUPLED, typename TD, int MAT>
-__global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args a) {
+__global__ void __launch_bounds__(128, MAT == MAT_NEOHOOKEAN || (DIM == 2 && !COUPLED) ? 2 : 1) k_particle_stage(gm_grid g, gm_stage_args a) {
   typedef Lay<DIM, COUPLED> L;
   constexpr bool neo_hookean = MAT == MAT_NEOHOOKEAN;
   constexpr int NY = L::NY, NZ = L::NZ;
@@ -768,17 +790,31 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
 #pragma unroll
       for (int k = 0; k < DIM; ++k) AtAg[i] += A.a[k][i] * Ag[k];
   }
+  // Neo-Hookean: the terms of d tau - p dJ I by column dH_ab that are not zero, d tau = mu (dH B + B^T
+  // dH^T) + lambda tr(A dH) I: mu B off the diagonal, and on it with and without a term of mu B
+  double mB[3][3], diag[3][3], both[3][3];
+  if constexpr (neo_hookean) {
+#pragma unroll
+    for (int bb = 0; bb < DIM; ++bb)
+#pragma unroll
+      for (int aa = 0; aa < DIM; ++aa) {
+        const double t = a.lam * A.a[bb][aa], u = fma(a.mu, B.a[bb][aa] + B.a[bb][aa], t), dJ = J * A.a[bb][aa];
+        mB[bb][aa] = a.mu * B.a[bb][aa];
+        diag[bb][aa] = COUPLED ? fma(-pp, dJ, t) : t;
+        both[bb][aa] = COUPLED ? fma(-pp, dJ, u) : u;
+      }
+  }
   const double kdt = a.mobility * a.dt * a.p_vol, kdtJ = kdt * J, ts = 0.5 / a.mu * a.p_vol * J;
   TD* D = (TD*)a.D + (long)k0 * NY * NZ;
-#pragma unroll
-  for (int y = 0; y < NY; ++y) {
+  each([&](auto index) {
+    constexpr int y = decltype(index)::value;
     double row[NZ];
 #pragma unroll
     for (int z = 0; z < NZ; ++z) row[z] = 0.0;
     if (y < L::NH) {
       // dP = -V0 [ dA^T M + A^T (dtau - p dJ I) ],  (dA^T X)[i][c] = -A[b][i] (A^T X)[a][c]
       const int i = y / DIM, c = y % DIM;
-      double T[DIM][3], ab = 0.0;  // Hencky family: A^T d tau by (a, j); Neo-Hookean: (A^T B^T)_ib below
+      double T[DIM][3], ab = 0.0;  // Hencky family: A^T d tau by (a, j)
       if constexpr (!neo_hookean) {
 #pragma unroll
         for (int aa = 0; aa < DIM; ++aa)
@@ -799,23 +835,21 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
 #pragma unroll
         for (int bb = 0; bb < DIM; ++bb) {  // column dH_ab
           const double dJ = J * A.a[bb][aa];
-          double t2;
+          double t2 = 0.0;
           if constexpr (neo_hookean) {
-            // d tau = mu (dH B + B^T dH^T) + lambda tr(A dH) I
-            t2 = a.mu * A.a[aa][i] * B.a[bb][c] + A.a[c][i] * a.lam * A.a[bb][aa];
-            if (aa == c) {
-              double s = 0.0;
+            // in the order and with the roundings of the full product (see k_update_lp)
 #pragma unroll
-              for (int k = 0; k < DIM; ++k) s += A.a[k][i] * B.a[bb][k];
-              t2 += a.mu * s;
+            for (int k = 0; k < DIM; ++k) {
+              if (k != aa && c != aa && k != c) continue;
+              t2 = fma(A.a[k][i], k != c ? mB[bb][k == aa ? c : k] : (c == aa ? both[bb][aa] : diag[bb][aa]), t2);
             }
           } else {
             t2 = ab * A.a[bb][aa];
 #pragma unroll
             for (int j = 0; j < 3; ++j) t2 += T[aa][j] * B.a[bb][j];
+            if (COUPLED) t2 -= A.a[c][i] * pp * dJ;
           }
-          if (COUPLED) t2 -= A.a[c][i] * pp * dJ;
-          row[aa * DIM + bb] = -a.p_vol * (t2 - A.a[bb][i] * AtM.a[aa][c]);
+          row[aa * DIM + bb] = -a.p_vol * fma(-A.a[bb][i], AtM.a[aa][c], t2);
         }
       if constexpr (COUPLED) row[L::Z_P] = a.p_vol * J * A.a[c][i];  // dP/dp = V0 J A^T
     } else if constexpr (COUPLED) {
@@ -857,16 +891,17 @@ __global__ void __launch_bounds__(128) k_particle_stage(gm_grid g, gm_stage_args
 #pragma unroll
         for (int k = 0; k < DIM; ++k) row[L::Z_G + k] = kdtJ * (DIM == 3 ? A.a[k][y - L::Y_M] : AtA[y - L::Y_M][k]);
     }
-    constexpr int TS = R * NZ | 1;
+    constexpr int W = R * NZ, TS = W | 1, P = W <= 4 ? 4 : W <= 8 ? 8 : W <= 16 ? 16 : 32;
+    static_assert(W <= P, "a row fits its lanes");
     const int slot = y % R;
     if (slot == 0) drows.sync();
 #pragma unroll
     for (int z = 0; z < NZ; ++z) drows.tile[lane * TS + slot * NZ + z] = (TD)row[z];
     if (slot == R - 1 || y == NY - 1) {
       drows.sync();
-      drows.template flush<R * NZ>(D + (y - slot) * NZ, NY * NZ, (slot + 1) * NZ);
+      drows.template flush_padded<W, P, NY * NZ>(D + (y - slot) * NZ, (slot + 1) * NZ);
     }
-  }
+  }, std::make_integer_sequence<int, NY>{});
 }
 
 extern "C" int gm_particle_stage(const gm_grid* g, const gm_stage_args* a, hipStream_t s) {

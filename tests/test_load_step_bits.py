@@ -332,3 +332,32 @@ def test_mixed_3d_hierarchy_keeps_the_host_inverse():
     A = _coarsest(mgh)
     assert mgh.dense and mgh.fp32
     assert np.array_equal(mgh.cinv.cpu().numpy().reshape(A.shape), MG._robust_inverse(A))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('stiffness,depth', [(0.921, 0.044), (0.902, 0.0441), (1.114, 0.0438), (0.992, 0.0438),
+                                             (0.946, 0.0509), (0.868, 0.0459)])
+def test_large_mixed_load_steps_clip_the_same_domains(stiffness, depth):
+    """Three load steps of the 64 x 64 x 32-cell indentation (mixed form): the 16,384 particles of the bottom
+    layer whose domains the box cuts are those of the fixture, recorded before the kernels of the step were
+    made faster.  On these six paths a sum in another order in any of the stage, the residual, the Jacobian,
+    the P2G, the mass or the coarsest inverse flips one to twenty of them."""
+    import os
+    import geowarp_amd.solvers as gs
+    from geowarp_amd import problems as P
+    cfg = P.indent3d(material='Neo-Hookean', precision='mixed', tol=1e-10, n_iter=12, footing=0.2, depth=depth,
+                     footing_start='surface', penalty_form='physical', dp_apex='return', shape_factor=0.1)
+    cfg['material_dict']['youngs_modulus'] *= stiffness
+    s = P.build_solver(gs, cfg, device='cuda')
+    cfg['particle_flags'](s.x_particles, s.particle_traction_flag_array, s.particle_pressure_boundary_flag_array)
+    s.line_search = True
+    s.linear_maxiter = 1500
+    bottom = s.x_particles[:, 2] < 0.5 * s.dz
+    for k in range(3):
+        s.advance_one_step(k, cfg['total_steps'])
+    cut = (s.GIMP_lp[:, 2] == s.x_particles[:, 2] - s.domain_min_z - 1e-6)[bottom].cpu().numpy()
+    with np.load(os.path.join(os.path.dirname(__file__), 'golden', 'indent_mixed_clips.npz')) as f:
+        want = np.unpackbits(f['%s_%s' % (stiffness, depth)]).astype(bool)
+    print(stiffness, depth, 'cut', int(cut.sum()), 'of', cut.size, 'other', int((cut != want).sum()))
+    assert cut.size == want.size == 16384
+    assert np.array_equal(cut, want)
