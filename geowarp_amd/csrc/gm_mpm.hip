@@ -1193,39 +1193,37 @@ __global__ void __launch_bounds__(192) k_strip_jacobian(gm_grid g, const double*
 }
 
 // ================================================================== node residual
-template <int DIM, bool COUPLED>
+// 3D u-p, a thread per node (gm_node_residual_binned sums per bin)
 __global__ void __launch_bounds__(128) k_node_residual(gm_grid g, const double* x_s, const double* lp_s,
                                                        const int* cell_start, const uint8_t* ext_s, const double* Y,
                                                        const uint8_t* freem, double* rhs) {
-  typedef Lay<DIM, COUPLED> L;
+  typedef Lay<3, true> L;
   int I = blockIdx.x * blockDim.x + threadIdx.x;
   if (I >= g.n_nodes) return;
   int ci[3] = {0, 0, 0};
-  node_coords<DIM>(g, I, ci);
+  node_coords<3>(g, I, ci);
   double r[L::NB];
 #pragma unroll
   for (int k = 0; k < L::NB; ++k) r[k] = 0.0;
-  for_candidates<DIM>(g, ci, cell_start, ext_s, [&](int k, const int* o, const int* b, bool in) {
+  for_candidates<3>(g, ci, cell_start, ext_s, [&](int k, const int* o, const int* b, bool in) {
     if (!in) return;
-    Axis ax[DIM];
-    load_axes<DIM>(g, x_s, lp_s, k, ax);
+    Axis ax[3];
+    load_axes<3>(g, x_s, lp_s, k, ax);
     double w, G[3], wa;
-    node_geom<DIM>(ax, o, w, G, wa);
+    node_geom<3>(ax, o, w, G, wa);
     const double* yp = Y + (long)k * L::NY;
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) {
+    for (int c = 0; c < 3; ++c) {
       double s = 0.0;
 #pragma unroll
-      for (int bb = 0; bb < DIM; ++bb) s += G[bb] * yp[bb * DIM + c];
+      for (int bb = 0; bb < 3; ++bb) s += G[bb] * yp[bb * 3 + c];
       r[c] += s + w * yp[L::Y_T + c];
     }
-    if (COUPLED) {
-      double s = w * yp[L::Y_Q];
+    double s = w * yp[L::Y_Q];
 #pragma unroll
-      for (int bb = 0; bb < DIM; ++bb) s += G[bb] * yp[L::Y_M + bb];
-      s += (w - wa) * yp[L::Y_S];
-      r[DIM] += s;
-    }
+    for (int bb = 0; bb < 3; ++bb) s += G[bb] * yp[L::Y_M + bb];
+    s += (w - wa) * yp[L::Y_S];
+    r[3] += s;
   });
 #pragma unroll
   for (int k = 0; k < L::NB; ++k) rhs[I * L::NB + k] = freem[I * L::NB + k] ? r[k] : 0.0;
@@ -1241,7 +1239,7 @@ extern "C" int gm_node_residual(const gm_grid* g, const gm_bins* b, const double
   else if (g->dim == 2)
     k_strip_residual<true><<<gm_blocks(n, RES_ROWS_UP), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else if (coupled)
-    k_node_residual<3, true><<<blk, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
+    k_node_residual<<<blk, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, Y, freem, rhs);
   else {
     gm::set_error("gm_node_residual: 3D single-phase is not a supported form");
     return -1;
@@ -1251,27 +1249,27 @@ extern "C" int gm_node_residual(const gm_grid* g, const gm_bins* b, const double
 }
 
 // ================================================================== node Jacobian
-// One 64-lane wavefront per block row.  Lane l owns compressed slots l and l+64.
-template <int DIM, bool COUPLED, typename TD, typename TV>
+// 3D u-p: one 64-lane wavefront per block row.  Lane l owns compressed slots l and l+64.
+template <typename TD, typename TV>
 __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double* x_s, const double* lp_s,
                                                       const int* cell_start, const uint8_t* ext_s, const TD* D,
                                                       const uint8_t* freem, const int* row_ptr,
                                                       const uint64_t* row_mask, TV* vals) {
-  typedef Lay<DIM, COUPLED> L;
+  typedef Lay<3, true> L;
   const int NB = L::NB, NZ = L::NZ, NY = L::NY;
   // the particles of a bin are taken JB at a time: their axis data, support flags and
   // E = L_I D_p rows are formed in parallel, then every slot lane accumulates them in
   // bin order (the order and arithmetic of one-particle-at-a-time processing)
   constexpr int JB = 8;
   __shared__ double E[JB][NB * NZ];
-  __shared__ Axis AX[JB][DIM];
+  __shared__ Axis AX[JB][3];
   __shared__ int INS[JB];
   __shared__ uint8_t EXS[JB];
   int I = blockIdx.x;
   if (I >= g.n_nodes) return;
   int lane = threadIdx.x;
   int ci[3] = {0, 0, 0};
-  node_coords<DIM>(g, I, ci);
+  node_coords<3>(g, I, ci);
   uint64_t m0 = row_mask[2 * I], m1 = row_mask[2 * I + 1];
   int nnz = __popcll(m0) + __popcll(m1);
   int rp = row_ptr[I];
@@ -1285,8 +1283,7 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
     myoff[s2][0] = myoff[s2][1] = myoff[s2][2] = 0;
     if (has[s2]) {
       int cnt = 0, bit = 0;
-      const int nbits = (DIM == 2) ? 25 : 125;
-      for (bit = 0; bit < nbits; ++bit) {
+      for (bit = 0; bit < 125; ++bit) {
         uint64_t w = (bit < 64) ? m0 : m1;
         if ((w >> (bit & 63)) & 1ull) {
           if (cnt == slot) break;
@@ -1295,7 +1292,7 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
       }
       myoff[s2][0] = bit % 5 - 2;
       myoff[s2][1] = (bit / 5) % 5 - 2;
-      myoff[s2][2] = (DIM == 3) ? bit / 25 - 2 : 0;
+      myoff[s2][2] = bit / 25 - 2;
     }
   }
   double acc[2][NB * NB];
@@ -1305,8 +1302,7 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
     for (int k = 0; k < NB * NB; ++k) acc[s2][k] = 0.0;
 
   int ncell[3] = {g.nx, g.ny, g.nz};
-  const int oz_n = (DIM == 3) ? 3 : 1;
-  for (int oz = 0; oz < oz_n; ++oz)
+  for (int oz = 0; oz < 3; ++oz)
     for (int oy = 0; oy < 3; ++oy)
       for (int ox = 0; ox < 3; ++ox) {
         // base cell I - o: its particles have node I at stencil offset o (candidate walk order)
@@ -1314,12 +1310,12 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
         int bc[3];
         bool ok = true;
 #pragma unroll
-        for (int a = 0; a < DIM; ++a) {
+        for (int a = 0; a < 3; ++a) {
           bc[a] = ci[a] - o[a];
           if (bc[a] < 0 || bc[a] > ncell[a]) ok = false;
         }
         if (!ok) continue;
-        int bn = node_index<DIM>(g, bc);
+        int bn = node_index<3>(g, bc);
         int ks = cell_start[bn], ke = cell_start[bn + 1];
         for (int k0 = ks; k0 < ke; k0 += JB) {
           const int nj = min(JB, ke - k0);
@@ -1328,13 +1324,13 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
             uint8_t ex = ext_s[k];
             bool in = true;
 #pragma unroll
-            for (int a = 0; a < DIM; ++a) in = in && (o[a] < (((ex >> a) & 1) ? 3 : 2));
+            for (int a = 0; a < 3; ++a) in = in && (o[a] < (((ex >> a) & 1) ? 3 : 2));
             INS[lane] = in ? 1 : 0;
             EXS[lane] = ex;
-            Axis ax[DIM];
-            load_axes<DIM>(g, x_s, lp_s, k, ax);
+            Axis ax[3];
+            load_axes<3>(g, x_s, lp_s, k, ax);
 #pragma unroll
-            for (int a = 0; a < DIM; ++a) AX[lane][a] = ax[a];
+            for (int a = 0; a < 3; ++a) AX[lane][a] = ax[a];
           }
           __syncthreads();
           // E = L_I D_p  (NB x NZ) for each particle of the batch
@@ -1342,18 +1338,18 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
             int pj = q / (NB * NZ), qq = q % (NB * NZ);
             if (!INS[pj]) continue;
             double wI, GI[3], waI;
-            node_geom<DIM>(AX[pj], o, wI, GI, waI);
+            node_geom<3>(AX[pj], o, wI, GI, waI);
             const TD* Dp = D + (long)(k0 + pj) * NY * NZ;
             int r = qq / NZ, z = qq % NZ;
             double sE = 0.0;
-            if (r < DIM) {
+            if (r < 3) {
 #pragma unroll
-              for (int bb = 0; bb < DIM; ++bb) sE += GI[bb] * (double)Dp[(bb * DIM + r) * NZ + z];
+              for (int bb = 0; bb < 3; ++bb) sE += GI[bb] * (double)Dp[(bb * 3 + r) * NZ + z];
               sE += wI * (double)Dp[(L::Y_T + r) * NZ + z];
             } else {
               sE = wI * (double)Dp[L::Y_Q * NZ + z];
 #pragma unroll
-              for (int bb = 0; bb < DIM; ++bb) sE += GI[bb] * (double)Dp[(L::Y_M + bb) * NZ + z];
+              for (int bb = 0; bb < 3; ++bb) sE += GI[bb] * (double)Dp[(L::Y_M + bb) * NZ + z];
               sE += (wI - waI) * (double)Dp[L::Y_S * NZ + z];
             }
             E[pj][qq] = sE;
@@ -1367,30 +1363,28 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
               int oJ[3];
               bool inJ = true;
 #pragma unroll
-              for (int aa = 0; aa < DIM; ++aa) {
+              for (int aa = 0; aa < 3; ++aa) {
                 oJ[aa] = o[aa] + myoff[s2][aa];  // offset of J inside this particle's stencil
                 int e = ((EXS[pj] >> aa) & 1) ? 3 : 2;
                 inJ = inJ && (oJ[aa] >= 0) && (oJ[aa] < e);
               }
               if (!inJ) continue;
               double wJ, GJ[3], waJ;
-              node_geom<DIM>(AX[pj], oJ, wJ, GJ, waJ);
+              node_geom<3>(AX[pj], oJ, wJ, GJ, waJ);
 #pragma unroll
               for (int r = 0; r < NB; ++r) {
 #pragma unroll
-                for (int e = 0; e < DIM; ++e) {
+                for (int e = 0; e < 3; ++e) {
                   double sv = 0.0;
 #pragma unroll
-                  for (int aa = 0; aa < DIM; ++aa) sv += E[pj][r * NZ + aa * DIM + e] * GJ[aa];
-                  if (DIM == 3 && COUPLED && e == 2) sv += E[pj][r * NZ + L::Z_DU] * wJ;
+                  for (int aa = 0; aa < 3; ++aa) sv += E[pj][r * NZ + aa * 3 + e] * GJ[aa];
+                  if (e == 2) sv += E[pj][r * NZ + L::Z_DU] * wJ;
                   acc[s2][r * NB + e] += sv;
                 }
-                if (COUPLED) {
-                  double sv = E[pj][r * NZ + L::Z_P] * wJ + E[pj][r * NZ + L::Z_PB] * waJ;
+                double sv = E[pj][r * NZ + L::Z_P] * wJ + E[pj][r * NZ + L::Z_PB] * waJ;
 #pragma unroll
-                  for (int aa = 0; aa < DIM; ++aa) sv += E[pj][r * NZ + L::Z_G + aa] * GJ[aa];
-                  acc[s2][r * NB + DIM] += sv;
-                }
+                for (int aa = 0; aa < 3; ++aa) sv += E[pj][r * NZ + L::Z_G + aa] * GJ[aa];
+                acc[s2][r * NB + 3] += sv;
               }
             }
           }
@@ -1402,7 +1396,7 @@ __global__ void __launch_bounds__(64, 3) k_node_jacobian(gm_grid g, const double
   for (int s2 = 0; s2 < 2; ++s2) {
     if (!has[s2]) continue;
     int cj[3] = {ci[0] + myoff[s2][0], ci[1] + myoff[s2][1], ci[2] + myoff[s2][2]};
-    int Jn = node_index<DIM>(g, cj);
+    int Jn = node_index<3>(g, cj);
     bool diag = (Jn == I);
     TV* out = vals + (long)(rp + lane + 64 * s2) * NB * NB;
 #pragma unroll
@@ -1572,48 +1566,32 @@ extern "C" int gm_node_jacobian(const gm_grid* g, const gm_bins* b, const gm_pat
                                 hipStream_t s) {
   GM_REQUIRE(g && b && pat, "gm_node_jacobian: null argument");
   int n = g->n_nodes;
-#define GM_JAC(DIM, CP, TD, TV)                                                                           \
-  k_node_jacobian<DIM, CP, TD, TV><<<n, 64, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s,          \
-                                                    (const TD*)D, freem, pat->row_ptr, pat->row_mask, (TV*)vals)
-#define GM_JAC_T(DIM, CP)                                  \
-  do {                                                     \
-    if (tangent_fp32 && vals_fp32) GM_JAC(DIM, CP, float, float);   \
-    else if (tangent_fp32) GM_JAC(DIM, CP, float, double);          \
-    else if (vals_fp32) GM_JAC(DIM, CP, double, float);             \
-    else GM_JAC(DIM, CP, double, double);                           \
-  } while (0)
-#define GM_STRIP(CP, TD, TV)                                                                                  \
-  k_strip_jacobian<CP, TD, TV><<<gm_blocks(n, (CP) ? 7 : 16), 192, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, \
-                                                                           b->ext_s, (const TD*)D, freem,     \
-                                                                           pat->row_ptr, pat->row_mask, (TV*)vals)
-#define GM_STRIP_T(CP)                                      \
-  do {                                                     \
-    if (tangent_fp32 && vals_fp32) GM_STRIP(CP, float, float);   \
-    else if (tangent_fp32) GM_STRIP(CP, float, double);          \
-    else if (vals_fp32) GM_STRIP(CP, double, float);             \
-    else GM_STRIP(CP, double, double);                           \
-  } while (0)
-  if (g->dim == 2 && !coupled) GM_STRIP_T(false);
-  else if (g->dim == 2) GM_STRIP_T(true);
-  else if (coupled && !getenv("GM_JACOBIAN_ROW_WAVE")) {
-    // lanes per (column, column dof) of a bin (k_node_jacobian_up3); GM_JACOBIAN_ROW_WAVE=1
-    // selects the one-wavefront-per-row form, which assembles the same matrix
-#define GM_JAC3(TD, TV)                                                                                   \
-  k_node_jacobian_up3<TD, TV><<<n, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, (const TD*)D, \
-                                                freem, pat->row_ptr, pat->row_mask, (TV*)vals)
-    if (tangent_fp32 && vals_fp32) GM_JAC3(float, float);
-    else if (tangent_fp32) GM_JAC3(float, double);
-    else if (vals_fp32) GM_JAC3(double, float);
-    else GM_JAC3(double, double);
-#undef GM_JAC3
-  } else if (coupled) GM_JAC_T(3, true);
-  else {
+  if (g->dim != 2 && !coupled) {
     gm::set_error("gm_node_jacobian: 3D single-phase is not a supported form");
     return -1;
   }
-#undef GM_STRIP_T
-#undef GM_STRIP
-#undef GM_JAC_T
+  // 3D u-p: lanes per (column, column dof) of a bin (k_node_jacobian_up3); GM_JACOBIAN_ROW_WAVE=1
+  // selects the one-wavefront-per-row form, which assembles the same matrix
+  const bool row_wave = getenv("GM_JACOBIAN_ROW_WAVE");
+#define GM_JAC(TD, TV)                                                                                           \
+  do {                                                                                                           \
+    if (g->dim == 2 && !coupled)                                                                                 \
+      k_strip_jacobian<false, TD, TV><<<gm_blocks(n, 16), 192, 0, s>>>(                                          \
+          *g, b->x_s, b->lp_s, b->cell_start, b->ext_s, (const TD*)D, freem, pat->row_ptr, pat->row_mask, (TV*)vals); \
+    else if (g->dim == 2)                                                                                        \
+      k_strip_jacobian<true, TD, TV><<<gm_blocks(n, 7), 192, 0, s>>>(                                            \
+          *g, b->x_s, b->lp_s, b->cell_start, b->ext_s, (const TD*)D, freem, pat->row_ptr, pat->row_mask, (TV*)vals); \
+    else if (row_wave)                                                                                           \
+      k_node_jacobian<TD, TV><<<n, 64, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, (const TD*)D, freem, \
+                                               pat->row_ptr, pat->row_mask, (TV*)vals);                          \
+    else                                                                                                         \
+      k_node_jacobian_up3<TD, TV><<<n, 128, 0, s>>>(*g, b->x_s, b->lp_s, b->cell_start, b->ext_s, (const TD*)D,  \
+                                                    freem, pat->row_ptr, pat->row_mask, (TV*)vals);              \
+  } while (0)
+  if (tangent_fp32 && vals_fp32) GM_JAC(float, float);
+  else if (tangent_fp32) GM_JAC(float, double);
+  else if (vals_fp32) GM_JAC(double, float);
+  else GM_JAC(double, double);
 #undef GM_JAC
   GM_LAUNCH_CHECK();
   return 0;
