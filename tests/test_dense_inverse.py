@@ -116,3 +116,60 @@ def test_host_inverse_beyond_the_device_limit(monkeypatch, problem):
     A, n = _coarsest(mgh), mgh.levels[mgh.n_levels - 1].n_nodes * mgh.nb
     assert mgh.dense and n > 10 and mgh.cwork is None and mgh.cerr is None
     assert np.array_equal(mgh.cinv.cpu().numpy().reshape(n, n), MG._robust_inverse(A))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind', ['singular', 'leading block'])
+def test_hierarchy_falls_back_to_the_host(monkeypatch, kind):
+    """A coarsest operator that the device's elimination cannot invert -- a node without stiffness; a regular
+    one whose leading 32 x 32 block is zero -- ends as the host's inverse or pseudo-inverse, over what
+    the device left."""
+    from geowarp_amd.solvers import _multigrid as MG
+    from geowarp_amd.solvers._engine import _stream
+    s, mgh = _solved('bar', 'fp64')
+    lv = mgh.levels[mgh.n_levels - 1]
+    nx1, n = lv.nx + 1, lv.n_nodes
+    k = mgh._keep[-1]
+    rp, ci = k['rp'].cpu().numpy().astype(int), k['ci'].cpu().numpy().astype(int)
+    row = np.repeat(np.arange(n), np.diff(rp))
+    v = np.zeros((len(ci), 2, 2))
+    if kind == 'singular':
+        v[ci == row] = np.eye(2) * 3.0
+        v[(ci == row) & (row == 5)] = 0.0
+    else:  # the first two lines of nodes exchanged with the next two
+        assert 4 * nx1 >= 32 and 4 * nx1 <= n
+        pair = np.where(np.arange(n) < 2 * nx1, np.arange(n) + 2 * nx1,
+                        np.where(np.arange(n) < 4 * nx1, np.arange(n) - 2 * nx1, np.arange(n)))
+        v[ci == pair[row]] = np.eye(2) * 2.0
+    import torch
+    k['vals'].copy_(torch.as_tensor(v.reshape(-1), device=k['vals'].device))
+
+    class Kept:  # the library, with the coarse operators left as they are
+        def __getattr__(self, name):
+            return (lambda *a: 0) if name == 'gm_mg_setup' else getattr(lib, name)
+
+    lib = L.lib()
+    monkeypatch.setattr(L, '_lib', Kept())
+    mgh.cinv.fill_(float('nan'))
+    mgh.setup(_stream())
+    A, X = _coarsest(mgh), mgh.cinv.cpu().numpy().reshape(2 * n, 2 * n)
+    print(kind, 'dofs', 2 * n, 'probe', float(mgh.cerr))
+    assert not float(mgh.cerr) <= MG.DENSE_TOL
+    assert np.isfinite(X).all() and np.abs(A @ X @ A - A).max() < 1e-12
+    assert np.array_equal(X, MG._robust_inverse(A))
+
+
+@pytest.mark.gpu
+def test_dense_inverse_of_the_largest_coarsest_operators():
+    """2,999 dofs: 94 blocks, the last of 23."""
+    rng, n, band = np.random.default_rng(0), 2999, 60
+    i = np.arange(n)
+    A = rng.uniform(-1, 1, (n, n))
+    A[np.abs(i[:, None] - i[None, :]) > band] = 0.0
+    A *= 0.5 / np.abs(A).sum(1, keepdims=True)
+    A[i, i] = 1.0
+    row, ci = np.nonzero(A)
+    X, err = _inverse(1, A[row, ci], np.r_[0, np.bincount(row, minlength=n).cumsum()], ci)
+    e = np.abs(A @ X - np.eye(n)).max()  # |inverse| <= 2 in the row-sum norm, as above
+    print('max |A X - I|', e, 'probe', err)
+    assert e < 1e-13 and err < 1e-12
