@@ -26,9 +26,9 @@ residual has passed the Newton test) on the previous iteration's Jacobian
 (chord_iters counts them; they stay Newton iterations of the count, each
 evaluating the residual, solving and updating as the others do).
 
-roofline: the dominant kernel of the timed form, the line phase of the
-Jacobian assembly (k_jac_line: the 27 x 27 block products of every particle bin
-on the matrix cores, summed along lines of bins), timed live with HIP events on its launch stream over
+roofline: the dominant kernel of the timed form, the per-bin phase of the
+Jacobian assembly (k_jac_bin: the 27 x 27 block products of every particle bin
+on the matrix cores), timed live with HIP events on its launch stream over
 repeated launches on the last tangent of the timed region; achieved =
 algorithmic flops per launch (2 x 60 per particle and block pair x 729 pairs)
 over that time, against the dense FP32 matrix peak; traffic is the counted HBM
@@ -257,7 +257,7 @@ def smoother_roofline(s, reps=50):
 
 
 def jacobian_roofline(s, reps=20):
-    """Time the line phase of the binned Jacobian assembly (k_jac_line through
+    """Time the per-bin phase of the binned Jacobian assembly (k_jac_bin through
     gm_jacobian_bins: every bin's 27 x 27 block products on the matrix cores) on the
     last tangent of the timed region, with HIP events on the launch stream.
     Algorithmic flops per launch: 2 x 60 per (particle, block pair) -- 4 rows x 15
@@ -294,20 +294,15 @@ def jacobian_roofline(s, reps=20):
         return e0.elapsed_time(e1) / reps
 
     avg_ms = avg(launch)
-    # the whole assembly (line sums + gather into the matrix), same stream
+    # the whole assembly (per-bin products + gather into the matrix), same stream
     asm_ms = avg(assemble)
     tune = eng.stats.get('jacobian_tune') or {}
     n_p = int(s.n_particles)
     flops = 2.0 * 60 * 729 * n_p
-    full = (eng.cell_start[1:] != eng.cell_start[:-1]).view(-1, eng.grid.nx + 1)
-    nonempty = int(full.sum().item())
-    # nodes a line's bins reach: 405 blocks of line sums each (the bin's node and the next two)
-    reach = full.clone()
-    reach[:, 1:] |= full[:, :-1]
-    reach[:, 2:] |= full[:, :-2]
+    nonempty = int((eng.cell_start[1:] != eng.cell_start[:-1]).sum().item())
     sz = 4 if fp32 else 8
-    bytes_ = n_p * (17 * 15 * sz + 48) + int(reach.sum().item()) * 405 * 16 * sz
-    return dict(kernel='k_jac_line<%s> (gm_jacobian_bins, variant %s)' % ('float' if fp32 else 'double',
+    bytes_ = n_p * (17 * 15 * sz + 48) + nonempty * 27 * 27 * 16 * sz
+    return dict(kernel='k_jac_bin<%s> (gm_jacobian_bins, variant %s)' % ('float' if fp32 else 'double',
                                                                         tune.get('bins_variant', 0)),
                 avg_us=avg_ms * 1e3, assembly_ms=asm_ms, tune=tune,
                 flops_per_launch=flops, achieved_TFs=flops / (avg_ms * 1e-3) / 1e12, bytes_per_launch=bytes_,
@@ -496,7 +491,7 @@ def c3_bench(steps):
 
 def measured_traffic(cells, material, kernel='k_spmv'):
     """HBM bytes per launch of a kernel (k_spmv: the FP32 SpMV; k_level: the FP16
-    smoother sweep; k_jac_line: the Jacobian's products along lines of bins) from the committed
+    smoother sweep; k_jac_bin: the per-bin Jacobian products) from the committed
     rocprofv3 FETCH_SIZE / WRITE_SIZE passes (profiles/<kernel>_c4_indentation*),
     scaled by the calibration kernel; None for other workloads."""
     path = os.path.join(ROOT, 'profiles', '%s_c4_indentation_traffic.json' % kernel)
@@ -674,7 +669,7 @@ def main():
         del s64
         torch.cuda.empty_cache()
 
-    # roofline of the dominant kernel of the timed form (the Jacobian line sums), of the
+    # roofline of the dominant kernel of the timed form (the per-bin Jacobian products), of the
     # level-0 smoother sweep and of the Krylov SpMV (last Jacobian of the timed region)
     jr = jacobian_roofline(smx)
     smo = smoother_roofline(smx)
@@ -682,7 +677,7 @@ def main():
     peak = MFMA_FP32_PEAK_TFS if smx.engine._tangent_fp32() else MFMA_FP64_PEAK_TFS
     out['roofline'] = {'bound': 'mfma', 'achieved': round(jr['achieved_TFs'], 2), 'peak': peak, 'unit': 'TFLOP/s',
                        'frac': round(jr['achieved_TFs'] / peak, 4),
-                       'traffic': measured_traffic(cells, args.material, 'k_jac_line'),
+                       'traffic': measured_traffic(cells, args.material, 'k_jac_bin'),
                        'kernel': jr['kernel'], 'avg_us': round(jr['avg_us'], 2),
                        'algorithmic_flops': jr['flops_per_launch'],
                        'bytes_per_launch': jr['bytes_per_launch'],
