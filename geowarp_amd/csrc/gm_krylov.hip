@@ -1739,7 +1739,10 @@ static int gmres_impl(int n_rows, const int* rp, const int* ci, const TM* vals, 
   const int ab = (int)std::min<long>(GS_BLOCKS, gm_blocks(n, RED_T));
   // chunks of a product with one of k basis vectors: 256 fill the chip.  Up to 64 k entries at most
   // 16, of at least 1024 entries each: few enough for every block of the update to add them up itself
-  // (fold), which saves the launch of k_gs_fin; above, the blocks are many and it costs more
+  // (fold), which saves the launches of k_gs_fin and k_gs_norm; above, the blocks are many and it
+  // costs more (FP64, us a step over 10 and 40 steps, folded against apart: 32,000 entries 44 and 41
+  // against 47 and 46, 65,000 49 and 46 against 49 and 51, 90,000 54 and 55 against 52 and 55, 200,000
+  // 75 and 82 against 63 and 74; FP32 alike)
   const bool fold = n <= 65536;
   auto chunks = [&](int k) {
     if (fold) return std::max(1, std::min((int)std::min<long>(16, n / 1024), (cap - GS_BLOCKS) / (k + 1)));
